@@ -53,8 +53,8 @@ def listed():
              rectangular=1, num_phi=160, num_branches=8, fmm_order=28, mixed=1),
         # uneven fields of 50 to 1000 equal masses, num_phi 504 with 4 branches, FP64
         dict(name="batch 24 fp64", kind="batch", fields=24, stars_lo=50, stars_hi=1000, num_phi=504, num_branches=4),
-        # the same fields in mixed precision, more of them
-        dict(name="batch 48 mixed", kind="batch", fields=48, stars_lo=50, stars_hi=1000, num_phi=504, num_branches=4, mixed=1),
+        # such fields in mixed precision, more of them
+        dict(name="batch 32 mixed", kind="batch", fields=32, stars_lo=50, stars_hi=1000, num_phi=504, num_branches=4, mixed=1),
         # f0, f1, w, length scale and 1/mu bound at host points of the 10 000-star field (a map of the field)
         dict(name="eval 100000 of 10000", kind="eval", num_stars=10000, mass="salpeter", kappa=0.5, kappa_star=0.5, shear=0.2,
              n=100000),
@@ -220,10 +220,8 @@ def run(state):
         b = state["batch"]
         if not b.run(0):
             raise RuntimeError(b.last_error())
-        # the fields' curves end to end, as one array of each kind
         n = range(len(b.params))
-        return dict(ccs=np.concatenate([b.array(i, ccf_amd.ARRAY_CCS).ravel() for i in n]),
-                    caustics=np.concatenate([b.array(i, ccf_amd.ARRAY_CAUSTICS).ravel() for i in n]))
+        return dict(ccs=[b.array(i, ccf_amd.ARRAY_CCS) for i in n], caustics=[b.array(i, ccf_amd.ARRAY_CAUSTICS) for i in n])
     c = state["ctx"]
     if kind == "run":
         if not c.run(0):
