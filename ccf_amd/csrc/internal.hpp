@@ -144,7 +144,8 @@ struct RootGrid
 // Work buffers of the Aberth sweeps over up to `rows` rows of R roots.
 struct SweepBufs
 {
-	int rows = 0, R = 0, tile = 0, max_items = 0;
+	int rows = 0, R = 0;
+	size_t part_room = 0;    // entries of part
 	int* act = nullptr;      // [2][rows][R] active root indices (ping-pong)
 	int* cnt = nullptr;      // [2][rows]
 	int* fl = nullptr;       // [rows][R] roots that need the Cauchy sums this sweep
@@ -155,7 +156,7 @@ struct SweepBufs
 	int* tile_off = nullptr; // [rows + 1] first tile of each row
 	int* plan = nullptr;     // [4] tiles, slices per tile; rows summed by the root-sum FMM in a phase's first and second sweep
 	int* ticket = nullptr;   // [1] workgroups of the sweep's Witt kernel done (the last forms the plan and resets it)
-	double2* part = nullptr; // [max_items][tile] partial Cauchy sums
+	double2* part = nullptr; // [items of a sweep][tile] partial Cauchy sums
 	// root-sum FMM (grid.order > 0 only)
 	RootGrid grid;
 	int* slot = nullptr;     // [rows][R] position of root a in fl this sweep, -1 otherwise

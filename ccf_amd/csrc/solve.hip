@@ -15,14 +15,15 @@
 //   K2 plan_sums   cuts the (stars + roots) term range of every tile of
 //                  RPT*256 listed roots into S slices so that dense and sparse
 //                  sweeps alike give enough equal work items to fill the chip;
-//   K3 k_sums      one work item = one tile x one slice: the slice's terms are
+//   K3 k_sums*     one work item = one tile x one slice: the slice's terms are
 //                  streamed through LDS and every lane accumulates
 //                  2 sum 1/(z - s_i) - sum 1/(z - z_j) for its RPT roots;
 //                  partials go to a buffer so the result is deterministic;
 //   K4 k_finalize  reduces the partials, forms z - f0 / (f1 + f0 S), tests
 //                  |dz| / theta < 1e-9, writes the root and appends the
 //                  unconverged ones to the next sweep's active list.
-// K3 exists in FP64 (the reference's arithmetic) and in FP32 with a per-chunk
+// K3 exists in FP64 (k_sums64 term by term for the branch centres,
+// k_sums64_quad with shared reciprocals after them) and in FP32 with a per-chunk
 // fallback: a lane whose nearest root in an LDS chunk is closer than
 // CLUSTER_REL times the field's half-length (where an FP32 difference of two
 // positions keeps fewer than ~12 bits) redoes that chunk in FP64.
@@ -76,8 +77,14 @@ namespace
 constexpr int BLOCK = 256;
 constexpr int CHUNK64 = 1024;         // FP64 complex values per LDS chunk (16 KiB)
 constexpr int CHUNK32 = 2048;         // FP32 complex values per LDS chunk (16 KiB)
+constexpr int ROOTS_PER_THREAD = 2;   // of k_sums32 and k_sums64 unless given or tuned
 constexpr int MAX_SLICES = 64;
 constexpr int MIN_SLICE = 1024;       // fewest terms per slice
+// k_sums64_quad, whose items are single waves: fewest terms per slice, and the
+// slices of a tile once the tiles alone are more than half the device's waves
+// (a last round of whole tiles would leave most SIMDs with a wave or none)
+constexpr int QUAD_MIN_SLICE = 256;
+constexpr int QUAD_SLICES = 4;
 
 inline int grid(long long n, int b = BLOCK) { return (int)((n + b - 1) / b); }
 
@@ -289,12 +296,12 @@ struct SweepView
 	double2* rsum;
 };
 
-SweepView view(const SweepBufs& B, int parity)
+SweepView view(const SweepBufs& B, int parity, int tile = 0)
 {
 	SweepView v;
 	v.R = B.R;
 	v.rows = B.rows;
-	v.tile = B.tile;
+	v.tile = tile;
 	const size_t list = (size_t)B.rows * B.R;
 	v.act = B.act + parity * list;
 	v.act_next = B.act + (parity ^ 1) * list;
@@ -409,7 +416,7 @@ __device__ inline Near coop_near(const LensView& L, int node, cd z, double (*red
 
 struct PlanArgs
 {
-	int nrows, terms, target, fmm_min, sweep;
+	int nrows, terms, target, fmm_min, sweep, tile, quad;
 };
 
 __device__ inline void plan_sums(SweepView V, const PlanArgs& P)
@@ -430,7 +437,7 @@ __device__ inline void plan_sums(SweepView V, const PlanArgs& P)
 		// this sweep's active count is consumed (k_witt read it): cleared
 		// here, it is the list the next sweep's k_witt appends stepped roots to
 		if (r < nrows) V.cnt[r] = 0;
-		const int v = (r < nrows && !fmm) ? (nf + V.tile - 1) / V.tile : 0;
+		const int v = (r < nrows && !fmm) ? (nf + P.tile - 1) / P.tile : 0;
 		int x = v;
 		for (int d = 1; d < 64; d <<= 1)
 		{
@@ -454,7 +461,13 @@ __device__ inline void plan_sums(SweepView V, const PlanArgs& P)
 	{
 		const int tiles = carry;
 		int S = 1;
-		if (tiles > 0 && tiles < target)
+		if (P.quad)
+		{
+			// as many items as the device holds waves, all in one round
+			if (tiles > 0) S = 2 * tiles <= target ? target / tiles : QUAD_SLICES;
+			S = min(min(S, MAX_SLICES), max(1, terms / QUAD_MIN_SLICE));
+		}
+		else if (tiles > 0 && tiles < target)
 		{
 			S = (target + tiles - 1) / tiles;
 			S = min(S, MAX_SLICES);
@@ -685,7 +698,12 @@ __device__ inline int row_of_tile(const int* __restrict__ tile_off, int nrows, i
 
 #include "rootfmm.hpp"
 
-// K3 in FP64: partial 2 sum_stars 1/(z - s) - sum_roots 1/(z - w) over one slice
+// K3 in FP64 of the initial solve: partial 2 sum_stars 1/(z - s) -
+// sum_roots 1/(z - w) over one slice, term by term in a fixed order. From
+// the seeds a rounding of these sums decides, for a few roots in 10 000,
+// which index takes which root (the sweeps before they settle are chaotic;
+// a continuation step starts next to its roots and is not), so the order
+// and form of the terms stay as they are here and a field keeps its indices.
 template <int RPT>
 __global__ __launch_bounds__(BLOCK) void k_sums64(const double2* __restrict__ spos, int Np, const double2* __restrict__ roots,
 	RowMap M, SweepView V, int nrows)
@@ -765,6 +783,184 @@ __global__ __launch_bounds__(BLOCK) void k_sums64(const double2* __restrict__ sp
 #pragma unroll
 		for (int k = 0; k < RPT; k++)
 			V.part[(size_t)item * T + k * BLOCK + threadIdx.x] = make_double2(2 * ax[k] - bx[k], -(2 * ay[k] - by[k]));
+	}
+}
+
+// K3 in FP64 of the continuation steps and of single sweeps
+// (k_sums64_quad): the same partial sums with the reciprocals shared.
+//
+// Four Cauchy terms d_i / |d_i|^2, d_i = z - w_i, added to (ax, ay) over one
+// reciprocal: with n_i = |d_i|^2 and the pair numerators d_0 n_1 + d_1 n_0
+// and d_2 n_3 + d_3 n_2, their sum is
+//   ((d_0 n_1 + d_1 n_0) n_2 n_3 + (d_2 n_3 + d_3 n_2) n_0 n_1) / (n_0 n_1 n_2 n_3).
+// 36 FP64 instructions and one v_rcp_f64 (3.4 instructions' time) for four
+// terms, against 11 (one of them v_max_f64, 1.7) and one for each term of
+// its own. No numerator cancels more than the sum of the terms itself does,
+// and the accumulator rounds once in four terms. NORM_FLOOR makes the term
+// of the root itself (d = 0) zero; it does not reach the last bit of any
+// n_i of two positions further apart than 1e-22. Products stay within range
+// while every |d_i| is below 1e38; beyond it the sums are not finite and the
+// slice is summed again term by term.
+//
+// Bound by the FP64 VALU: 20 000 roots against 30 000 terms take 0.22 ms
+// (2.7e12 terms/s; the loop alone reaches 3.2e12), 0.33 ms in k_sums64. A
+// continuation step's sparse sweeps gain more: waves as items, lanes over the
+// sources. Relative error of the sums against 80-bit ones, fields of 200 to
+// 20 000 roots: 2e-16 to 5e-16 rms, 4e-16 to 1.3e-15 term by term.
+constexpr double NORM_FLOOR = 1e-60;
+
+// 1/x from the hardware estimate r (relative error about 2^-23) as
+// r (1 + e + e^2), e = 1 - x r: one third-order step, whose error e^3 is far
+// below the rounding of the last multiply-add
+__device__ __forceinline__ double rcp64_cubic(double x)
+{
+	const double r = __builtin_amdgcn_rcp(x);
+	const double e = fma(-x, r, 1.0);
+	return fma(r, fma(e, e, e), r);
+}
+
+// the four terms times SIGN (1 or -1) added to (ax, ay)
+template <int SIGN>
+__device__ __forceinline__ void cauchy4(double zx, double zy, const double2 (&w)[4], double& ax, double& ay)
+{
+	double dx[4], dy[4], n[4];
+#pragma unroll
+	for (int i = 0; i < 4; i++)
+	{
+		dx[i] = zx - w[i].x;
+		dy[i] = zy - w[i].y;
+		n[i] = fma(dx[i], dx[i], fma(dy[i], dy[i], NORM_FLOOR));
+	}
+	const double p = n[0] * n[1], q = n[2] * n[3];
+	const double x01 = fma(dx[0], n[1], dx[1] * n[0]), y01 = fma(dy[0], n[1], dy[1] * n[0]);
+	const double x23 = fma(dx[2], n[3], dx[3] * n[2]), y23 = fma(dy[2], n[3], dy[3] * n[2]);
+	const double iv = SIGN * rcp64_cubic(p * q);
+	ax = fma(fma(x01, q, x23 * p), iv, ax);
+	ay = fma(fma(y01, q, y23 * p), iv, ay);
+}
+
+// one Cauchy term times SIGN; d = 0 gives zero
+template <int SIGN>
+__device__ __forceinline__ void cauchy1(double zx, double zy, double2 w, double& ax, double& ay)
+{
+	const double dx = zx - w.x, dy = zy - w.y;
+	const double iv = SIGN * rcp64(fmax(fma(dx, dx, dy * dy), 1e-300));
+	ax = fma(dx, iv, ax);
+	ay = fma(dy, iv, ay);
+}
+
+// the terms of src[lo, hi) for a lane's target: every lane of the wave reads
+// the same source, so the sources come through scalar loads
+template <int SIGN>
+__device__ __forceinline__ void cauchy_run(const double2* __restrict__ src, int lo, int hi, double zx, double zy, double& ax,
+	double& ay)
+{
+	int q = lo;
+#pragma unroll 2
+	for (; q + 4 <= hi; q += 4)
+	{
+		const double2 w[4] = {src[q], src[q + 1], src[q + 2], src[q + 3]};
+		cauchy4<SIGN>(zx, zy, w, ax, ay);
+	}
+	for (; q < hi; q++) cauchy1<SIGN>(zx, zy, src[q], ax, ay);
+}
+
+// the same terms of one target, the wave's lanes over the sources (four of
+// its own at a time): the lane's part of the sum
+template <int SIGN>
+__device__ __forceinline__ void cauchy_lanes(const double2* __restrict__ src, int lo, int hi, double zx, double zy, double& ax,
+	double& ay)
+{
+	const int lane = threadIdx.x & 63;
+	int q0 = lo;
+#pragma unroll 1
+	for (; q0 + 256 <= hi; q0 += 256)
+	{
+		const double2 w[4] = {src[q0 + lane], src[q0 + 64 + lane], src[q0 + 128 + lane], src[q0 + 192 + lane]};
+		cauchy4<SIGN>(zx, zy, w, ax, ay);
+	}
+#pragma unroll 1
+	for (int q = q0 + lane; q < hi; q += 64) cauchy1<SIGN>(zx, zy, src[q], ax, ay);
+}
+
+// One wave takes an item, a tile of QUAD_TILE listed roots and a slice of
+// the terms, by itself: no LDS and no barrier. A row with at most QUAD_SPARSE
+// listed roots has the wave's lanes over the slice's sources instead of over
+// the targets (a slice stays in the CU's cache over them). The form goes by
+// the row, not by the tile: a root's place in the list follows from the
+// order of atomics, and its sum must not.
+constexpr int QUAD_TILE = 64;
+constexpr int QUAD_SPARSE = 24;
+
+__global__ __launch_bounds__(BLOCK, 8) void k_sums64_quad(const double2* __restrict__ spos, int Np,
+	const double2* __restrict__ roots, RowMap M, SweepView V, int nrows)
+{
+	const int tiles = V.plan[0], S = V.plan[1];
+	const int items = tiles * S;
+	const int R = M.R;
+	const int lane = threadIdx.x & 63;
+	const long long Lt = (long long)Np + R;
+	for (int item = __builtin_amdgcn_readfirstlane(blockIdx.x * (BLOCK / 64) + (threadIdx.x >> 6)); item < items;
+		 item += gridDim.x * (BLOCK / 64))
+	{
+		const int g = item / S, s = item - g * S;
+		const int r = row_of_tile(V.tile_off, nrows, g);
+		const int t = g - V.tile_off[r];
+		const int nf = V.fcnt[r], nt = nf - t * QUAD_TILE; // the row's listed roots and the tile's, at least one
+		int row;
+		double phi;
+		M.get(r, row, phi);
+		const double2* __restrict__ xrow = roots + (size_t)row * R;
+		const int* __restrict__ fl = V.fl + (size_t)r * R + (size_t)t * QUAD_TILE;
+		double2* __restrict__ part = V.part + (size_t)item * QUAD_TILE;
+		const long long lo = s * Lt / S, hi = (s + 1) * Lt / S;
+		const int s0 = (int)lo, s1 = (int)min(hi, (long long)Np);
+		const int r0 = (int)(max(lo, (long long)Np) - Np), r1 = (int)(hi - Np);
+		if (nf <= QUAD_SPARSE)
+		{
+#pragma unroll 1
+			for (int k = 0; k < nt; k++)
+			{
+				const double2 z = xrow[fl[k]];
+				double ax = 0, ay = 0;
+				cauchy_lanes<1>(spos, s0, s1, z.x, z.y, ax, ay);
+				ax *= 2;
+				ay *= 2;
+				cauchy_lanes<-1>(xrow, r0, r1, z.x, z.y, ax, ay);
+				if (!(isfinite(ax) && isfinite(ay)))
+				{
+					// out of cauchy4's range: the lane's terms one by one
+					ax = ay = 0;
+					for (int q = s0 + lane; q < s1; q += 64) cauchy1<1>(z.x, z.y, spos[q], ax, ay);
+					ax *= 2;
+					ay *= 2;
+					for (int q = r0 + lane; q < r1; q += 64) cauchy1<-1>(z.x, z.y, xrow[q], ax, ay);
+				}
+				for (int o = 32; o >= 1; o >>= 1)
+				{
+					ax += __shfl_xor(ax, o, 64);
+					ay += __shfl_xor(ay, o, 64);
+				}
+				if (lane == 0) part[k] = make_double2(ax, -ay);
+			}
+			continue;
+		}
+		const double2 z = xrow[fl[lane < nt ? lane : 0]];
+		double ax = 0, ay = 0;
+		cauchy_run<1>(spos, s0, s1, z.x, z.y, ax, ay); // ccf_functions.cuh:218-227
+		ax *= 2;
+		ay *= 2;
+		cauchy_run<-1>(xrow, r0, r1, z.x, z.y, ax, ay); // ccf_functions.cuh:232-239
+		if (!(isfinite(ax) && isfinite(ay)))
+		{
+			// out of cauchy4's range: the terms one by one
+			ax = ay = 0;
+			for (int q = s0; q < s1; q++) cauchy1<1>(z.x, z.y, spos[q], ax, ay);
+			ax *= 2;
+			ay *= 2;
+			for (int q = r0; q < r1; q++) cauchy1<-1>(z.x, z.y, xrow[q], ax, ay);
+		}
+		part[lane] = make_double2(ax, -ay);
 	}
 }
 
@@ -1044,10 +1240,15 @@ __global__ __launch_bounds__(BLOCK) void k_finalize(double theta, double2* __res
 		}
 		else
 		{
-			for (int s = 0; s < S; s++)
+			// in slice order, eight loads at a time
+			for (int s0 = 0; s0 < S; s0 += 8)
 			{
-				const double2 q = V.part[(g * S + s) * V.tile + loc];
-				sum += cd(q.x, q.y);
+				double2 q[8];
+#pragma unroll
+				for (int k = 0; k < 8; k++) q[k] = V.part[(g * S + min(s0 + k, S - 1)) * V.tile + loc];
+#pragma unroll
+				for (int k = 0; k < 8; k++)
+					if (s0 + k < S) sum += cd(q[k].x, q[k].y);
 			}
 		}
 		if (V.slot) V.slot[(size_t)r * R + a] = -1;
@@ -1562,26 +1763,67 @@ __global__ void k_generate_stars(int n, unsigned long long seed, int rect, doubl
 
 // ---------------------------------------------------------------------------
 
-struct SumsLaunch
+// the kernel that forms a sweep's Cauchy sums
+enum SumsForm
 {
-	int grid = 0;
-	int target = 0;
-	int rpt = 2;
+	SUMS_32,      // k_sums32 (mixed form)
+	SUMS_64,      // k_sums64: the FP64 form's branch centres
+	SUMS_64_QUAD, // k_sums64_quad: its continuation steps and single sweeps
 };
 
-SumsLaunch sums_launch(ccf_ctx* ctx, bool f32)
+struct SumsLaunch
+{
+	SumsForm form = SUMS_32;
+	int grid = 0;
+	int target = 0;    // items (tile, slice) a sweep's plan aims at
+	int min_slice = 0; // fewest terms of a slice
+	int rpt = 0;       // roots per thread of SUMS_32 and SUMS_64
+	int tile = 0;      // listed roots of a tile: a workgroup's, or of SUMS_64_QUAD a wave's
+};
+
+SumsLaunch sums_launch(ccf_ctx* ctx, SumsForm form)
 {
 	SumsLaunch l;
-	l.rpt = ctx->P.roots_per_thread > 0 ? ctx->P.roots_per_thread : 2;
+	l.form = form;
+	l.rpt = ctx->P.roots_per_thread > 0 ? ctx->P.roots_per_thread : ROOTS_PER_THREAD;
 	int per_cu = 0;
 	const void* fn;
-	if (f32) fn = l.rpt == 1 ? (const void*)k_sums32<1> : (l.rpt == 4 ? (const void*)k_sums32<4> : (const void*)k_sums32<2>);
+	if (form == SUMS_64_QUAD) fn = (const void*)k_sums64_quad;
+	else if (form == SUMS_32) fn = l.rpt == 1 ? (const void*)k_sums32<1> : (l.rpt == 4 ? (const void*)k_sums32<4> : (const void*)k_sums32<2>);
 	else fn = l.rpt == 1 ? (const void*)k_sums64<1> : (l.rpt == 4 ? (const void*)k_sums64<4> : (const void*)k_sums64<2>);
 	if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, BLOCK, 0) != hipSuccess || per_cu < 1) per_cu = 2;
 	const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
 	l.grid = cus * per_cu;
-	l.target = 4 * l.grid;
+	if (form == SUMS_64_QUAD)
+	{
+		l.tile = QUAD_TILE;
+		l.min_slice = QUAD_MIN_SLICE;
+		l.target = l.grid * (BLOCK / 64); // the waves the device holds
+	}
+	else
+	{
+		l.tile = BLOCK * l.rpt;
+		l.min_slice = MIN_SLICE;
+		l.target = 4 * l.grid;
+	}
 	return l;
+}
+
+inline SumsForm sums_form(const ccf_ctx* ctx, const RowMap& M)
+{
+	if (ctx->P.precision == 1) return SUMS_32;
+	return M.rows_per_branch == 1 ? SUMS_64 : SUMS_64_QUAD;
+}
+
+// the partial sums of a sweep over `rows` rows of R roots and `terms` terms:
+// the most tiles times slices that plan_sums can make of them, times the tile
+inline size_t sums_room(const SumsLaunch& l, int rows, int R, int terms)
+{
+	const long long tiles = (long long)rows * ((R + l.tile - 1) / l.tile);
+	const long long s = std::min(MAX_SLICES, std::max(1, terms / l.min_slice));
+	if (l.form == SUMS_64_QUAD)
+		return (size_t)std::max(std::min(tiles * s, (long long)l.target), tiles * std::min(s, (long long)QUAD_SLICES)) * l.tile;
+	return (size_t)(std::min(tiles * s, tiles + l.target) + tiles) * l.tile;
 }
 
 // `cap` sweeps over the rows of M (ccf.cuh:929-939 and 1013-1018): the
@@ -1639,7 +1881,8 @@ bool run_sweeps_groups(ccf_ctx* ctx, SweepGroup* gs, int G, double2* roots, int 
 	const bool fmm_pole = f32 && ctx->tree.order > 0;
 	const int circ_exact = (!ctx->rectangular && !ctx->P.approx) ? 1 : 0;
 	const int Np = fmm_pole ? 0 : ctx->num_stars;
-	const SumsLaunch sl = sums_launch(ctx, f32);
+	// the groups of a call are in one phase
+	const SumsLaunch sl = sums_launch(ctx, sums_form(ctx, gs[0].M));
 	ctx->fmm_rows_sweep[0] = ctx->fmm_rows_sweep[1] = -1; // unknown until a read-back
 	int rows_total = 0, left = 0;
 	for (int g = 0; g < G; g++)
@@ -1650,7 +1893,7 @@ bool run_sweeps_groups(ccf_ctx* ctx, SweepGroup* gs, int G, double2* roots, int 
 			return false;
 		}
 		left += !gs[g].done;
-		if (gs[g].B->tile != BLOCK * sl.rpt)
+		if (gs[g].B->part_room < sums_room(sl, gs[g].nrows, gs[g].M.R, Np + gs[g].M.R))
 		{
 			ctx->fail("Error. sweep buffers were sized for another tile\n");
 			return false;
@@ -1708,10 +1951,10 @@ bool run_sweeps_groups(ccf_ctx* ctx, SweepGroup* gs, int G, double2* roots, int 
 			hipStream_t s = q.s;
 			const dim3 g_rows(grid(R), nrows);
 			const dim3 g_witt(xcd_round(grid(R)), nrows);
-			const SweepView V = view(B, it & 1);
+			const SweepView V = view(B, it & 1, sl.tile);
 			const bool fmm = B.grid.order > 0 && it < 32 && ((q.fmm_mask >> it) & 1u);
 			q.fmm_any = q.fmm_any || fmm;
-			const PlanArgs plan{nrows, Np + R, sl.target, fmm ? root_fmm_min(R) : 0, it};
+			const PlanArgs plan{nrows, Np + R, sl.target, fmm ? root_fmm_min(R) : 0, it, sl.tile, sl.form == SUMS_64_QUAD ? 1 : 0};
 			ccf::Timer tw;
 			if (ctx->P.timing)
 			{
@@ -1741,6 +1984,10 @@ bool run_sweeps_groups(ccf_ctx* ctx, SweepGroup* gs, int G, double2* roots, int 
 				if (sl.rpt == 1) k_sums32<1><<<sl.grid, BLOCK, 0, s>>>(ctx->spos32, Np, roots, M, V, nrows, cd2, ctx->counters);
 				else if (sl.rpt == 4) k_sums32<4><<<sl.grid, BLOCK, 0, s>>>(ctx->spos32, Np, roots, M, V, nrows, cd2, ctx->counters);
 				else k_sums32<2><<<sl.grid, BLOCK, 0, s>>>(ctx->spos32, Np, roots, M, V, nrows, cd2, ctx->counters);
+			}
+			else if (sl.form == SUMS_64_QUAD)
+			{
+				k_sums64_quad<<<sl.grid, BLOCK, 0, s>>>(ctx->spos, Np, roots, M, V, nrows);
 			}
 			else
 			{
@@ -1785,7 +2032,7 @@ bool run_sweeps_groups(ccf_ctx* ctx, SweepGroup* gs, int G, double2* roots, int 
 					}
 				}
 				if (before_tail && !before_tail(q.id)) return false;
-				const SweepView Vn = view(B, (it + 1) & 1);
+				const SweepView Vn = view(B, (it + 1) & 1, sl.tile);
 				const double d = CLUSTER_REL * ctx->root_half_length;
 				ccf::Timer tt;
 				if (ctx->P.timing)
@@ -1856,35 +2103,28 @@ bool run_sweeps(ccf_ctx* ctx, SweepBufs& B, double2* roots, const RowMap& M, int
 // The sweep buffers of `rows` rows of R roots (and, when the root-sum FMM
 // applies, its grid over the field): take(p, count) provides each array of
 // count elements, from the context's device pool or from a slice of the
-// fixed scratch array. exact_items sizes the split-K partials for the plan
-// plan_sums can make for these terms (at most MAX_SLICES slices of at least
-// MIN_SLICE terms per tile, ceil(target / tiles) wanted); otherwise for any
-// slice count up to the target.
+// fixed scratch array.
 template <class Take>
 bool root_layout(ccf_ctx* ctx, SweepBufs& b, Take&& take);
 
 template <class Take>
-bool sweep_layout(ccf_ctx* ctx, SweepBufs& b, int rows, int R, bool exact_items, Take&& take)
+bool sweep_layout(ccf_ctx* ctx, SweepBufs& b, int rows, int R, Take&& take)
 {
 	const bool f32 = ctx->P.precision == 1;
-	const SumsLaunch sl = sums_launch(ctx, f32);
 	b.rows = rows;
 	b.R = R;
-	b.tile = BLOCK * sl.rpt;
-	// items per sweep <= max(tiles, target) + tiles
-	const long long tiles_max = (long long)rows * ((R + b.tile - 1) / b.tile);
-	b.max_items = (int)(tiles_max + sl.target + tiles_max);
-	if (exact_items)
-	{
-		const int Np = (f32 && ctx->tree.order > 0) ? 0 : ctx->num_stars;
-		const long long scap = std::min(MAX_SLICES, std::max(1, (Np + R) / MIN_SLICE));
-		b.max_items = (int)(std::min(tiles_max * scap, tiles_max + sl.target) + tiles_max);
-	}
+	// the partials of every kernel the buffers can be used with (before the
+	// tree is built its order is 0, and the stars count)
+	const int terms = ((f32 && ctx->tree.order > 0) ? 0 : ctx->num_stars) + R;
+	b.part_room = 0;
+	for (SumsForm form : {SUMS_32, SUMS_64, SUMS_64_QUAD})
+		if ((form == SUMS_32) == f32)
+			b.part_room = std::max(b.part_room, sums_room(sums_launch(ctx, form), rows, R, terms));
 	const size_t list = (size_t)rows * R;
 	if (!(take(b.act, 2 * list) && take(b.cnt, 2 * (size_t)rows) && take(b.fl, list) && take(b.fcnt, 2 * (size_t)rows) &&
 			take(b.f0, list) && take(b.f1, list) && take(b.ex, list) &&
 			take(b.tile_off, (size_t)rows + 1) && take(b.plan, 4) && take(b.ticket, 1) &&
-			take(b.part, (size_t)b.max_items * b.tile)))
+			take(b.part, b.part_room)))
 		return false;
 	if (ctx->P.root_fmm != 1 || R < ROOT_FMM_MIN_ROOTS) return true;
 	return root_layout(ctx, b, take);
@@ -1948,7 +2188,7 @@ bool alloc_sweep(ccf_ctx* ctx, SweepBufs& b, int rows, int R)
 {
 	free_sweep(ctx, b);
 	auto take = [ctx](auto*& p, size_t count) { return CCF_HIP(ctx, ctx->dmalloc(&p, count * sizeof(*p))); };
-	if (!sweep_layout(ctx, b, rows, R, false, take)) return false;
+	if (!sweep_layout(ctx, b, rows, R, take)) return false;
 	const size_t list = (size_t)rows * R;
 	if (!CCF_HIP(ctx, hipMemsetAsync(b.cnt, 0, 2 * rows * sizeof(int), ctx->stream)) ||
 		!CCF_HIP(ctx, hipMemsetAsync(b.fcnt, 0, 2 * rows * sizeof(int), ctx->stream)) ||
@@ -2114,7 +2354,7 @@ bool autotune_dev(ccf_ctx* ctx, int verbose)
 					  << " ms\n";
 		return good;
 	};
-	int best_rpt = sums_launch(ctx, ctx->P.precision == 1).rpt;
+	int best_rpt = ctx->P.roots_per_thread > 0 ? ctx->P.roots_per_thread : ROOTS_PER_THREAD;
 	int best_order = ctx->P.root_fmm_order > 0 ? ctx->P.root_fmm_order : ROOT_FMM_ORDER;
 	int best_leaf = ctx->P.root_fmm_leaf > 0 ? ctx->P.root_fmm_leaf : ROOT_FMM_LEAF;
 	float best = 1e30f;
@@ -2417,7 +2657,7 @@ bool find_ccs_dev(ccf_ctx* ctx, int verbose)
 		ctx->info.root_fmm_order = g.order;
 		ctx->info.root_fmm_leaf_level = g.leaf;
 		ctx->info.root_fmm_leaf = g.order > 0 ? (ctx->P.root_fmm_leaf > 0 ? ctx->P.root_fmm_leaf : ROOT_FMM_LEAF) : 0;
-		ctx->info.roots_per_thread = sums_launch(ctx, ctx->P.precision == 1).rpt;
+		ctx->info.roots_per_thread = ctx->P.roots_per_thread > 0 ? ctx->P.roots_per_thread : ROOTS_PER_THREAD;
 		// the tails: every evaluation forms f0 and f1 (mixed form), every
 		// full update sums the row (and the stars without the FMM pole sum)
 		const double tail_evals = (double)(c[C_TAIL_FULL] + c[C_TAIL_EARLY] + c[C_TAIL_NEWTON]);
@@ -2628,7 +2868,7 @@ bool aberth_sweep_noalloc_dev(ccf_ctx* ctx, const double* roots, int n, double p
 	double2* row = nullptr;
 	ScratchCarve size{nullptr};
 	size(row, (size_t)n);
-	if (!sweep_layout(ctx, B, 1, n, true, size)) return false;
+	if (!sweep_layout(ctx, B, 1, n, size)) return false;
 	if (size.used > NOALLOC_SCRATCH_BYTES)
 	{
 		ctx->fail("Error. ccf_aberth_sweep_noalloc: a sweep of " + std::to_string(n) + " roots needs " + std::to_string(size.used) +
@@ -2638,7 +2878,7 @@ bool aberth_sweep_noalloc_dev(ccf_ctx* ctx, const double* roots, int n, double p
 	B = SweepBufs{};
 	ScratchCarve carve{base};
 	carve(row, (size_t)n);
-	if (!sweep_layout(ctx, B, 1, n, true, carve)) return false;
+	if (!sweep_layout(ctx, B, 1, n, carve)) return false;
 	hipStream_t s = ctx->stream;
 	// the Witt kernel's ticket starts at 0, the slots of listed roots at -1,
 	// the row's FMM mode at 0; k_prepare sets the active list and clears the
