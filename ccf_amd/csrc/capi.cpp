@@ -165,8 +165,6 @@ void ccf_ctx::free_device()
 	ccf::free_sweep(this, sw);
 	for (ccf::SweepBufs& b : swg) ccf::free_sweep(this, b);
 	F(counters);
-	if (host_counts) (void)hipHostFree(host_counts);
-	host_counts = nullptr;
 	// the events themselves live until ccf_destroy
 	timers.clear();
 	witt_timers.clear();
@@ -698,8 +696,11 @@ void ccf_destroy(ccf_ctx* c)
 	for (hipEvent_t e : c->events) (void)hipEventDestroy(e);
 	for (hipEvent_t e : c->fmm_rows_event)
 		if (e) (void)hipEventDestroy(e);
+	for (hipEvent_t e : c->step_event)
+		if (e) (void)hipEventDestroy(e);
 	for (hipEvent_t e : c->read_event)
 		if (e) (void)hipEventDestroy(e);
+	if (c->host_counts) (void)hipHostFree(c->host_counts);
 	if (c->host_stage) (void)hipHostFree(c->host_stage);
 	if (c->err_event) (void)hipEventDestroy(c->err_event);
 	if (c->err_stream) (void)hipStreamDestroy(c->err_stream);

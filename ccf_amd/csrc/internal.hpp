@@ -41,6 +41,10 @@ constexpr int MAX_ROOT_GRID_LEVELS = 10;
 // default; streams that share a queue serialise.
 constexpr int CONT_GROUPS = 3;
 constexpr int CONT_STEP_GROUPS = 2;
+// sweeps of a continuation step whose counts are tracked (SweepBufs::plan), and
+// the steps whose counts the host keeps, per group
+constexpr int TRACK_SWEEPS = 32;
+constexpr int TRACK_STEPS = 4;
 
 // Quadtree over the stars, structure of arrays indexed by node id. Nodes of
 // a level are contiguous ([level_off[l], level_off[l] + level_cnt[l])) and
@@ -154,7 +158,8 @@ struct SweepBufs
 	double2* f1 = nullptr;   // [rows][R] its z-derivative
 	double2* ex = nullptr;   // [rows][R] terms of the Aberth sum formed per root
 	int* tile_off = nullptr; // [rows + 1] first tile of each row
-	int* plan = nullptr;     // [4] tiles, slices per tile; rows summed by the root-sum FMM in a phase's first and second sweep
+	int* plan = nullptr;     // [4 + 2 TRACK_SWEEPS] tiles, slices per tile; rows summed by the root-sum FMM in a phase's
+	                         // first and second sweep; the most roots of a row active at each sweep's start and listed in it
 	int* ticket = nullptr;   // [1] workgroups of the sweep's Witt kernel done (the last forms the plan and resets it)
 	double2* part = nullptr; // [items of a sweep][tile] partial Cauchy sums
 	// root-sum FMM (grid.order > 0 only)
@@ -242,11 +247,14 @@ struct ccf_ctx
 		}
 		return events[events_used++];
 	}
-	int* host_counts = nullptr;   // pinned: active roots per row, the two FMM row counts of a read-back, then per continuation group two slots of two for the mixed continuation
+	int* host_counts = nullptr;   // pinned, coherent: active roots per row, the two FMM row counts of a read-back, then per continuation group two slots of two for the mixed continuation
 	int tree_hint_stars = -1, tree_hint_fields = -1, tree_hint_nodes = 0; // the last tree build's node count
 	double* host_stage = nullptr; // pinned (STAGE_DOUBLES), until ccf_destroy: a tree build's level counts and binomial table, a run's folded statistics
 	hipStream_t err_stream = nullptr; // the error pass of find_ccs, beside the continuation (default priority)
 	hipEvent_t err_event = nullptr;   // a row set's roots are final (no timing)
+	size_t host_counts_size = 0;  // ints host_counts holds: kept from run to run, grown when one needs more
+	int* host_track = nullptr; // its last part: [CONT_GROUPS][TRACK_STEPS][2 TRACK_SWEEPS] the tracked counts of a group's last steps
+	hipEvent_t step_event[2 * ccf::CONT_GROUPS] = {}; // mixed continuation: before a step's tail, per group and parity (no timing)
 	hipEvent_t fmm_rows_event[2 * ccf::CONT_GROUPS] = {}; // mixed continuation: after the copy of a step's FMM row count, per group (no timing)
 	hipEvent_t read_event[ccf::CONT_GROUPS] = {}; // after the copy of a sweep's active counts, per group (no timing)
 	hipStream_t group_streams[ccf::CONT_GROUPS - 1] = {}; // mixed form: the streams of the groups of branches after the first (default priority)

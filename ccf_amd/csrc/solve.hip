@@ -414,18 +414,31 @@ __device__ inline Near coop_near(const LensView& L, int node, cd z, double (*red
 // from the FMM pass instead and gets no tiles. Formed by the last workgroup
 // of k_witt to finish, once every row's listed count is final.
 
+// the kernel that forms a sweep's Cauchy sums
+enum SumsForm
+{
+	SUMS_32,      // k_sums32 (mixed form)
+	SUMS_32_TAIL, // k_sums32_tail: its continuation steps' later sweeps
+	SUMS_64,      // k_sums64: the FP64 form's branch centres
+	SUMS_64_QUAD, // k_sums64_quad: its continuation steps and single sweeps
+};
+
 struct PlanArgs
 {
-	int nrows, terms, target, fmm_min, sweep, tile, quad;
+	int nrows, terms, target, fmm_min, sweep, tile;
+	SumsForm form;
 };
+// (SUMS_32_TAIL: a tile is what a workgroup of TAIL_WAVES waves takes at a
+// time, several waves a root when few are listed)
+constexpr int TAIL_WAVES = 8;
 
 __device__ inline void plan_sums(SweepView V, const PlanArgs& P)
 {
 	const int nrows = P.nrows, terms = P.terms, target = P.target, fmm_min = P.fmm_min, sweep = P.sweep;
 	__shared__ int wsum[16];
-	__shared__ int carry, nfmm;
+	__shared__ int carry, nfmm, amax, lmax;
 	const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
-	if (threadIdx.x == 0) carry = nfmm = 0;
+	if (threadIdx.x == 0) carry = nfmm = amax = lmax = 0;
 	__syncthreads();
 	for (int base = 0; base < nrows; base += blockDim.x)
 	{
@@ -436,8 +449,15 @@ __device__ inline void plan_sums(SweepView V, const PlanArgs& P)
 		if (fmm) atomicAdd(&nfmm, 1);
 		// this sweep's active count is consumed (k_witt read it): cleared
 		// here, it is the list the next sweep's k_witt appends stepped roots to
-		if (r < nrows) V.cnt[r] = 0;
-		const int v = (r < nrows && !fmm) ? (nf + P.tile - 1) / P.tile : 0;
+		if (r < nrows)
+		{
+			atomicMax(&amax, V.cnt[r]);
+			atomicMax(&lmax, nf);
+			V.cnt[r] = 0;
+		}
+		int tile = P.tile;
+		if (P.form == SUMS_32_TAIL) tile = nf >= TAIL_WAVES ? TAIL_WAVES : (nf >= TAIL_WAVES / 2 ? TAIL_WAVES / 2 : (nf >= TAIL_WAVES / 4 ? TAIL_WAVES / 4 : 1));
+		const int v = (r < nrows && !fmm) ? (nf + tile - 1) / tile : 0;
 		int x = v;
 		for (int d = 1; d < 64; d <<= 1)
 		{
@@ -461,7 +481,8 @@ __device__ inline void plan_sums(SweepView V, const PlanArgs& P)
 	{
 		const int tiles = carry;
 		int S = 1;
-		if (P.quad)
+		if (P.form == SUMS_32_TAIL) S = 0; // the sums come in ex
+		else if (P.form == SUMS_64_QUAD)
 		{
 			// as many items as the device holds waves, all in one round
 			if (tiles > 0) S = 2 * tiles <= target ? target / tiles : QUAD_SLICES;
@@ -478,6 +499,11 @@ __device__ inline void plan_sums(SweepView V, const PlanArgs& P)
 		V.plan[1] = S;
 		// FMM rows of the phase's first and second sweep (cleared by k_prepare)
 		if (sweep < 2 && nfmm) V.plan[2 + sweep] += nfmm;
+		if (sweep < TRACK_SWEEPS)
+		{
+			V.plan[4 + sweep] = amax;
+			V.plan[4 + TRACK_SWEEPS + sweep] = lmax;
+		}
 	}
 }
 
@@ -533,6 +559,45 @@ __device__ inline Near wave_near(const LensView& L, int node, cd z)
 	return nr;
 }
 
+// The same sums in k_tail's order (coop_near over TAIL_WAVES waves): the wave
+// takes each of those waves' stars in turn, and adds their sums in wave order.
+__device__ inline Near wave_near_tail(const LensView& L, int node, cd z)
+{
+	Near sum;
+	const int lane = threadIdx.x & 63;
+	const int ranges = L.nnf[node];
+#pragma unroll 1
+	for (int w = 0; w < TAIL_WAVES; w++)
+	{
+		Near nr;
+		for (int k = 0; k < ranges; k++)
+		{
+			const int2 rg = L.nf[node * MAX_NEAR_RANGES + k];
+			for (int s = rg.x + w * 64 + lane; s < rg.x + rg.y; s += 64 * TAIL_WAVES)
+			{
+				const double2 q = L.spos[s];
+				const cd t = cd(z.re - q.x, z.im - q.y).inv();
+				nr.s0 += t;
+				const cd t1 = t * L.smass[s];
+				nr.s1 += t1;
+				const cd t2 = t1 * t;
+				nr.s2 += t2;
+				nr.s3 += t2 * t;
+			}
+			if (w == 0) sum.count += rg.y;
+		}
+		double v[8] = {nr.s0.re, nr.s0.im, nr.s1.re, nr.s1.im, nr.s2.re, nr.s2.im, nr.s3.re, nr.s3.im};
+#pragma unroll
+		for (int q = 0; q < 8; q++)
+			for (int o = 32; o >= 1; o >>= 1) v[q] += __shfl_xor(v[q], o, 64);
+		sum.s0 += cd(v[0], v[1]);
+		sum.s1 += cd(v[2], v[3]);
+		sum.s2 += cd(v[4], v[5]);
+		sum.s3 += cd(v[6], v[7]);
+	}
+	return sum;
+}
+
 // Counts of a workgroup's Witt evaluations (block_stats adds them to the
 // device counters)
 struct EvalCounts
@@ -544,10 +609,11 @@ struct EvalCounts
 // (witt_root), called by every lane of a wave (valid: the lane has a root).
 // A root outside the tree (whose near field is every star,
 // tree_node.cuh:529-561) takes its near-field sums from its whole wave
-// (wave_near), one such root at a time.
+// (wave_near, or late, in a continuation step's later sweeps, in k_tail's
+// order), one such root at a time.
 template <bool MIXED>
 __device__ __forceinline__ int witt_eval(const LensView& L, double2* xrow, int a, bool valid, double cp, double sp, int circ_exact,
-	int fmm_pole, int newton, cd& f0, cd& f1, cd& ex, EvalCounts& c)
+	int fmm_pole, int newton, bool late, cd& f0, cd& f1, cd& ex, EvalCounts& c)
 {
 	double2* const p = xrow + a;
 	cd z;
@@ -562,7 +628,9 @@ __device__ __forceinline__ int witt_eval(const LensView& L, double2* xrow, int a
 	for (unsigned long long m = __ballot(outside); m; m &= m - 1)
 	{
 		const int src = __ffsll(m) - 1;
-		const Near t = wave_near(L, __shfl(node, src, 64), cd(__shfl(z.re, src, 64), __shfl(z.im, src, 64)));
+		const int nd = __shfl(node, src, 64);
+		const cd zs(__shfl(z.re, src, 64), __shfl(z.im, src, 64));
+		const Near t = MIXED && late ? wave_near_tail(L, nd, zs) : wave_near(L, nd, zs);
 		if ((int)(threadIdx.x & 63) == src) nr = t;
 	}
 	if (!valid) return -1;
@@ -606,7 +674,7 @@ __device__ __forceinline__ void append_full(const SweepView& V, int r, int R, in
 // sweep's Cauchy sums.
 template <bool MIXED>
 __global__ __launch_bounds__(BLOCK) void k_witt(LensView L, double2* __restrict__ roots, RowMap M, SweepView V,
-	unsigned long long* __restrict__ stats, int circ_exact, int fmm_pole, PlanArgs P)
+	unsigned long long* __restrict__ stats, int circ_exact, int fmm_pole, int twice, PlanArgs P)
 {
 	__shared__ int s_last;
 	const int2 sl = xcd_slot();
@@ -628,10 +696,10 @@ __global__ __launch_bounds__(BLOCK) void k_witt(LensView L, double2* __restrict_
 		const bool valid = i < n;
 		int a = valid ? V.act[(size_t)r * R + i] : 0;
 		cd f0, f1, ex;
-		const int st = witt_eval<MIXED>(L, xrow, a, valid, cp, sp, circ_exact, fmm_pole, M.j > 0, f0, f1, ex, c);
+		const int st = witt_eval<MIXED>(L, xrow, a, valid, cp, sp, circ_exact, fmm_pole, M.j > 0, !twice, f0, f1, ex, c);
 		append_full(V, r, R, a, st == ROOT_FULL, f0, f1, ex);
 		bool stepped = st == ROOT_STEPPED;
-		if (MIXED)
+		if (MIXED && twice)
 		{
 			// the workgroup's stepped roots, in thread order, to its first threads
 			__shared__ int s_a2[BLOCK];
@@ -654,7 +722,7 @@ __global__ __launch_bounds__(BLOCK) void k_witt(LensView L, double2* __restrict_
 			{
 				const bool v2 = (int)threadIdx.x < n2;
 				a = v2 ? s_a2[threadIdx.x] : 0;
-				const int st2 = witt_eval<MIXED>(L, xrow, a, v2, cp, sp, circ_exact, fmm_pole, 1, f0, f1, ex, c);
+				const int st2 = witt_eval<MIXED>(L, xrow, a, v2, cp, sp, circ_exact, fmm_pole, 1, false, f0, f1, ex, c);
 				append_full(V, r, R, a, st2 == ROOT_FULL, f0, f1, ex);
 				stepped = st2 == ROOT_STEPPED;
 			}
@@ -1280,15 +1348,170 @@ __global__ __launch_bounds__(BLOCK) void k_finalize(double theta, double2* __res
 // row's slice of act (both halves), fl, f0, f1 and ex (the sweep kernels are
 // done with them), so a row of any size fits. The waves of the workgroup
 // see each other's global writes across its barriers.
-constexpr int TAIL_BLOCK = 512;
+constexpr int TAIL_BLOCK = 64 * TAIL_WAVES;
 constexpr int TAIL_LDS = 128;
 constexpr int TAIL_DEFER = 64; // roots outside the tree per sweep taken by the whole workgroup
-// sweeps of a continuation step before the tail launch: the first sweep
-// evaluates every root of every row, which takes the whole device; after it
-// a row has a few per cent of its roots left, mostly ending by Newton steps,
-// which one workgroup per row finishes while the other group of branches'
-// first sweep fills the device
-constexpr int TAIL_AT = 1;
+// The sweeps of a continuation step before its tail launch. The first sweep
+// evaluates every root of every row, which takes the whole device; on a fine
+// phi grid a few per cent of a row's roots are left after it, mostly ending
+// by Newton steps, which one workgroup per row finishes while the other group
+// of branches' first sweep fills the device. On a coarse grid (steps of 2 pi
+// / 160: the predictor misses) most of a row is still active after it, and
+// one workgroup would evaluate it all, 25 us for every 512 roots. So a step
+// hands its rows over at the first sweep whose rows are small enough: by the
+// counts of TAIL_LAG steps before (tail_sweep), and in the first TAIL_LAG
+// steps by reading the counts back (TAIL_READ). 100 060 roots a row, 16 rows,
+// 10 steps of 2 pi / 160: the continuation takes 41 ms, 458 ms with every
+// tail after its first sweep; 20 000 roots a row in steps of 2 pi / 2000 take
+// it there from the sixth step on (14.8 ms, as with a fixed place).
+constexpr int EARLY_SWEEPS = 1; // one more while the predictor has fewer than two earlier steps
+constexpr int TAIL_LAG = 3;
+constexpr double TAIL_US = 100.0; // microseconds of a tail's first sweep below which it takes over
+constexpr int TAIL_READ = -1;
+constexpr int TAIL_ACTIVE = TAIL_BLOCK; // most active roots of a row that a read-back hands to the tail
+
+// waves of a TAIL_BLOCK workgroup that share a listed root's sums when nf
+// roots of its row are listed (a power of two)
+__device__ __forceinline__ int tail_waves(int nf)
+{
+	constexpr int NW = TAIL_WAVES;
+	return nf >= NW ? 1 : (nf >= NW / 2 ? 2 : (nf >= NW / 4 ? 4 : NW));
+}
+
+// 2 sum_stars 1/(z - s) - sum_roots 1/(z - w) of root a of a row (the parts'
+// real sums (x, y), y not yet negated) by wpt waves of the workgroup, wave
+// wv for its root wv / wpt, their lanes strided over the row; valid in lane
+// 0 of the root's first wave. Every thread of the workgroup calls it.
+constexpr int TAIL_LOADS = 8;
+
+struct TailSum
+{
+	double x, y;
+	int close; // the lane's terms formed in FP64
+};
+
+__device__ __forceinline__ TailSum tail_sum(const double2* __restrict__ xrow, int R, const float2* __restrict__ spos32, int Np, int a,
+	bool live, int wpt, float cluster_d2, double (*s_red)[8])
+{
+	int close = 0;
+	const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+	const int sub = wv % wpt, lanes = 64 * wpt, ln = sub * 64 + lane;
+	const double2 zg = xrow[a];
+	const float fx = (float)zg.x, fy = (float)zg.y;
+	float ax = 0, ay = 0, bx = 0, by = 0;
+	double cx = 0, cy = 0;
+	// TAIL_LOADS loads of a lane issued before their terms, which are summed
+	// in the order of the row
+#pragma unroll 1
+	for (int q0 = live ? ln : Np; q0 < Np; q0 += lanes * TAIL_LOADS)
+	{
+		float2 w[TAIL_LOADS];
+#pragma unroll
+		for (int u = 0; u < TAIL_LOADS; u++) w[u] = spos32[min(q0 + u * lanes, Np - 1)];
+#pragma unroll
+		for (int u = 0; u < TAIL_LOADS; u++)
+		{
+			if (q0 + u * lanes >= Np) continue;
+			const float dx = fx - w[u].x, dy = fy - w[u].y;
+			const float iv = __builtin_amdgcn_rcpf(fmaf(dx, dx, dy * dy));
+			ax = fmaf(dx, iv, ax);
+			ay = fmaf(dy, iv, ay);
+		}
+	}
+#pragma unroll 1
+	for (int q0 = live ? ln : R; q0 < R; q0 += lanes * TAIL_LOADS)
+	{
+		double2 wd[TAIL_LOADS];
+#pragma unroll
+		for (int u = 0; u < TAIL_LOADS; u++) wd[u] = xrow[min(q0 + u * lanes, R - 1)];
+#pragma unroll
+		for (int u = 0; u < TAIL_LOADS; u++)
+		{
+			const int q = q0 + u * lanes;
+			if (q >= R) continue;
+			const float dx = fx - (float)wd[u].x, dy = fy - (float)wd[u].y;
+			const float d2 = fmaf(dx, dx, dy * dy);
+			if (d2 < cluster_d2 && q != a)
+			{
+				const double ex = zg.x - wd[u].x, ey = zg.y - wd[u].y;
+				const double iv = rcp64(fmax(fma(ex, ex, ey * ey), 1e-300));
+				cx = fma(ex, iv, cx);
+				cy = fma(ey, iv, cy);
+				close++;
+			}
+			else
+			{
+				// the own root gives dx = dy = 0 and, floored, a zero term
+				const float iv = __builtin_amdgcn_rcpf(fmaxf(d2, 1e-30f));
+				bx = fmaf(dx, iv, bx);
+				by = fmaf(dy, iv, by);
+			}
+		}
+	}
+	double vx = 2.0 * (double)ax - ((double)bx + cx), vy = 2.0 * (double)ay - ((double)by + cy);
+	for (int o = 32; o >= 1; o >>= 1)
+	{
+		vx += __shfl_xor(vx, o, 64);
+		vy += __shfl_xor(vy, o, 64);
+	}
+	if (wpt > 1)
+	{
+		// the waves of a root add their sums in wave order
+		if (lane == 0)
+		{
+			s_red[wv][0] = vx;
+			s_red[wv][1] = vy;
+		}
+		__syncthreads();
+		if (lane == 0 && sub == 0)
+			for (int k = 1; k < wpt; k++)
+			{
+				vx += s_red[wv + k][0];
+				vy += s_red[wv + k][1];
+			}
+		__syncthreads();
+	}
+	return TailSum{vx, vy, close};
+}
+
+// The sums of a continuation step's later sweeps over the whole device: an
+// item is the listed roots of a row that a workgroup takes at a time, each
+// summed exactly as k_tail sums it (tail_sum), the whole Aberth sum left in
+// ex. A step's roots so do not depend on where its tail starts, which the
+// counts of earlier steps decide. Bound by the latency of the row's loads
+// when few roots are listed (a wave a root): TAIL_LOADS of them in flight
+// took the launch from 561 to 228 us on rows of 100 060 roots, and k_tail,
+// which shares the loop, from 106 to 74 us on rows of 20 000.
+__global__ __launch_bounds__(TAIL_BLOCK) void k_sums32_tail(const float2* __restrict__ spos32, int Np, const double2* __restrict__ roots,
+	RowMap M, SweepView V, int nrows, float cluster_d2, unsigned long long* __restrict__ stats)
+{
+	constexpr int NW = TAIL_BLOCK / 64;
+	__shared__ double s_red[NW][8];
+	const int tiles = V.plan[0], R = M.R;
+	const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+	unsigned long long nclus = 0;
+	for (int item = blockIdx.x; item < tiles; item += gridDim.x)
+	{
+		const int r = row_of_tile(V.tile_off, nrows, item);
+		const int nf = V.fcnt[r], wpt = tail_waves(nf);
+		const int g = (item - V.tile_off[r]) * (NW / wpt) + wv / wpt;
+		int row;
+		double phi;
+		M.get(r, row, phi);
+		const size_t k = (size_t)r * R + g;
+		const bool live = g < nf;
+		const int a = live ? V.fl[k] : 0;
+		const TailSum sum = tail_sum(roots + (size_t)row * R, R, spos32, Np, a, live, wpt, cluster_d2, s_red);
+		nclus += sum.close;
+		if (lane == 0 && wv % wpt == 0 && live)
+		{
+			const double2 e = V.ex[k];
+			V.ex[k] = make_double2(sum.x + e.x, -sum.y + e.y);
+		}
+	}
+	nclus = wave_sum(nclus);
+	if (lane == 0 && nclus) atomicAdd(stat_slot(stats, C_CLUSTER), nclus);
+}
 
 // k_tail: the outcome of root a's evaluation w, as in k_witt: listed for
 // the sums (entry k of the listed roots: LDS for k < TAIL_LDS, else the
@@ -1337,7 +1560,7 @@ __device__ __forceinline__ void tail_settle(const LensView& L, int a, double2* p
 
 __global__ __launch_bounds__(TAIL_BLOCK) void k_tail(LensView L, double2* __restrict__ roots, RowMap M, SweepView V,
 	unsigned long long* __restrict__ stats, int circ_exact, int fmm_pole, int cap, float cluster_d2,
-	const float2* __restrict__ spos32, int Np, double theta)
+	const float2* __restrict__ spos32, int Np, double theta, int first)
 {
 	__shared__ int s_a[2][TAIL_LDS];
 	__shared__ int s_fl[TAIL_LDS];
@@ -1417,7 +1640,11 @@ __global__ __launch_bounds__(TAIL_BLOCK) void k_tail(LensView L, double2* __rest
 	__syncthreads();
 	int n = s_nn;
 	__syncthreads();
-	if (threadIdx.x == 0) s_nn = 0;
+	if (threadIdx.x == 0)
+	{
+		s_nn = 0;
+		if (first < TRACK_SWEEPS) atomicMax(&V.plan[4 + first], n);
+	}
 	__syncthreads();
 	int p = 0;
 	for (int it = 0; it < cap && n > 0; it++)
@@ -1462,76 +1689,22 @@ __global__ __launch_bounds__(TAIL_BLOCK) void k_tail(LensView L, double2* __rest
 			__syncthreads();
 		}
 		const int nf = s_nf;
+		if (it == 0 && threadIdx.x == 0 && first < TRACK_SWEEPS) atomicMax(&V.plan[4 + TRACK_SWEEPS + first], nf);
 		// waves per listed root: all of them share the row when few roots
-		// are listed (a power of two, lanes strided over the row)
-		const int wpt = nf >= NW ? 1 : (nf >= NW / 2 ? 2 : (nf >= NW / 4 ? 4 : NW));
-		const int sub = wv % wpt, lanes = 64 * wpt, ln = sub * 64 + lane;
+		// are listed
+		const int wpt = tail_waves(nf);
 		for (int g0 = 0; g0 < nf; g0 += NW / wpt)
 		{
 			const int g = g0 + wv / wpt;
 			const bool live = g < nf;
 			const int a = live ? (g < TAIL_LDS ? s_fl[g] : gfl[g]) : 0;
-			const double2 zg = xrow[a];
-			const float fx = (float)zg.x, fy = (float)zg.y;
-			float ax = 0, ay = 0, bx = 0, by = 0;
-			double cx = 0, cy = 0;
-			for (int q = live ? ln : Np; q < Np; q += lanes)
-			{
-				const float2 w = spos32[q];
-				const float dx = fx - w.x, dy = fy - w.y;
-				const float iv = __builtin_amdgcn_rcpf(fmaf(dx, dx, dy * dy));
-				ax = fmaf(dx, iv, ax);
-				ay = fmaf(dy, iv, ay);
-			}
-			for (int q = live ? ln : R; q < R; q += lanes)
-			{
-				const double2 wd = xrow[q];
-				const float dx = fx - (float)wd.x, dy = fy - (float)wd.y;
-				const float d2 = fmaf(dx, dx, dy * dy);
-				if (d2 < cluster_d2 && q != a)
-				{
-					const double ex = zg.x - wd.x, ey = zg.y - wd.y;
-					const double iv = rcp64(fmax(fma(ex, ex, ey * ey), 1e-300));
-					cx = fma(ex, iv, cx);
-					cy = fma(ey, iv, cy);
-					nclus++;
-				}
-				else
-				{
-					// the own root gives dx = dy = 0 and, floored, a zero term
-					const float iv = __builtin_amdgcn_rcpf(fmaxf(d2, 1e-30f));
-					bx = fmaf(dx, iv, bx);
-					by = fmaf(dy, iv, by);
-				}
-			}
-			double vx = 2.0 * (double)ax - ((double)bx + cx), vy = 2.0 * (double)ay - ((double)by + cy);
-			for (int o = 32; o >= 1; o >>= 1)
-			{
-				vx += __shfl_xor(vx, o, 64);
-				vy += __shfl_xor(vy, o, 64);
-			}
-			if (wpt > 1)
-			{
-				// the waves of a root add their sums in wave order
-				if (lane == 0)
-				{
-					s_red[wv][0] = vx;
-					s_red[wv][1] = vy;
-				}
-				__syncthreads();
-				if (lane == 0 && sub == 0)
-					for (int k = 1; k < wpt; k++)
-					{
-						vx += s_red[wv + k][0];
-						vy += s_red[wv + k][1];
-					}
-				__syncthreads();
-			}
+			const TailSum sum = tail_sum(xrow, R, spos32, Np, a, live, wpt, cluster_d2, s_red);
+			nclus += sum.close;
 			// the whole Aberth sum: the root part (conjugated) and the terms formed per root
-			if (lane == 0 && sub == 0 && live)
+			if (lane == 0 && wv % wpt == 0 && live)
 			{
 				double2* e = g < TAIL_LDS ? &s_ex[g] : &gex[g];
-				*e = make_double2(vx + e->x, -vy + e->y);
+				*e = make_double2(sum.x + e->x, -sum.y + e->y);
 			}
 		}
 		__syncthreads();
@@ -1574,8 +1747,10 @@ __global__ __launch_bounds__(TAIL_BLOCK) void k_tail(LensView L, double2* __rest
 
 // initial roots of a phase: row centre+sgn*j from the rows of the previous
 // steps (prepare_roots_kernel, ccf_functions.cuh:261-295; order > 0
-// extrapolates), every root active, the sweep counters cleared
-__global__ void k_prepare(double2* roots, RowMap M, SweepBufs B, int order, const int* __restrict__ perm)
+// extrapolates), every root active, the sweep counters cleared. track (or
+// null): pinned host memory that takes the counts the group's previous step
+// tracked before they are cleared
+__global__ void k_prepare(double2* roots, RowMap M, SweepBufs B, int order, const int* __restrict__ perm, int* track)
 {
 	const int r = blockIdx.y;
 	const int R = M.R;
@@ -1605,7 +1780,13 @@ __global__ void k_prepare(double2* roots, RowMap M, SweepBufs B, int order, cons
 			B.plan[3] = 0;
 		}
 	}
+	if (r == 0 && a < 2 * TRACK_SWEEPS)
+	{
+		if (track) __hip_atomic_store(&track[a], B.plan[4 + a], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+		B.plan[4 + a] = 0;
+	}
 }
+static_assert(2 * TRACK_SWEEPS <= BLOCK, "k_prepare hands the tracked counts on with its first block");
 
 // 1/mu error bound at every point of the solved rows, reduced to its max
 // with a non-finite flag (find_errors_kernel + has_nan_err_kernel +
@@ -1763,14 +1944,6 @@ __global__ void k_generate_stars(int n, unsigned long long seed, int rect, doubl
 
 // ---------------------------------------------------------------------------
 
-// the kernel that forms a sweep's Cauchy sums
-enum SumsForm
-{
-	SUMS_32,      // k_sums32 (mixed form)
-	SUMS_64,      // k_sums64: the FP64 form's branch centres
-	SUMS_64_QUAD, // k_sums64_quad: its continuation steps and single sweeps
-};
-
 struct SumsLaunch
 {
 	SumsForm form = SUMS_32;
@@ -1861,6 +2034,8 @@ struct SweepGroup
 	int row0 = 0;       // first slot of its rows' active counts in a read-back
 	bool done = false;  // no root active, or handed to the tail launch
 	bool fmm_any = false;
+	int early = 1 << 30; // sweeps from this one on take the tail's form (one evaluation, tail_sum) wherever they run
+	int tail_at = 0;    // the sweep the tail launch starts at (0: no tail; TAIL_READ: read back first)
 };
 
 // `cap` sweeps over the rows of every group (ccf.cuh:929-939 and 1013-1018).
@@ -1869,10 +2044,10 @@ struct SweepGroup
 // sweeps may take the root sums of dense rows from the FMM pass (when the
 // buffers carry a root grid). A read-back (after sweep_check's sweeps)
 // waits for every group still running and stops the groups whose rows have
-// no active root. With tail_at, the sweeps after the first tail_at of each
-// group run in one tail launch, with no read-back; before_tail(g), when
-// set, runs once group g's first tail_at sweeps are queued.
-bool run_sweeps_groups(ccf_ctx* ctx, SweepGroup* gs, int G, double2* roots, int cap, int first_check = 3, int tail_at = 0,
+// no active root. A group with tail_at runs its sweeps from tail_at on in one
+// tail launch; before_tail(g), when set, runs once the sweeps before it are
+// queued.
+bool run_sweeps_groups(ccf_ctx* ctx, SweepGroup* gs, int G, double2* roots, int cap, int first_check = 3,
 	const std::function<bool(int)>& before_tail = {})
 {
 	ctx->phase_sweeps = cap;
@@ -1930,7 +2105,7 @@ bool run_sweeps_groups(ccf_ctx* ctx, SweepGroup* gs, int G, double2* roots, int 
 			if (ctx->sweep_verbose >= 3)
 				std::cout << "sweep " << it + 1 << (G > 1 ? ", group " + std::to_string(g) : std::string()) << ": " << active
 						  << " roots active, at most " << amax << " in a row\n";
-			if (active == 0)
+			if (active == 0 && q.tail_at != TAIL_READ)
 			{
 				q.done = true;
 				if (--left == 0) ended = it + 1;
@@ -1952,9 +2127,10 @@ bool run_sweeps_groups(ccf_ctx* ctx, SweepGroup* gs, int G, double2* roots, int 
 			const dim3 g_rows(grid(R), nrows);
 			const dim3 g_witt(xcd_round(grid(R)), nrows);
 			const SweepView V = view(B, it & 1, sl.tile);
-			const bool fmm = B.grid.order > 0 && it < 32 && ((q.fmm_mask >> it) & 1u);
+			const bool late = it >= q.early; // a sweep that the tail could have taken, in its form
+			const bool fmm = B.grid.order > 0 && !late && it < 32 && ((q.fmm_mask >> it) & 1u);
 			q.fmm_any = q.fmm_any || fmm;
-			const PlanArgs plan{nrows, Np + R, sl.target, fmm ? root_fmm_min(R) : 0, it, sl.tile, sl.form == SUMS_64_QUAD ? 1 : 0};
+			const PlanArgs plan{nrows, Np + R, sl.target, fmm ? root_fmm_min(R) : 0, it, sl.tile, late ? SUMS_32_TAIL : sl.form};
 			ccf::Timer tw;
 			if (ctx->P.timing)
 			{
@@ -1962,8 +2138,8 @@ bool run_sweeps_groups(ccf_ctx* ctx, SweepGroup* gs, int G, double2* roots, int 
 				tw.b = ctx->next_event();
 				if (tw.a) (void)hipEventRecord(tw.a, s);
 			}
-			if (f32) k_witt<true><<<g_witt, BLOCK, 0, s>>>(L, roots, M, V, ctx->counters, circ_exact, fmm_pole ? 1 : 0, plan);
-			else k_witt<false><<<g_witt, BLOCK, 0, s>>>(L, roots, M, V, ctx->counters, circ_exact, 0, plan);
+			if (f32) k_witt<true><<<g_witt, BLOCK, 0, s>>>(L, roots, M, V, ctx->counters, circ_exact, fmm_pole ? 1 : 0, late ? 0 : 1, plan);
+			else k_witt<false><<<g_witt, BLOCK, 0, s>>>(L, roots, M, V, ctx->counters, circ_exact, 0, 0, plan);
 			if (ctx->P.timing && tw.a && tw.b)
 			{
 				(void)hipEventRecord(tw.b, s);
@@ -1977,7 +2153,12 @@ bool run_sweeps_groups(ccf_ctx* ctx, SweepGroup* gs, int G, double2* roots, int 
 				if (tm.a) (void)hipEventRecord(tm.a, s);
 			}
 			if (fmm) root_fmm_pass(B, roots, M, nrows, ctx->counters, s);
-			if (f32)
+			if (f32 && late)
+			{
+				const double d = CLUSTER_REL * ctx->root_half_length;
+				k_sums32_tail<<<2 * ctx->num_cus, TAIL_BLOCK, 0, s>>>(ctx->spos32, Np, roots, M, V, nrows, (float)(d * d), ctx->counters);
+			}
+			else if (f32)
 			{
 				const double d = CLUSTER_REL * ctx->root_half_length;
 				const float cd2 = (float)(d * d);
@@ -2000,12 +2181,21 @@ bool run_sweeps_groups(ccf_ctx* ctx, SweepGroup* gs, int G, double2* roots, int 
 				(void)hipEventRecord(tm.b, s);
 				ctx->timers.push_back(tm);
 			}
-			// mixed form, continuation: the sweeps after the first tail_at of
-			// the step in one launch, with no read-back, which begins with
+			// a tail that waits for its counts: once the previous sweep left
+			// no row more active roots than TAIL_ACTIVE (this sweep's sums are
+			// queued meanwhile, so the device does not idle on the host)
+			if (q.tail_at == TAIL_READ && pend >= 0)
+			{
+				if (!CCF_HIP(ctx, hipEventSynchronize(ctx->read_event[q.id]))) return false;
+				int most = 0;
+				for (int r = 0; r < nrows; r++) most = std::max(most, ctx->host_counts[q.row0 + r]);
+				if (most <= TAIL_ACTIVE) q.tail_at = it + 1;
+			}
+			// mixed form, continuation: the sweeps from tail_at on in one launch, with no read-back, which begins with
 			// this sweep's updates. The rows the root-sum FMM took in the
 			// step's first two sweeps go to the host for the choice two steps
 			// later.
-			const bool tail_now = tail_at > 0 && it + 1 == tail_at && it + 1 < cap;
+			const bool tail_now = q.tail_at > 0 && it + 1 == q.tail_at && it + 1 < cap;
 			if (!tail_now) k_finalize<<<g_rows, BLOCK, 0, s>>>(ctx->theta, roots, M, V, ctx->counters);
 			if (!CCF_LAUNCH(ctx, "find_critical_curve_roots_kernel")) return false;
 			ctx->info.sweeps++;
@@ -2042,7 +2232,7 @@ bool run_sweeps_groups(ccf_ctx* ctx, SweepGroup* gs, int G, double2* roots, int 
 					if (tt.a && tt.b) (void)hipEventRecord(tt.a, s);
 				}
 				k_tail<<<nrows, TAIL_BLOCK, 0, s>>>(L, roots, M, Vn, ctx->counters, circ_exact, fmm_pole ? 1 : 0, cap - (it + 1),
-					(float)(d * d), ctx->spos32, Np, ctx->theta);
+					(float)(d * d), ctx->spos32, Np, ctx->theta, it + 1);
 				if (ctx->P.timing && tt.a && tt.b)
 				{
 					(void)hipEventRecord(tt.b, s);
@@ -2067,7 +2257,9 @@ bool run_sweeps_groups(ccf_ctx* ctx, SweepGroup* gs, int G, double2* roots, int 
 			if (!take_counts(pend)) return false;
 			pend = -1;
 		}
-		if (left > 0 && readback && (ctx->sweep_verbose >= 3 || sweep_check(it + 1, cap, first_check)))
+		bool tail_read = false; // a group whose tail waits for its counts: after every sweep
+		for (int g = 0; g < G; g++) tail_read = tail_read || (!gs[g].done && gs[g].tail_at == TAIL_READ);
+		if (left > 0 && readback && (ctx->sweep_verbose >= 3 || tail_read || sweep_check(it + 1, cap, first_check)))
 		{
 			for (int g = 0; g < G; g++)
 			{
@@ -2089,15 +2281,36 @@ bool run_sweeps_groups(ccf_ctx* ctx, SweepGroup* gs, int G, double2* roots, int 
 	return true;
 }
 
-// run_sweeps_groups for one group on `stream` (the context's by default),
-// with the host slots of group `group`
+// run_sweeps_groups for one group on the context's stream
 bool run_sweeps(ccf_ctx* ctx, SweepBufs& B, double2* roots, const RowMap& M, int nrows, int cap, unsigned fmm_mask,
-	int first_check = 3, int tail_at = 0, const std::function<bool()>& before_tail = {}, hipStream_t stream = nullptr,
-	int group = 0)
+	int first_check = 3)
 {
-	SweepGroup q{&B, M, nrows, stream ? stream : ctx->stream, fmm_mask, group};
-	return run_sweeps_groups(ctx, &q, 1, roots, cap, first_check, tail_at,
-		before_tail ? std::function<bool(int)>([&](int) { return before_tail(); }) : std::function<bool(int)>());
+	SweepGroup q{&B, M, nrows, ctx->stream, fmm_mask, 0};
+	return run_sweeps_groups(ctx, &q, 1, roots, cap, first_check);
+}
+
+// The counts a group's step tracked (host_track), kept for TRACK_STEPS steps
+inline int* track_slot(ccf_ctx* ctx, int group, int j)
+{
+	return ctx->host_track + ((size_t)group * TRACK_STEPS + (j & (TRACK_STEPS - 1))) * 2 * TRACK_SWEEPS;
+}
+
+// The sweep at which a step's tail would best have started, from the counts
+// it tracked: track[k] is the most roots of a row active at sweep k's start,
+// track[TRACK_SWEEPS + k] the most listed in it for the Cauchy sums, known
+// for the sweeps up to its tail's first, at. The tail's workgroup evaluates
+// TAIL_BLOCK roots in about 25 us and sums 8 listed roots over 11 000 terms
+// in about 8 us; a device-wide sweep is worth its launches (three per sweep,
+// about 100 us of a group's time with the other group running) from there.
+int tail_sweep(const int* track, int at, int R)
+{
+	for (int k = 1; k <= at && k < TRACK_SWEEPS; k++)
+	{
+		const double evals = 25.0 * ((track[k] + TAIL_BLOCK - 1) / TAIL_BLOCK);
+		const double sums = (double)track[TRACK_SWEEPS + k] * R / 11000.0;
+		if (evals + sums <= TAIL_US) return k;
+	}
+	return at + 1;
 }
 
 // The sweep buffers of `rows` rows of R roots (and, when the root-sum FMM
@@ -2117,13 +2330,13 @@ bool sweep_layout(ccf_ctx* ctx, SweepBufs& b, int rows, int R, Take&& take)
 	// tree is built its order is 0, and the stars count)
 	const int terms = ((f32 && ctx->tree.order > 0) ? 0 : ctx->num_stars) + R;
 	b.part_room = 0;
-	for (SumsForm form : {SUMS_32, SUMS_64, SUMS_64_QUAD})
+	for (SumsForm form : {SUMS_32, SUMS_64, SUMS_64_QUAD}) // (SUMS_32_TAIL has no partials)
 		if ((form == SUMS_32) == f32)
 			b.part_room = std::max(b.part_room, sums_room(sums_launch(ctx, form), rows, R, terms));
 	const size_t list = (size_t)rows * R;
 	if (!(take(b.act, 2 * list) && take(b.cnt, 2 * (size_t)rows) && take(b.fl, list) && take(b.fcnt, 2 * (size_t)rows) &&
 			take(b.f0, list) && take(b.f1, list) && take(b.ex, list) &&
-			take(b.tile_off, (size_t)rows + 1) && take(b.plan, 4) && take(b.ticket, 1) &&
+			take(b.tile_off, (size_t)rows + 1) && take(b.plan, 4 + 2 * TRACK_SWEEPS) && take(b.ticket, 1) &&
 			take(b.part, b.part_room)))
 		return false;
 	if (ctx->P.root_fmm != 1 || R < ROOT_FMM_MIN_ROOTS) return true;
@@ -2259,6 +2472,22 @@ bool alloc_groups(ccf_ctx* ctx)
 	return true;
 }
 
+// the pinned host slots of the read-backs and of the tracked counts
+bool host_slots(ccf_ctx* ctx)
+{
+	const size_t counts = (size_t)ctx->max_rows + 6 * CONT_GROUPS, track = (size_t)CONT_GROUPS * TRACK_STEPS * 2 * TRACK_SWEEPS;
+	if (ctx->host_counts_size < counts + track)
+	{
+		if (ctx->host_counts) (void)hipHostFree(ctx->host_counts);
+		ctx->host_counts = nullptr;
+		ctx->host_counts_size = 0;
+		if (!CCF_HIP(ctx, hipHostMalloc((void**)&ctx->host_counts, (counts + track) * sizeof(int), hipHostMallocCoherent))) return false;
+		ctx->host_counts_size = counts + track;
+	}
+	ctx->host_track = ctx->host_counts + counts;
+	return true;
+}
+
 bool alloc_solver(ccf_ctx* ctx)
 {
 	const int R = ctx->num_roots, np = ctx->P.num_phi, nb = ctx->P.num_branches;
@@ -2277,7 +2506,7 @@ bool alloc_solver(ccf_ctx* ctx)
 	return CCF_HIP(ctx, ctx->dmalloc(&ctx->dseeds, (size_t)R * sizeof(double2))) &&
 		CCF_HIP(ctx, hipMemcpyAsync(ctx->dseeds, ctx->seeds.data(), (size_t)R * sizeof(double2), hipMemcpyHostToDevice, ctx->stream)) &&
 		CCF_HIP(ctx, ctx->dmalloc(&ctx->ccs_init, pts * sizeof(double2))) && alloc_groups(ctx) &&
-		CCF_HIP(ctx, hipHostMalloc((void**)&ctx->host_counts, (ctx->max_rows + 6 * CONT_GROUPS) * sizeof(int), hipHostMallocDefault)) &&
+		host_slots(ctx) &&
 		CCF_HIP(ctx, ctx->dmalloc(&ctx->phase, (size_t)(np + nb) * sizeof(double2))) && launch_phase(ctx) &&
 		CCF_HIP(ctx, ctx->dmalloc(&ctx->counters, (STAT_WORDS + C_COUNT) * sizeof(unsigned long long))) &&
 		CCF_HIP(ctx, hipMemsetAsync(ctx->counters, 0, STAT_WORDS * sizeof(unsigned long long), ctx->stream));
@@ -2342,7 +2571,7 @@ bool autotune_dev(ccf_ctx* ctx, int verbose)
 		bool good = alloc_sweep(ctx, B, nbg, R) && seed_rows(ctx, 0, nbg, s);
 		if (good)
 		{
-			k_prepare<<<dim3(grid(R), nbg), BLOCK, 0, s>>>(ctx->ccs_init, M, B, 0, ctx->dorder);
+			k_prepare<<<dim3(grid(R), nbg), BLOCK, 0, s>>>(ctx->ccs_init, M, B, 0, ctx->dorder, nullptr);
 			SweepGroup q{&B, M, nbg, s, (1u << ROOT_FMM_INIT_SWEEPS) - 1u, 0};
 			good = CCF_LAUNCH(ctx, "prepare_roots_kernel") && CCF_HIP(ctx, hipEventRecord(e0, s)) &&
 				run_sweeps_groups(ctx, &q, 1, ctx->ccs_init, cap) && CCF_HIP(ctx, hipEventRecord(e1, s)) &&
@@ -2435,7 +2664,7 @@ bool find_initial_roots_dev(ccf_ctx* ctx, int verbose)
 	}
 	for (int g = 0; g < G; g++)
 	{
-		k_prepare<<<dim3(grid(R), gs[g].nrows), BLOCK, 0, gs[g].s>>>(ctx->ccs_init, gs[g].M, *gs[g].B, 0, ctx->dorder);
+		k_prepare<<<dim3(grid(R), gs[g].nrows), BLOCK, 0, gs[g].s>>>(ctx->ccs_init, gs[g].M, *gs[g].B, 0, ctx->dorder, nullptr);
 		if (!CCF_LAUNCH(ctx, "prepare_roots_kernel")) return false;
 	}
 	if (!run_sweeps_groups(ctx, gs, G, ctx->ccs_init, cap)) return false;
@@ -2463,12 +2692,12 @@ bool find_ccs_dev(ccf_ctx* ctx, int verbose)
 	// sweeps the previous step needed (FP64 form: its first read-back)
 	const int first0 = 3;
 	int first = first0;
-	// the mixed form runs the sweeps after the first TAIL_AT of a step (the
-	// first TAIL_AT + 1 while the predictor still has fewer than two earlier
-	// steps) in the tail launch, without read-backs: the FMM choice of its
-	// first sweeps uses the row counts of the step before the previous one,
-	// copied back while the previous step ran (a fixed lag, so the choice
-	// does not depend on timing)
+	// the mixed form runs a step's later sweeps in the tail launch, after
+	// TAIL_LAG steps without read-backs: where the tail starts follows from
+	// the counts of TAIL_LAG steps before, the FMM choice of the first sweeps
+	// from the row counts of the step before the previous one, both handed
+	// over while later steps ran (fixed lags, so the choices do not depend on
+	// timing)
 	const bool tailed = ctx->P.precision == 1;
 	ctx->sweep_verbose = verbose;
 
@@ -2489,9 +2718,9 @@ bool find_ccs_dev(ccf_ctx* ctx, int verbose)
 	if (!ctx->err_stream && !CCF_HIP(ctx, hipStreamCreateWithFlags(&ctx->err_stream, hipStreamNonBlocking))) return false;
 	if (!ctx->err_event && !CCF_HIP(ctx, hipEventCreateWithFlags(&ctx->err_event, hipEventDisableTiming))) return false;
 	hipStream_t es = ctx->err_stream;
-	auto errors = [&](const RowMap& Me, int nrows, hipStream_t after) -> bool {
-		if (!CCF_HIP(ctx, hipEventRecord(ctx->err_event, after)) || !CCF_HIP(ctx, hipStreamWaitEvent(es, ctx->err_event, 0)))
-			return false;
+	auto errors = [&](const RowMap& Me, int nrows, hipStream_t after, hipEvent_t& event) -> bool {
+		if (!event && !CCF_HIP(ctx, hipEventCreateWithFlags(&event, hipEventDisableTiming))) return false;
+		if (!CCF_HIP(ctx, hipEventRecord(event, after)) || !CCF_HIP(ctx, hipStreamWaitEvent(es, event, 0))) return false;
 		k_errors<<<dim3(xcd_round(grid(R)), nrows), BLOCK, 0, es>>>(L, ctx->ccs_init, R, Me, np + nb, ctx->dorder, ctx->counters,
 			wc ? ctx->caustics : nullptr, wm ? ctx->mu_scales : nullptr);
 		return CCF_LAUNCH(ctx, "find_errors_kernel");
@@ -2519,8 +2748,25 @@ bool find_ccs_dev(ccf_ctx* ctx, int verbose)
 	// per row; without a tail, after the step
 	auto prev_rows = [&](int j, int g) { return RowMap{R, np, nb, j - 1, j == 1 ? 1 : 2, 0.0, ctx->phase, gb[g]}; };
 	auto prev_count = [&](int j, int g) { return (j == 1 ? 1 : 2) * (gb[g + 1] - gb[g]); };
+	int tail_at[CONT_GROUPS][TRACK_STEPS] = {}; // the sweep each group's tail started at, for the last steps
 	for (int j = 1; j <= steps; j++)
 	{
+		SweepGroup q[CONT_GROUPS];
+		bool prev_done[CONT_GROUPS] = {};
+		// the previous step's error pass, ordered after what group g has queued
+		const auto prev_errors = [&](int g) {
+			prev_done[g] = true;
+			return errors(prev_rows(j, g), prev_count(j, g), gs[g], ctx->step_event[2 * g + (j & 1)]);
+		};
+		// the tail's first sweep: from the counts of TAIL_LAG steps before,
+		// which step j - 2's k_prepare handed to the host (done once that
+		// step's event is, recorded before its tail)
+		// (the exact sheets are discontinuous at the field's edge, where a root
+		// can hop across it until the cap: it follows the last bit of its
+		// evaluation, which the sweep kernels and the tail round differently,
+		// so those fields keep one place for it)
+		const bool counted = tailed && ctx->P.approx;
+		const bool lagged = tailed && (j > TAIL_LAG || !counted);
 		for (int g = 0; g < G; g++)
 		{
 			const int nbg = gb[g + 1] - gb[g];
@@ -2542,27 +2788,44 @@ bool find_ccs_dev(ccf_ctx* ctx, int verbose)
 				// probe: its launches over empty rows cost more than the
 				// direct FP32 sums of a continuation sweep, O(listed R),
 				// that it could replace
-				for (int q = 0; q < ROOT_FMM_STEP_SWEEPS; q++)
-					if (j < 3 || rows2[q] > 0) mask |= 1u << q;
+				for (int q2 = 0; q2 < ROOT_FMM_STEP_SWEEPS; q2++)
+					if (j < 3 || rows2[q2] > 0) mask |= 1u << q2;
 			}
 			else
-				for (int q = 0; q < ROOT_FMM_STEP_SWEEPS; q++)
-					if (prev[q] != 0 || j % ROOT_FMM_PROBE == 1) mask |= 1u << q;
+				for (int q2 = 0; q2 < ROOT_FMM_STEP_SWEEPS; q2++)
+					if (prev[q2] != 0 || j % ROOT_FMM_PROBE == 1) mask |= 1u << q2;
+			q[g] = SweepGroup{gsw[g], M, 2 * nbg, gs[g], mask, g};
+			if (tailed) q[g].early = j < 3 ? EARLY_SWEEPS + 1 : EARLY_SWEEPS;
+			if (tailed && !counted)
+				q[g].tail_at = q[g].early;
+			else if (lagged)
+			{
+				if (!CCF_HIP(ctx, hipEventSynchronize(ctx->step_event[2 * g + (j & 1)]))) return false;
+				q[g].tail_at = tail_sweep(track_slot(ctx, g, j - TAIL_LAG), tail_at[g][(j - TAIL_LAG) & (TRACK_STEPS - 1)], R);
+			}
+			else if (tailed)
+				q[g].tail_at = TAIL_READ;
 			// the exact smooth sheets are discontinuous at the field's edge
 			// (boxcar / heaviside terms), where extrapolated roots could cross
 			// onto another branch: those keep the previous step's roots
 			const int order = ctx->P.approx ? ctx->P.predictor : 0;
-			k_prepare<<<dim3(grid(R), 2 * nbg), BLOCK, 0, gs[g]>>>(ctx->ccs_init, M, *gsw[g], order, ctx->dorder);
+			k_prepare<<<dim3(grid(R), 2 * nbg), BLOCK, 0, gs[g]>>>(ctx->ccs_init, M, *gsw[g], order, ctx->dorder,
+				counted && j > 1 ? track_slot(ctx, g, j - 1) : nullptr);
 			if (!CCF_LAUNCH(ctx, "prepare_roots_kernel")) return false;
-			bool prev_done = false;
-			const auto at_tail = [&]() {
-				prev_done = true;
-				return errors(prev_rows(j, g), prev_count(j, g), gs[g]);
-			};
-			if (!run_sweeps(ctx, *gsw[g], ctx->ccs_init, M, 2 * nbg, cap, mask, tailed ? cap + 1 : first,
-					tailed ? (j < 3 ? TAIL_AT + 1 : TAIL_AT) : 0, at_tail, gs[g], g))
-				return false;
-			if (!prev_done && !errors(prev_rows(j, g), prev_count(j, g), gs[g])) return false;
+			// without read-backs, group after group
+			if (lagged && !run_sweeps_groups(ctx, &q[g], 1, ctx->ccs_init, cap, cap + 1, prev_errors)) return false;
+		}
+		if (!lagged && !run_sweeps_groups(ctx, q, G, ctx->ccs_init, cap, tailed ? 1 : first, prev_errors)) return false;
+		for (int g = 0; g < G; g++)
+		{
+			tail_at[g][j & (TRACK_STEPS - 1)] = q[g].tail_at > 0 ? q[g].tail_at : cap;
+			if (!prev_done[g] && !prev_errors(g)) return false;
+		}
+		if (verbose >= 3 && tailed)
+		{
+			std::cout << "step " << j << ": tail after";
+			for (int g = 0; g < G; g++) std::cout << " " << q[g].tail_at;
+			std::cout << " sweeps\n";
 		}
 		prev[0] = ctx->fmm_rows_sweep[0];
 		prev[1] = ctx->fmm_rows_sweep[1];
@@ -2578,7 +2841,7 @@ bool find_ccs_dev(ccf_ctx* ctx, int verbose)
 		}
 	}
 	for (int g = 0; g < G; g++)
-		if (!errors(prev_rows(steps + 1, g), steps == 0 ? gb[g + 1] - gb[g] : 2 * (gb[g + 1] - gb[g]), gs[g])) return false;
+		if (!errors(prev_rows(steps + 1, g), steps == 0 ? gb[g + 1] - gb[g] : 2 * (gb[g + 1] - gb[g]), gs[g], ctx->err_event)) return false;
 	// the stages after the continuation run on the context's stream
 	if (G > 1 && !group_streams_join(ctx, G)) return false;
 	if (!CCF_HIP(ctx, hipStreamSynchronize(s))) return false;
@@ -2760,7 +3023,7 @@ bool aberth_sweep_dev(ccf_ctx* ctx, const double* roots, int n, double phi, doub
 	if (ok)
 	{
 		const RowMap M{n, 2, 1, 0, 0, phi};
-		k_prepare<<<dim3(grid(n), 1), BLOCK, 0, s>>>(row, M, B, 0, nullptr);
+		k_prepare<<<dim3(grid(n), 1), BLOCK, 0, s>>>(row, M, B, 0, nullptr, nullptr);
 		ok = CCF_LAUNCH(ctx, "prepare") && run_sweeps(ctx, B, row, M, 1, 1, 1) &&
 			CCF_HIP(ctx, hipMemcpyAsync(out, row, (size_t)n * sizeof(double2), hipMemcpyDeviceToHost, s)) &&
 			CCF_HIP(ctx, hipStreamSynchronize(s));
@@ -2887,7 +3150,7 @@ bool aberth_sweep_noalloc_dev(ccf_ctx* ctx, const double* roots, int n, double p
 	if (B.slot && !(fill_int(ctx, B.slot, (size_t)n, -1) && fill_int(ctx, B.rmode, 1, 0))) return false;
 	if (!CCF_HIP(ctx, hipMemcpyAsync(row, roots, (size_t)n * sizeof(double2), hipMemcpyHostToDevice, s))) return false;
 	const RowMap M{n, 2, 1, 0, 0, phi};
-	k_prepare<<<dim3(grid(n), 1), BLOCK, 0, s>>>(row, M, B, 0, nullptr);
+	k_prepare<<<dim3(grid(n), 1), BLOCK, 0, s>>>(row, M, B, 0, nullptr, nullptr);
 	if (!CCF_LAUNCH(ctx, "prepare")) return false;
 	// no timing events (creating them would allocate)
 	const int timing = ctx->P.timing;
