@@ -28,6 +28,7 @@
 //  * the launches of a solve are captured in a HIP graph and replayed.
 // An autotuner picks the workgroup size of each phase by timing the phase's
 // launch on the batch itself.
+#include "chain.hpp"
 #include "lens.hpp"
 
 #include <algorithm>
@@ -48,15 +49,6 @@ constexpr int BLOCK = 256;
 constexpr int MAX_BATCH_PER_CU = 8;
 
 inline int grid(long long n, int b = BLOCK) { return (int)((n + b - 1) / b); }
-
-__device__ inline double rcp64(double x)
-{
-	double r = __builtin_amdgcn_rcp(x);
-	double e = fma(-x, r, 1.0);
-	r = fma(r, e, r);
-	e = fma(-x, r, 1.0);
-	return fma(r, e, r);
-}
 
 __device__ inline unsigned long long wave_sum(unsigned long long v)
 {

@@ -27,6 +27,7 @@
 // fallback: a lane whose nearest root in an LDS chunk is closer than
 // CLUSTER_REL times the field's half-length (where an FP32 difference of two
 // positions keeps fewer than ~12 bits) redoes that chunk in FP64.
+#include "chain.hpp"
 #include "lens.hpp"
 
 #include <hiprand/hiprand_kernel.h>
@@ -203,20 +204,10 @@ __device__ inline int block_append(int* counter, bool pred)
 	return pos;
 }
 
-// 1/x for x > 0: hardware reciprocal estimate refined by two Newton steps
-// (each squares the relative error of the ~2^-23 estimate)
-__device__ inline double rcp64(double x)
-{
-	double r = __builtin_amdgcn_rcp(x);
-	double e = fma(-x, r, 1.0);
-	r = fma(r, e, r);
-	e = fma(-x, r, 1.0);
-	return fma(r, e, r);
-}
-
 // phi-row index and angle of solved row r of a phase (ccf_functions.cuh:338-374).
 // rows_per_branch 1: the branch centres (j = 0); 2: both sides of step j;
-// 0: row r of a caller-supplied array, all at angle phi_fixed.
+// 0: row r of a caller-supplied array, all at angle phi_fixed; -1: row r of
+// the output, whose phase comes from cs.
 // angle of phi step j on side sgn of branch c (ccf_functions.cuh:338-374)
 __device__ inline double branch_phi(int c, int sgn, int j, int np, int nb)
 {
@@ -231,19 +222,23 @@ struct RowMap
 	double phi_fixed;
 	const double2* cs = nullptr; // (cos phi, sin phi) of every phi row, or null
 	int c0 = 0;                  // the first branch of the rows (a group of branches solved on its own stream)
+	int side = 0;                // rows_per_branch 1: step j's rows of this side (-1 or 1), or the centres (0)
+	__device__ inline int sgn(int r) const
+	{
+		return rows_per_branch == 1 ? side : ((r % rows_per_branch) == 0 ? -1 : 1);
+	}
 	__device__ inline void get(int r, int& row, double& phi) const
 	{
-		if (rows_per_branch == 0)
+		if (rows_per_branch <= 0)
 		{
 			row = r;
 			phi = phi_fixed;
 			return;
 		}
 		const int c = c0 + r / rows_per_branch;
-		const int sgn = rows_per_branch == 1 ? 0 : ((r % rows_per_branch) == 0 ? -1 : 1);
 		const int center = np / (2 * nb) + c * (np / nb + 1);
-		row = center + sgn * j;
-		phi = branch_phi(c, sgn, j, np, nb);
+		row = center + sgn(r) * j;
+		phi = branch_phi(c, sgn(r), j, np, nb);
 	}
 	__device__ inline void phase(int row, double phi, double& cp, double& sp) const
 	{
@@ -505,58 +500,6 @@ __device__ inline void plan_sums(SweepView V, const PlanArgs& P)
 			V.plan[4 + TRACK_SWEEPS + sweep] = lmax;
 		}
 	}
-}
-
-// The near-field sums of a root outside the tree (its node is not a leaf:
-// every star of the node's ranges), by the lanes of one wave: lane l sums
-// the stars l, l + 64, ... of the ranges (p2p's terms), and a butterfly of
-// fixed order gives every lane the total. Every lane of the wave calls it
-// with the same z and node.
-__device__ inline Near wave_near(const LensView& L, int node, cd z)
-{
-	Near nr;
-	const int lane = threadIdx.x & 63;
-	const int ranges = L.nnf[node];
-	for (int k = 0; k < ranges; k++)
-	{
-		const int2 rg = L.nf[node * MAX_NEAR_RANGES + k];
-		const int e = rg.x + rg.y;
-		// the lane's stars in order, two loads issued before their terms
-		for (int s0 = rg.x + lane; s0 < e; s0 += 2 * 64)
-		{
-			double2 q[2];
-			double m[2];
-#pragma unroll
-			for (int u = 0; u < 2; u++)
-			{
-				const int s = min(s0 + u * 64, e - 1);
-				q[u] = L.spos[s];
-				m[u] = L.smass[s];
-			}
-#pragma unroll
-			for (int u = 0; u < 2; u++)
-				if (s0 + u * 64 < e)
-				{
-					const cd t = cd(z.re - q[u].x, z.im - q[u].y).inv();
-					nr.s0 += t;
-					const cd t1 = t * m[u];
-					nr.s1 += t1;
-					const cd t2 = t1 * t;
-					nr.s2 += t2;
-					nr.s3 += t2 * t;
-				}
-		}
-		nr.count += rg.y;
-	}
-	double v[8] = {nr.s0.re, nr.s0.im, nr.s1.re, nr.s1.im, nr.s2.re, nr.s2.im, nr.s3.re, nr.s3.im};
-#pragma unroll
-	for (int q = 0; q < 8; q++)
-		for (int o = 32; o >= 1; o >>= 1) v[q] += __shfl_xor(v[q], o, 64);
-	nr.s0 = cd(v[0], v[1]);
-	nr.s1 = cd(v[2], v[3]);
-	nr.s2 = cd(v[4], v[5]);
-	nr.s3 = cd(v[6], v[7]);
-	return nr;
 }
 
 // The same sums in k_tail's order (coop_near over TAIL_WAVES waves): the wave
@@ -854,68 +797,13 @@ __global__ __launch_bounds__(BLOCK) void k_sums64(const double2* __restrict__ sp
 	}
 }
 
-// K3 in FP64 of the continuation steps and of single sweeps
-// (k_sums64_quad): the same partial sums with the reciprocals shared.
-//
-// Four Cauchy terms d_i / |d_i|^2, d_i = z - w_i, added to (ax, ay) over one
-// reciprocal: with n_i = |d_i|^2 and the pair numerators d_0 n_1 + d_1 n_0
-// and d_2 n_3 + d_3 n_2, their sum is
-//   ((d_0 n_1 + d_1 n_0) n_2 n_3 + (d_2 n_3 + d_3 n_2) n_0 n_1) / (n_0 n_1 n_2 n_3).
-// 36 FP64 instructions and one v_rcp_f64 (3.4 instructions' time) for four
-// terms, against 11 (one of them v_max_f64, 1.7) and one for each term of
-// its own. No numerator cancels more than the sum of the terms itself does,
-// and the accumulator rounds once in four terms. NORM_FLOOR makes the term
-// of the root itself (d = 0) zero; it does not reach the last bit of any
-// n_i of two positions further apart than 1e-22. Products stay within range
-// while every |d_i| is below 1e38; beyond it the sums are not finite and the
-// slice is summed again term by term.
+// K3 in FP64 of the continuation steps and of single sweeps: the same partial
+// sums with the reciprocals shared (cauchy4).
 //
 // Bound by the FP64 VALU: 20 000 roots against 30 000 terms take 0.22 ms
 // (2.7e12 terms/s; the loop alone reaches 3.2e12), 0.33 ms in k_sums64. A
 // continuation step's sparse sweeps gain more: waves as items, lanes over the
-// sources. Relative error of the sums against 80-bit ones, fields of 200 to
-// 20 000 roots: 2e-16 to 5e-16 rms, 4e-16 to 1.3e-15 term by term.
-constexpr double NORM_FLOOR = 1e-60;
-
-// 1/x from the hardware estimate r (relative error about 2^-23) as
-// r (1 + e + e^2), e = 1 - x r: one third-order step, whose error e^3 is far
-// below the rounding of the last multiply-add
-__device__ __forceinline__ double rcp64_cubic(double x)
-{
-	const double r = __builtin_amdgcn_rcp(x);
-	const double e = fma(-x, r, 1.0);
-	return fma(r, fma(e, e, e), r);
-}
-
-// the four terms times SIGN (1 or -1) added to (ax, ay)
-template <int SIGN>
-__device__ __forceinline__ void cauchy4(double zx, double zy, const double2 (&w)[4], double& ax, double& ay)
-{
-	double dx[4], dy[4], n[4];
-#pragma unroll
-	for (int i = 0; i < 4; i++)
-	{
-		dx[i] = zx - w[i].x;
-		dy[i] = zy - w[i].y;
-		n[i] = fma(dx[i], dx[i], fma(dy[i], dy[i], NORM_FLOOR));
-	}
-	const double p = n[0] * n[1], q = n[2] * n[3];
-	const double x01 = fma(dx[0], n[1], dx[1] * n[0]), y01 = fma(dy[0], n[1], dy[1] * n[0]);
-	const double x23 = fma(dx[2], n[3], dx[3] * n[2]), y23 = fma(dy[2], n[3], dy[3] * n[2]);
-	const double iv = SIGN * rcp64_cubic(p * q);
-	ax = fma(fma(x01, q, x23 * p), iv, ax);
-	ay = fma(fma(y01, q, y23 * p), iv, ay);
-}
-
-// one Cauchy term times SIGN; d = 0 gives zero
-template <int SIGN>
-__device__ __forceinline__ void cauchy1(double zx, double zy, double2 w, double& ax, double& ay)
-{
-	const double dx = zx - w.x, dy = zy - w.y;
-	const double iv = SIGN * rcp64(fmax(fma(dx, dx, dy * dy), 1e-300));
-	ax = fma(dx, iv, ax);
-	ay = fma(dy, iv, ay);
-}
+// sources.
 
 // the terms of src[lo, hi) for a lane's target: every lane of the wave reads
 // the same source, so the sources come through scalar loads
@@ -1367,6 +1255,7 @@ constexpr int TAIL_DEFER = 64; // roots outside the tree per sweep taken by the 
 constexpr int EARLY_SWEEPS = 1; // one more while the predictor has fewer than two earlier steps
 constexpr int TAIL_LAG = 3;
 constexpr double TAIL_US = 100.0; // microseconds of a tail's first sweep below which it takes over
+constexpr double TAIL64_US = 30.0; // and of the FP64 form's tail (two sides of the branches take turns on the device)
 constexpr int TAIL_READ = -1;
 constexpr int TAIL_ACTIVE = TAIL_BLOCK; // most active roots of a row that a read-back hands to the tail
 
@@ -1745,6 +1634,100 @@ __global__ __launch_bounds__(TAIL_BLOCK) void k_tail(LensView L, double2* __rest
 	block_stats<8, TAIL_BLOCK>(stats, which, v);
 }
 
+// The FP64 continuation of a small field in one launch: a workgroup per
+// (branch, side) takes its whole chain of phi steps, the row, its stars and
+// its lists in LDS (chain_row). A step's sweeps over a few hundred roots are
+// bound by the latency of their launches (and were by their read-backs: 9.4
+// ms for the 50 steps of 200 roots at num_phi 100, 2.9 ms in one launch).
+// 1024 threads, though they spill 12 bytes at 128 VGPRs: four waves a SIMD
+// keep the FP64 pipe busier than two do (3.4 ms with 512 threads and no
+// spill). A workgroup's time grows with the square of its roots, a device-
+// wide step of so few roots takes about 145 us whatever they are: the chains
+// are faster up to CHAIN_ROOTS (400 roots: 112 us a step; 600: 184).
+constexpr int CHAIN_BLOCK = 1024;
+constexpr int CHAIN_ROOTS = 480;
+
+inline size_t chain_lds(int R, int N)
+{
+	return (size_t)R * (3 * sizeof(double2) + 3 * sizeof(int)) + (size_t)N * sizeof(double2) + sizeof(int);
+}
+
+__global__ __launch_bounds__(CHAIN_BLOCK) void k_chains(LensView L, double2* __restrict__ roots, const double2* __restrict__ cs, int R,
+	int N, int np, int nb, int steps, int cap, int predictor, int circ_exact, const int* __restrict__ order,
+	unsigned long long* __restrict__ stats)
+{
+	extern __shared__ double2 chain_mem[];
+	__shared__ int s_cnt[2];
+	double2* const zc = chain_mem;
+	double2* const st = zc + R;
+	ChainLists ls;
+	ls.f0 = st + N;
+	ls.f1 = ls.f0 + R;
+	ls.la = reinterpret_cast<int*>(ls.f1 + R);
+	ls.lb = ls.la + R;
+	ls.fl = ls.lb + R;
+	const int c = blockIdx.x >> 1, sgn = (blockIdx.x & 1) == 0 ? -1 : 1;
+	const int center = np / (2 * nb) + c * (np / nb + 1);
+	int cnt[CHAIN_COUNTS] = {0, 0, 0, 0, 0};
+	for (int s = threadIdx.x; s < N; s += CHAIN_BLOCK) st[s] = L.spos[s];
+	for (int j = 1; j <= steps; j++)
+	{
+		const int row = center + sgn * j;
+		const double2 e = cs[row];
+		double2* const out = roots + (size_t)row * R;
+		const int q = min(predictor, j - 1);
+		// (a thread reads what it wrote in the earlier steps)
+		for (int i = threadIdx.x; i < R; i += CHAIN_BLOCK)
+		{
+			zc[i] = predict_root(roots + (size_t)(row - sgn) * R + i, (long long)sgn * R, q);
+			ls.la[i] = order[i];
+		}
+		if (threadIdx.x == 0) s_cnt[0] = s_cnt[1] = 0;
+		__syncthreads();
+		chain_row<CHAIN_BLOCK>(L, R, N, circ_exact, cap, e.x, e.y, zc, st, ls, R, s_cnt, cnt);
+		for (int i = threadIdx.x; i < R; i += CHAIN_BLOCK) out[i] = zc[i];
+	}
+	const int which[CHAIN_COUNTS] = {C_TAIL_FULL, C_TAIL_EARLY, C_CONV, C_TAIL_NEAR, C_TAIL_SWEEPS};
+	unsigned long long v[CHAIN_COUNTS];
+	for (int t = 0; t < CHAIN_COUNTS; t++) v[t] = (unsigned long long)cnt[t];
+	block_stats<CHAIN_COUNTS, CHAIN_BLOCK>(stats, which, v);
+}
+
+// The FP64 form's tail: the sweeps of a continuation step after its device-
+// wide ones (k_finalize's updates among them) in one launch, a workgroup per
+// row, in place in the row and with the sweep buffers' slices as its lists.
+__global__ __launch_bounds__(CHAIN_BLOCK) void k_tail64(LensView L, double2* __restrict__ roots, RowMap M, SweepView V,
+	const double2* __restrict__ spos, int N, int cap, int first, unsigned long long* __restrict__ stats)
+{
+	__shared__ int s_cnt[2];
+	const int r = blockIdx.x, R = M.R;
+	int row;
+	double phi, cp, sp;
+	M.get(r, row, phi);
+	M.phase(row, phi, cp, sp);
+	const size_t base = (size_t)r * R;
+	const int n = V.cnt[r];
+	ChainLists ls;
+	ls.la = const_cast<int*>(V.act) + base;
+	ls.lb = V.act_next + base;
+	ls.fl = V.fl + base;
+	ls.f0 = V.f0 + base;
+	ls.f1 = V.f1 + base;
+	if (threadIdx.x == 0)
+	{
+		s_cnt[0] = s_cnt[1] = 0;
+		if (first < TRACK_SWEEPS) atomicMax(&V.plan[4 + first], n);
+	}
+	__syncthreads();
+	int cnt[CHAIN_COUNTS] = {0, 0, 0, 0, 0};
+	chain_row<CHAIN_BLOCK>(L, R, N, 0, cap, cp, sp, roots + (size_t)row * R, spos, ls, n, s_cnt, cnt);
+	if (threadIdx.x == 0) V.cnt[r] = 0; // empty for any sweep kernel that follows
+	const int which[CHAIN_COUNTS] = {C_TAIL_FULL, C_TAIL_EARLY, C_CONV, C_TAIL_NEAR, C_TAIL_SWEEPS};
+	unsigned long long v[CHAIN_COUNTS];
+	for (int t = 0; t < CHAIN_COUNTS; t++) v[t] = (unsigned long long)cnt[t];
+	block_stats<CHAIN_COUNTS, CHAIN_BLOCK>(stats, which, v);
+}
+
 // initial roots of a phase: row centre+sgn*j from the rows of the previous
 // steps (prepare_roots_kernel, ccf_functions.cuh:261-295; order > 0
 // extrapolates), every root active, the sweep counters cleared. track (or
@@ -1762,7 +1745,7 @@ __global__ void k_prepare(double2* roots, RowMap M, SweepBufs B, int order, cons
 	{
 		if (M.j > 0)
 		{
-			const int sgn = (r % M.rows_per_branch) == 0 ? -1 : 1;
+			const int sgn = M.sgn(r);
 			const int q = min(order, M.j - 1); // previous steps beyond j - 1 that exist
 			roots[(size_t)row * R + a] = predict_root(roots + (size_t)(row - sgn) * R + a, (long long)sgn * R, q);
 		}
@@ -1985,7 +1968,7 @@ SumsLaunch sums_launch(ccf_ctx* ctx, SumsForm form)
 inline SumsForm sums_form(const ccf_ctx* ctx, const RowMap& M)
 {
 	if (ctx->P.precision == 1) return SUMS_32;
-	return M.rows_per_branch == 1 ? SUMS_64 : SUMS_64_QUAD;
+	return M.rows_per_branch == 1 && M.side == 0 ? SUMS_64 : SUMS_64_QUAD;
 }
 
 // the partial sums of a sweep over `rows` rows of R roots and `terms` terms:
@@ -2189,14 +2172,14 @@ bool run_sweeps_groups(ccf_ctx* ctx, SweepGroup* gs, int G, double2* roots, int 
 				if (!CCF_HIP(ctx, hipEventSynchronize(ctx->read_event[q.id]))) return false;
 				int most = 0;
 				for (int r = 0; r < nrows; r++) most = std::max(most, ctx->host_counts[q.row0 + r]);
-				if (most <= TAIL_ACTIVE) q.tail_at = it + 1;
+				if (most <= (f32 ? TAIL_ACTIVE : 64)) q.tail_at = it + 1;
 			}
 			// mixed form, continuation: the sweeps from tail_at on in one launch, with no read-back, which begins with
 			// this sweep's updates. The rows the root-sum FMM took in the
 			// step's first two sweeps go to the host for the choice two steps
 			// later.
 			const bool tail_now = q.tail_at > 0 && it + 1 == q.tail_at && it + 1 < cap;
-			if (!tail_now) k_finalize<<<g_rows, BLOCK, 0, s>>>(ctx->theta, roots, M, V, ctx->counters);
+			if (!tail_now || !f32) k_finalize<<<g_rows, BLOCK, 0, s>>>(ctx->theta, roots, M, V, ctx->counters);
 			if (!CCF_LAUNCH(ctx, "find_critical_curve_roots_kernel")) return false;
 			ctx->info.sweeps++;
 			if (tail_now)
@@ -2231,8 +2214,11 @@ bool run_sweeps_groups(ccf_ctx* ctx, SweepGroup* gs, int G, double2* roots, int 
 					tt.b = ctx->next_event();
 					if (tt.a && tt.b) (void)hipEventRecord(tt.a, s);
 				}
-				k_tail<<<nrows, TAIL_BLOCK, 0, s>>>(L, roots, M, Vn, ctx->counters, circ_exact, fmm_pole ? 1 : 0, cap - (it + 1),
-					(float)(d * d), ctx->spos32, Np, ctx->theta, it + 1);
+				if (f32)
+					k_tail<<<nrows, TAIL_BLOCK, 0, s>>>(L, roots, M, Vn, ctx->counters, circ_exact, fmm_pole ? 1 : 0, cap - (it + 1),
+						(float)(d * d), ctx->spos32, Np, ctx->theta, it + 1);
+				else
+					k_tail64<<<nrows, CHAIN_BLOCK, 0, s>>>(L, roots, M, Vn, ctx->spos, Np, cap - (it + 1), it + 1, ctx->counters);
 				if (ctx->P.timing && tt.a && tt.b)
 				{
 					(void)hipEventRecord(tt.b, s);
@@ -2302,10 +2288,19 @@ inline int* track_slot(ccf_ctx* ctx, int group, int j)
 // TAIL_BLOCK roots in about 25 us and sums 8 listed roots over 11 000 terms
 // in about 8 us; a device-wide sweep is worth its launches (three per sweep,
 // about 100 us of a group's time with the other group running) from there.
-int tail_sweep(const int* track, int at, int R)
+// The FP64 form's (k_tail64; stars >= 0) sums about 16 000 terms a
+// microsecond, and evaluates CHAIN_BLOCK roots in about 15.
+int tail_sweep(const int* track, int at, int R, int stars)
 {
 	for (int k = 1; k <= at && k < TRACK_SWEEPS; k++)
 	{
+		if (stars >= 0)
+		{
+			// (every active root may need its sums)
+			const double us = 15.0 * ((track[k] + CHAIN_BLOCK - 1) / CHAIN_BLOCK) + (double)track[k] * (R + stars) / 16000.0;
+			if (us <= TAIL64_US) return k;
+			continue;
+		}
 		const double evals = 25.0 * ((track[k] + TAIL_BLOCK - 1) / TAIL_BLOCK);
 		const double sums = (double)track[TRACK_SWEEPS + k] * R / 11000.0;
 		if (evals + sums <= TAIL_US) return k;
@@ -2435,11 +2430,22 @@ bool launch_phase(ccf_ctx* ctx)
 	return CCF_LAUNCH(ctx, "phase table");
 }
 
-// groups of branches solved side by side: the mixed form's (at most
-// CONT_GROUPS, at most one per branch); the FP64 form reads its sweeps back
-// and runs one
+// whether the continuation hands its steps' later sweeps to a tail launch,
+// with no read-back after the first steps: the mixed form, and the FP64 form
+// with direct sums (the root-sum FMM's FP64 sweeps go by read-back row
+// counts) and without the exact sheets (chain_field)
+inline bool tailed_steps(const ccf_ctx* ctx)
+{
+	return ctx->P.precision == 1 || (ctx->P.root_fmm != 1 && ctx->P.approx);
+}
+
+// groups of rows solved side by side on their own streams: the mixed form's
+// groups of branches (at most CONT_GROUPS, at most one per branch); the FP64
+// form solves its centres in one group, whose sums so keep their slices, and
+// a tailed continuation in two, the sides of its branches
 inline int group_count(const ccf_ctx* ctx, bool init)
 {
+	if (ctx->P.precision == 0) return !init && tailed_steps(ctx) ? 2 : 1;
 	return ctx->P.precision == 1 ? std::max(1, std::min(init ? CONT_GROUPS : CONT_STEP_GROUPS, ctx->P.num_branches)) : 1;
 }
 
@@ -2466,7 +2472,8 @@ bool alloc_groups(ccf_ctx* ctx)
 	if (!alloc_sweep(ctx, ctx->sw, ctx->max_rows, R)) return false;
 	for (int g = 1; g < std::max(Gi, Gc); g++)
 	{
-		const int ri = g < Gi ? (g + 1) * nb / Gi - g * nb / Gi : 0, rc = g < Gc ? 2 * ((g + 1) * nb / Gc - g * nb / Gc) : 0;
+		const int ri = g < Gi ? (g + 1) * nb / Gi - g * nb / Gi : 0;
+		const int rc = g >= Gc ? 0 : (ctx->P.precision == 0 ? nb : 2 * ((g + 1) * nb / Gc - g * nb / Gc));
 		if (!alloc_sweep(ctx, ctx->swg[g - 1], std::max(ri, rc), R)) return false;
 	}
 	return true;
@@ -2676,6 +2683,15 @@ bool find_initial_roots_dev(ccf_ctx* ctx, int verbose)
 	return true;
 }
 
+// whether a field's continuation runs as k_chains: FP64 with direct sums, and
+// rows of at most CHAIN_ROOTS roots, above which the sweeps over the whole
+// device are faster. Not with the exact sheets, at whose edge a root can hop
+// until the cap and follows the last bit of its evaluation.
+bool chain_field(const ccf_ctx* ctx)
+{
+	return ctx->P.precision == 0 && ctx->P.approx && ctx->P.root_fmm != 1 && ctx->num_roots <= CHAIN_ROOTS;
+}
+
 bool find_ccs_dev(ccf_ctx* ctx, int verbose)
 {
 	const int R = ctx->num_roots, np = ctx->P.num_phi, nb = ctx->P.num_branches;
@@ -2698,7 +2714,7 @@ bool find_ccs_dev(ccf_ctx* ctx, int verbose)
 	// from the row counts of the step before the previous one, both handed
 	// over while later steps ran (fixed lags, so the choices do not depend on
 	// timing)
-	const bool tailed = ctx->P.precision == 1;
+	const bool tailed = tailed_steps(ctx);
 	ctx->sweep_verbose = verbose;
 
 	// the error pass (max 1/mu error and the NaN abort, ccf.cuh:1039-1069)
@@ -2721,6 +2737,7 @@ bool find_ccs_dev(ccf_ctx* ctx, int verbose)
 	auto errors = [&](const RowMap& Me, int nrows, hipStream_t after, hipEvent_t& event) -> bool {
 		if (!event && !CCF_HIP(ctx, hipEventCreateWithFlags(&event, hipEventDisableTiming))) return false;
 		if (!CCF_HIP(ctx, hipEventRecord(event, after)) || !CCF_HIP(ctx, hipStreamWaitEvent(es, event, 0))) return false;
+		if (nrows == 0) return true;
 		k_errors<<<dim3(xcd_round(grid(R)), nrows), BLOCK, 0, es>>>(L, ctx->ccs_init, R, Me, np + nb, ctx->dorder, ctx->counters,
 			wc ? ctx->caustics : nullptr, wm ? ctx->mu_scales : nullptr);
 		return CCF_LAUNCH(ctx, "find_errors_kernel");
@@ -2732,10 +2749,14 @@ bool find_ccs_dev(ccf_ctx* ctx, int verbose)
 	// other group's first sweep over all of its roots fills. The groups share
 	// only read-only inputs, the statistics (integer atomics) and the error
 	// pass's stream; each writes its own rows.
-	const int G = tailed ? solve_groups(ctx, false) : 1;
+	// a small field's chains run in one launch
+	const bool chained = chain_field(ctx) && steps > 0;
+	const int G = tailed && !chained ? solve_groups(ctx, false) : 1;
 	int gb[CONT_GROUPS + 1] = {};
 	hipStream_t gs[CONT_GROUPS] = {};
 	SweepBufs* gsw[CONT_GROUPS] = {};
+	// (the FP64 form's two groups are the sides of all branches)
+	const bool sides = ctx->P.precision == 0 && G == 2;
 	for (int g = 0; g <= G; g++) gb[g] = g * nb / G;
 	if (G > 1 && !group_streams_start(ctx, G)) return false;
 	for (int g = 0; g < G; g++)
@@ -2746,17 +2767,50 @@ bool find_ccs_dev(ccf_ctx* ctx, int verbose)
 	// the rows of a group's previous step (the centres before the first)
 	// take their pass while this step's tail runs, a launch of one workgroup
 	// per row; without a tail, after the step
-	auto prev_rows = [&](int j, int g) { return RowMap{R, np, nb, j - 1, j == 1 ? 1 : 2, 0.0, ctx->phase, gb[g]}; };
-	auto prev_count = [&](int j, int g) { return (j == 1 ? 1 : 2) * (gb[g + 1] - gb[g]); };
+	const auto rows_of = [&](int j, int g) {
+		if (sides && j > 0) return RowMap{R, np, nb, j, 1, 0.0, ctx->phase, 0, g == 0 ? -1 : 1};
+		return RowMap{R, np, nb, j, j == 0 ? 1 : 2, 0.0, ctx->phase, sides ? 0 : gb[g]};
+	};
+	const auto row_count = [&](int j, int g) {
+		if (sides) return j == 0 && g > 0 ? 0 : nb; // the centres with the first side
+		return (j == 0 ? 1 : 2) * (gb[g + 1] - gb[g]);
+	};
+	// the chains, then one error pass over all rows
+	if (chained)
+	{
+		ccf::Timer tt;
+		if (ctx->P.timing)
+		{
+			tt.a = ctx->next_event();
+			tt.b = ctx->next_event();
+			if (tt.a && tt.b) (void)hipEventRecord(tt.a, s);
+		}
+		k_chains<<<2 * nb, CHAIN_BLOCK, chain_lds(R, ctx->num_stars), s>>>(L, ctx->ccs_init, ctx->phase, R, ctx->num_stars, np, nb, steps,
+			cap, ctx->P.predictor, 0, ctx->dorder, ctx->counters);
+		if (ctx->P.timing && tt.a && tt.b)
+		{
+			(void)hipEventRecord(tt.b, s);
+			ctx->tail_timers.push_back(tt);
+		}
+		if (!CCF_LAUNCH(ctx, "find_critical_curve_roots_kernel") ||
+			!errors(RowMap{R, np, nb, 0, -1, 0.0, ctx->phase, 0}, np + nb, s, ctx->err_event))
+			return false;
+		ctx->info.tail_launches++;
+		if (verbose >= 1)
+		{
+			if (!CCF_HIP(ctx, hipStreamSynchronize(s))) return false;
+			std::cout << "\r[" << std::string(50, '=') << "] 100 %" << std::flush;
+		}
+	}
 	int tail_at[CONT_GROUPS][TRACK_STEPS] = {}; // the sweep each group's tail started at, for the last steps
-	for (int j = 1; j <= steps; j++)
+	for (int j = 1; j <= steps && !chained; j++)
 	{
 		SweepGroup q[CONT_GROUPS];
 		bool prev_done[CONT_GROUPS] = {};
 		// the previous step's error pass, ordered after what group g has queued
 		const auto prev_errors = [&](int g) {
 			prev_done[g] = true;
-			return errors(prev_rows(j, g), prev_count(j, g), gs[g], ctx->step_event[2 * g + (j & 1)]);
+			return errors(rows_of(j - 1, g), row_count(j - 1, g), gs[g], ctx->step_event[2 * g + (j & 1)]);
 		};
 		// the tail's first sweep: from the counts of TAIL_LAG steps before,
 		// which step j - 2's k_prepare handed to the host (done once that
@@ -2769,10 +2823,11 @@ bool find_ccs_dev(ccf_ctx* ctx, int verbose)
 		const bool lagged = tailed && (j > TAIL_LAG || !counted);
 		for (int g = 0; g < G; g++)
 		{
-			const int nbg = gb[g + 1] - gb[g];
-			const RowMap M{R, np, nb, j, 2, 0.0, ctx->phase, gb[g]};
+			const int nrows = row_count(j, g);
+			const RowMap M = rows_of(j, g);
 			unsigned mask = 0;
-			if (tailed)
+			if (ctx->P.precision == 0 && tailed) mask = 0; // no FMM pass
+			else if (tailed)
 			{
 				int rows2[2] = {-1, -1};
 				hipEvent_t e = ctx->fmm_rows_event[2 * g + (j & 1)];
@@ -2794,14 +2849,15 @@ bool find_ccs_dev(ccf_ctx* ctx, int verbose)
 			else
 				for (int q2 = 0; q2 < ROOT_FMM_STEP_SWEEPS; q2++)
 					if (prev[q2] != 0 || j % ROOT_FMM_PROBE == 1) mask |= 1u << q2;
-			q[g] = SweepGroup{gsw[g], M, 2 * nbg, gs[g], mask, g};
-			if (tailed) q[g].early = j < 3 ? EARLY_SWEEPS + 1 : EARLY_SWEEPS;
+			q[g] = SweepGroup{gsw[g], M, nrows, gs[g], mask, g};
+			if (ctx->P.precision == 1) q[g].early = j < 3 ? EARLY_SWEEPS + 1 : EARLY_SWEEPS;
 			if (tailed && !counted)
 				q[g].tail_at = q[g].early;
 			else if (lagged)
 			{
 				if (!CCF_HIP(ctx, hipEventSynchronize(ctx->step_event[2 * g + (j & 1)]))) return false;
-				q[g].tail_at = tail_sweep(track_slot(ctx, g, j - TAIL_LAG), tail_at[g][(j - TAIL_LAG) & (TRACK_STEPS - 1)], R);
+				q[g].tail_at = tail_sweep(track_slot(ctx, g, j - TAIL_LAG), tail_at[g][(j - TAIL_LAG) & (TRACK_STEPS - 1)], R,
+					ctx->P.precision == 0 ? ctx->num_stars : -1);
 			}
 			else if (tailed)
 				q[g].tail_at = TAIL_READ;
@@ -2809,7 +2865,7 @@ bool find_ccs_dev(ccf_ctx* ctx, int verbose)
 			// (boxcar / heaviside terms), where extrapolated roots could cross
 			// onto another branch: those keep the previous step's roots
 			const int order = ctx->P.approx ? ctx->P.predictor : 0;
-			k_prepare<<<dim3(grid(R), 2 * nbg), BLOCK, 0, gs[g]>>>(ctx->ccs_init, M, *gsw[g], order, ctx->dorder,
+			k_prepare<<<dim3(grid(R), nrows), BLOCK, 0, gs[g]>>>(ctx->ccs_init, M, *gsw[g], order, ctx->dorder,
 				counted && j > 1 ? track_slot(ctx, g, j - 1) : nullptr);
 			if (!CCF_LAUNCH(ctx, "prepare_roots_kernel")) return false;
 			// without read-backs, group after group
@@ -2840,8 +2896,8 @@ bool find_ccs_dev(ccf_ctx* ctx, int verbose)
 			std::cout << "] " << j * 100 / steps << " %" << std::flush;
 		}
 	}
-	for (int g = 0; g < G; g++)
-		if (!errors(prev_rows(steps + 1, g), steps == 0 ? gb[g + 1] - gb[g] : 2 * (gb[g + 1] - gb[g]), gs[g], ctx->err_event)) return false;
+	for (int g = 0; g < G && !chained; g++)
+		if (!errors(rows_of(steps, g), row_count(steps, g), gs[g], ctx->err_event)) return false;
 	// the stages after the continuation run on the context's stream
 	if (G > 1 && !group_streams_join(ctx, G)) return false;
 	if (!CCF_HIP(ctx, hipStreamSynchronize(s))) return false;
@@ -2921,12 +2977,12 @@ bool find_ccs_dev(ccf_ctx* ctx, int verbose)
 		ctx->info.root_fmm_leaf_level = g.leaf;
 		ctx->info.root_fmm_leaf = g.order > 0 ? (ctx->P.root_fmm_leaf > 0 ? ctx->P.root_fmm_leaf : ROOT_FMM_LEAF) : 0;
 		ctx->info.roots_per_thread = ctx->P.roots_per_thread > 0 ? ctx->P.roots_per_thread : ROOTS_PER_THREAD;
-		// the tails: every evaluation forms f0 and f1 (mixed form), every
+		// the tails: an evaluation forms f0 and f1 (FP64 early exits f0), every
 		// full update sums the row (and the stars without the FMM pole sum)
-		const double tail_evals = (double)(c[C_TAIL_FULL] + c[C_TAIL_EARLY] + c[C_TAIL_NEWTON]);
+		const double ef = ctx->P.precision == 1 ? 1.0 : 0.5; // share of f0 + f1 in an early exit
+		const double tail_evals = (double)(c[C_TAIL_FULL] + c[C_TAIL_NEWTON]) + ef * (double)c[C_TAIL_EARLY];
 		ctx->info.flops_tail = 36.0 * (double)c[C_TAIL_NEAR] + tail_evals * (16.0 * p + sm) +
 			(double)c[C_TAIL_FULL] * (10.0 * (Np + R - 1) + (fmm_pole ? 8.0 * p : 0.0));
-		const double ef = ctx->P.precision == 1 ? 1.0 : 0.5; // share of f0 + f1 in an early exit
 		const double early = (double)c[C_EARLY];
 		ctx->info.flops_update = ctx->info.flops_sums + 36.0 * (double)c[C_NEAR] + (full + (double)c[C_NEWTON]) * (16.0 * p + sm) +
 			ef * (36.0 * (double)c[C_NEAR_EARLY] + early * 16.0 * p) + early * sm + (fmm_pole ? full * 8.0 * p : 0.0);
