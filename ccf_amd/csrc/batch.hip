@@ -71,6 +71,7 @@ struct BField
 	double* mu;              // same layout
 	unsigned long long* stats; // [BSTAT]
 	int N, R, np, nb, circ_exact, predictor, cap_init, cap_step;
+	int chained;             // FP64 phi chains by chain_row (not with the exact sheets)
 	float cluster_d2;        // mixed form: squared root separation below which a Cauchy term is FP64
 };
 
@@ -468,6 +469,86 @@ __global__ __launch_bounds__(BS, BATCH_WAVES_PER_SIMD) void k_batch(const BField
 	}
 }
 
+// The phi chains of the FP64 form (phase 1): the tasks and the row's place of
+// k_batch, the sweeps of chain_row (sums with shared reciprocals, lanes
+// shared by the roots a sweep lists). A field with the exact sheets takes
+// solve_row's sweeps: at their edge a root can hop until the cap and follows
+// the last bit of its evaluation. 24 fields of 50 to 1000 stars at num_phi
+// 504: 69 ms, 120 ms with solve_row's serial and wave-wide sums; the longest
+// chains (2000 roots) run at about three quarters of a CU's FP64 rate.
+template <int BS>
+__global__ __launch_bounds__(BS, BATCH_WAVES_PER_SIMD) void k_batch_chains(const BField* __restrict__ fields,
+	const BTask* __restrict__ tasks, int ntasks, int* __restrict__ next, int, int rmax, int rlds, int nlds, ListSlice lists)
+{
+	extern __shared__ double2 smem[];
+	double2* sl = smem + rlds;
+	__shared__ int s_task;
+	__shared__ int s_n[2];
+	__shared__ unsigned long long s_red[BCNT][BS / 64];
+	const size_t lo = (size_t)blockIdx.x * rmax;
+	const ListSlice ls{lists.la + lo, lists.lb + lo, lists.fl + lo, lists.f0 + lo, lists.f1 + lo, lists.ex + lo};
+	const ChainLists cl{ls.la, ls.lb, ls.fl, ls.f0, ls.f1};
+	for (;;)
+	{
+		__syncthreads();
+		if (threadIdx.x == 0) s_task = atomicAdd(next, 1);
+		__syncthreads();
+		const int t = __builtin_amdgcn_readfirstlane(s_task);
+		if (t >= ntasks) break;
+		const BTask tk = tasks[t];
+		const BField& F = fields[tk.field];
+		const int R = F.R, c0 = centre_row(F, tk.branch), sgn = tk.side ? 1 : -1, steps = F.np / (2 * F.nb);
+		const bool lds_row = R <= rlds, lds_stars = F.N <= nlds;
+		if (lds_stars)
+			for (int s = threadIdx.x; s < F.N; s += BS) sl[s] = F.stars[s];
+		unsigned long long cnt[BCNT] = {0, 0, 0, 0, 0, 0};
+		int cc[CHAIN_COUNTS] = {0, 0, 0, 0, 0};
+		for (int j = 1; j <= steps; j++)
+		{
+			const int row = c0 + sgn * j;
+			const double2 e = F.cs[row];
+			double2* const out = F.roots + (size_t)row * R;
+			double2* zc = lds_row ? smem : out;
+			// (a thread reads what it wrote in the earlier steps; in place: row
+			// is written, the rows before it are read)
+			const int q = min(F.predictor, j - 1);
+			for (int i = threadIdx.x; i < R; i += BS)
+			{
+				zc[i] = predict_root(F.roots + (size_t)(row - sgn) * R + i, (long long)sgn * R, q);
+				if (F.chained) ls.la[i] = F.order[i];
+			}
+			if (!F.chained)
+				solve_row<BS, false>(F, row, F.cap_step, true, zc, lds_stars ? sl : F.stars, ls.la, ls.lb, ls, s_n, cnt);
+			else
+			{
+				if (threadIdx.x == 0) s_n[0] = s_n[1] = 0;
+				__syncthreads();
+				// (the row and the stars in LDS as such: pointers that may be
+				// either are read through the flat path)
+				if (lds_row && lds_stars) chain_row<BS>(F.L, R, F.N, 0, F.cap_step, e.x, e.y, smem, sl, cl, R, s_n, cc);
+				else chain_row<BS>(F.L, R, F.N, 0, F.cap_step, e.x, e.y, zc, lds_stars ? sl : F.stars, cl, R, s_n, cc);
+			}
+			if (lds_row)
+				for (int i = threadIdx.x; i < R; i += BS) out[i] = zc[i];
+		}
+		for (int k = 0; k < CHAIN_COUNTS; k++) cnt[k] += (unsigned long long)cc[k];
+#pragma unroll
+		for (int k = 0; k < BCNT; k++)
+		{
+			const unsigned long long s = wave_sum(cnt[k]);
+			if ((threadIdx.x & 63) == 0) s_red[k][threadIdx.x >> 6] = s;
+		}
+		__syncthreads();
+		if (threadIdx.x < BCNT)
+		{
+			unsigned long long s = 0;
+			for (int w = 0; w < BS / 64; w++) s += s_red[threadIdx.x][w];
+			const int which[BCNT] = {B_FULL, B_EARLY, B_CONV, B_NEAR, B_SWEEPS, B_NEWTON};
+			if (s) atomicAdd(&F.stats[which[threadIdx.x]], s);
+		}
+	}
+}
+
 __global__ void k_zero_int(int* p, int n)
 {
 	const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -591,13 +672,26 @@ __global__ __launch_bounds__(BLOCK) void k_batch_transpose(const BField* __restr
 using BatchKernel = void (*)(const BField*, const BTask*, int, int*, int, int, int, int, ListSlice);
 
 template <bool MIXED>
-BatchKernel pick_kernel(int bs)
+BatchKernel pick_batch(int bs)
 {
 	switch (bs)
 	{
 	case 256: return k_batch<256, MIXED>;
 	case 512: return k_batch<512, MIXED>;
 	default: return k_batch<1024, MIXED>;
+	}
+}
+
+// the kernel of a phase (0: branch centres, 1: phi chains)
+BatchKernel pick_kernel(int phase, bool mixed, int bs)
+{
+	if (mixed) return pick_batch<true>(bs);
+	if (phase == 0) return pick_batch<false>(bs);
+	switch (bs)
+	{
+	case 256: return k_batch_chains<256>;
+	case 512: return k_batch_chains<512>;
+	default: return k_batch_chains<1024>;
 	}
 }
 
@@ -670,7 +764,7 @@ int batch_grid(ccf_batch* b, int phase, int bs)
 	ccf_ctx* m = b->master;
 	BatchDevice& d = *b->dev;
 	const bool mixed = m->P.precision == 1;
-	const BatchKernel fn = mixed ? pick_kernel<true>(bs) : pick_kernel<false>(bs);
+	const BatchKernel fn = pick_kernel(phase, mixed, bs);
 	int per_cu = 0;
 	if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)fn, bs, batch_lds(d.rlds, d.nlds)) != hipSuccess || per_cu < 1)
 		per_cu = 1;
@@ -684,7 +778,7 @@ bool launch_batch_phase(ccf_batch* b, int phase, int bs, int g, hipStream_t s)
 	ccf_ctx* m = b->master;
 	BatchDevice& d = *b->dev;
 	const bool mixed = m->P.precision == 1;
-	const BatchKernel fn = mixed ? pick_kernel<true>(bs) : pick_kernel<false>(bs);
+	const BatchKernel fn = pick_kernel(phase, mixed, bs);
 	const size_t lds = batch_lds(d.rlds, d.nlds);
 	const int ntasks = phase == 0 ? d.n0 : d.n1;
 	if (g > d.list_wgs)
@@ -911,6 +1005,7 @@ bool batch_build(ccf_batch* b, int verbose)
 		F.nb = nb;
 		F.circ_exact = (!c->rectangular && !c->P.approx) ? 1 : 0;
 		F.predictor = c->P.approx ? c->P.predictor : 0;
+		F.chained = c->P.approx ? 1 : 0;
 		F.cap_init = c->P.init_iters > 0 ? c->P.init_iters : 60;
 		F.cap_step = c->P.step_iters > 0 ? c->P.step_iters : 20;
 		d.rmax = std::max(d.rmax, R);

@@ -194,19 +194,40 @@ __device__ __forceinline__ Near chain_near(const LensView& L, int node, cd z, in
 }
 
 // SIGN times the terms of src[0, m) for a target, by W lanes, lane sub the
-// terms sub, sub + W, ...; a group of four past the end takes the target
-// itself, whose term is zero
-template <int SIGN>
-__device__ __forceinline__ void chain_terms(const double2* src, int m, double2 z, int sub, int W, double& ax, double& ay)
+// terms sub, sub + W, ...: whole groups of 4 W terms, then one group that
+// takes the target itself, whose term is zero, past the end. The few lanes a
+// root of a sweep that lists many shares (WC = W = 1, 2, 4) are compiled in,
+// so that the loads' offsets are immediate: the address arithmetic of a
+// variable stride costs a fifth of the loop.
+template <int SIGN, int WC>
+__device__ __forceinline__ void chain_terms_w(const double2* src, int m, double2 z, int sub, int Wr, double& ax, double& ay)
 {
-#pragma unroll 2
-	for (int q = sub; q < m; q += 4 * W)
+	const int W = WC > 0 ? WC : Wr, rounds = m / (4 * W);
+	const double2* p = src + sub;
+#pragma unroll 1
+	for (int k = 0; k < rounds; k++)
+	{
+		const double2 w[4] = {p[0], p[W], p[2 * W], p[3 * W]};
+		p += 4 * W;
+		cauchy4<SIGN>(z.x, z.y, w, ax, ay);
+	}
+	const int q = rounds * 4 * W + sub;
+	if (rounds * 4 * W < m)
 	{
 		double2 w[4];
 #pragma unroll
 		for (int k = 0; k < 4; k++) w[k] = q + k * W < m ? src[q + k * W] : z;
 		cauchy4<SIGN>(z.x, z.y, w, ax, ay);
 	}
+}
+
+template <int SIGN>
+__device__ __forceinline__ void chain_terms(const double2* src, int m, double2 z, int sub, int W, double& ax, double& ay)
+{
+	if (W == 1) chain_terms_w<SIGN, 1>(src, m, z, sub, W, ax, ay);
+	else if (W == 2) chain_terms_w<SIGN, 2>(src, m, z, sub, W, ax, ay);
+	else if (W == 4) chain_terms_w<SIGN, 4>(src, m, z, sub, W, ax, ay);
+	else chain_terms_w<SIGN, 0>(src, m, z, sub, W, ax, ay);
 }
 
 // what a workgroup counts of its rows: full updates, early exits, converged,
