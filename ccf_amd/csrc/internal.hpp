@@ -341,6 +341,9 @@ struct ForestSpec
 	int order = 0;           // out: the expansion order used
 };
 bool build_forest(ccf_ctx* ctx, ForestSpec& spec, int verbose);
+// capi.cpp: device memory to the caller's, after what is queued on the
+// context's stream (large arrays through pinned slots by several threads)
+hipError_t copy_out(ccf_ctx* c, void* dst, const void* src, size_t bytes);
 // solve.hip
 bool alloc_sweep(ccf_ctx* ctx, SweepBufs& b, int rows, int R);
 void free_sweep(ccf_ctx* ctx, SweepBufs& b);

@@ -3060,8 +3060,7 @@ bool eval_points_dev(ccf_ctx* ctx, const double* z, int n, double phi, double* o
 	if (ok)
 	{
 		k_eval<<<grid(n), BLOCK, 0, s>>>(ctx->lens(), dz, n, phi, dout);
-		ok = CCF_LAUNCH(ctx, "eval kernel") && CCF_HIP(ctx, hipMemcpyAsync(out, dout, (size_t)n * 8 * sizeof(double), hipMemcpyDeviceToHost, s)) &&
-			CCF_HIP(ctx, hipStreamSynchronize(s));
+		ok = CCF_LAUNCH(ctx, "eval kernel") && CCF_HIP(ctx, copy_out(ctx, out, dout, (size_t)n * 8 * sizeof(double)));
 	}
 	ctx->dfree(dz);
 	ctx->dfree(dout);
