@@ -149,6 +149,7 @@ struct RootGrid
 struct SweepBufs
 {
 	int rows = 0, R = 0;
+	unsigned char* mem = nullptr; // the allocation that the arrays are slices of (null: not owned)
 	size_t part_room = 0;    // entries of part
 	int* act = nullptr;      // [2][rows][R] active root indices (ping-pong)
 	int* cnt = nullptr;      // [2][rows]
@@ -249,11 +250,12 @@ struct ccf_ctx
 	}
 	int* host_counts = nullptr;   // pinned, coherent: active roots per row, the two FMM row counts of a read-back, then per continuation group two slots of two for the mixed continuation
 	int tree_hint_stars = -1, tree_hint_fields = -1, tree_hint_nodes = 0; // the last tree build's node count
+	char* call_host = nullptr;    // its last part: in and out of the calls that take a few points or roots
 	double* host_stage = nullptr; // pinned (STAGE_DOUBLES), until ccf_destroy: a tree build's level counts and binomial table, a run's folded statistics
 	hipStream_t err_stream = nullptr; // the error pass of find_ccs, beside the continuation (default priority)
 	hipEvent_t err_event = nullptr;   // a row set's roots are final (no timing)
-	size_t host_counts_size = 0;  // ints host_counts holds: kept from run to run, grown when one needs more
-	int* host_track = nullptr; // its last part: [CONT_GROUPS][TRACK_STEPS][2 TRACK_SWEEPS] the tracked counts of a group's last steps
+	size_t host_size = 0;         // bytes of host_counts' allocation: kept from run to run, grown when one needs more
+	int* host_track = nullptr; // a part of it: [CONT_GROUPS][TRACK_STEPS][2 TRACK_SWEEPS] the tracked counts of a group's last steps
 	hipEvent_t step_event[2 * ccf::CONT_GROUPS] = {}; // mixed continuation: before a step's tail, per group and parity (no timing)
 	hipEvent_t fmm_rows_event[2 * ccf::CONT_GROUPS] = {}; // mixed continuation: after the copy of a step's FMM row count, per group (no timing)
 	hipEvent_t read_event[ccf::CONT_GROUPS] = {}; // after the copy of a sweep's active counts, per group (no timing)
@@ -345,7 +347,7 @@ bool build_forest(ccf_ctx* ctx, ForestSpec& spec, int verbose);
 // context's stream (large arrays through pinned slots by several threads)
 hipError_t copy_out(ccf_ctx* c, void* dst, const void* src, size_t bytes);
 // solve.hip
-bool alloc_sweep(ccf_ctx* ctx, SweepBufs& b, int rows, int R);
+bool alloc_sweep(ccf_ctx* ctx, SweepBufs& b, int rows, int R, bool clear = true);
 void free_sweep(ccf_ctx* ctx, SweepBufs& b);
 bool alloc_solver(ccf_ctx* ctx);
 bool find_initial_roots_dev(ccf_ctx* ctx, int verbose);

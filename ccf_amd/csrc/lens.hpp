@@ -294,7 +294,7 @@ struct Witt
 	cd d1, d2;      // d alpha_smooth / d zbar and its zbar-derivative
 };
 
-// the rest of witt_f0 once the near-field sums of z's node are known
+// Witt's function once the near-field sums of z's node are known
 __device__ inline Witt witt_from(const LensView& L, cd z, double cp, double sp, int node, const Near& nr)
 {
 	Witt w;
@@ -308,14 +308,6 @@ __device__ inline Witt witt_from(const LensView& L, cd z, double cp, double sp, 
 	const double a0 = w.f0.abs();
 	w.early = fabs(a0 * (a0 + 2 * w.a)) < 1e-9 && fabs(a0 * (a0 - 2 * w.a)) < 1e-9;
 	return w;
-}
-
-__device__ inline Witt witt_f0(const LensView& L, cd z, double phi)
-{
-	const int node = nearest_node(L, z);
-	double sp, cp;
-	sincos(phi, &sp, &cp);
-	return witt_from(L, z, cp, sp, node, p2p(L, node, z));
 }
 
 // f1 = d f0 / dz from the sums already formed for f0 (ccf_functions.cuh:108-121)

@@ -1881,22 +1881,53 @@ __global__ void k_caustics(LensView L, const double2* __restrict__ z, long long 
 	if (mu) mu[i] = m;
 }
 
-__global__ void k_eval(LensView L, const double2* __restrict__ z, int n, double phi, double* out)
+// ccf_eval_points: one evaluation of the field per point gives Witt's
+// function, its derivative, the lens map, the length scale and the 1/mu bound
+// (a point outside the tree sums every star: by its whole wave). Workgroups
+// of one wave, so that a few hundred points spread over the chip. z and out
+// may be pinned host memory.
+constexpr int EVAL_BLOCK = 64;
+
+__global__ __launch_bounds__(EVAL_BLOCK) void k_eval(LensView L, const double2* __restrict__ z, int n, double phi, double2* __restrict__ out)
 {
-	const int i = blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= n) return;
-	const cd zz(z[i].x, z[i].y);
-	Witt w = witt_f0(L, zz, phi);
-	const cd f1 = witt_f1(L, zz, w);
-	cd ws;
-	double m;
-	lens_map(L, zz, ws, m);
-	double* o = out + 8 * (size_t)i;
-	o[0] = w.f0.re; o[1] = w.f0.im;
-	o[2] = f1.re; o[3] = f1.im;
-	o[4] = ws.re; o[5] = ws.im;
-	o[6] = m;
-	o[7] = err_bound(w);
+	__shared__ double2 rows[EVAL_BLOCK][4];
+	const int i = blockIdx.x * EVAL_BLOCK + threadIdx.x;
+	cd zz;
+	int node = 0;
+	if (i < n)
+	{
+		const double2 v = z[i];
+		zz = cd(v.x, v.y);
+		node = nearest_node(L, zz);
+	}
+	const bool outside = i < n && L.nf_off[node] < 0;
+	Near nr;
+	for (unsigned long long m = __ballot(outside); m; m &= m - 1)
+	{
+		const int src = __ffsll(m) - 1;
+		const Near t = wave_near(L, __shfl(node, src, 64), cd(__shfl(zz.re, src, 64), __shfl(zz.im, src, 64)));
+		if ((int)threadIdx.x == src) nr = t;
+	}
+	if (i < n)
+	{
+		if (!outside) nr = p2p(L, node, zz);
+		double sp, cp;
+		sincos(phi, &sp, &cp);
+		const Witt w = witt_from(L, zz, cp, sp, node, nr);
+		const cd f1 = witt_f1(L, zz, w);
+		cd ws;
+		double m;
+		lens_map_from(L, zz, w.nr, w.fr, w.d1, w.d2, ws, m);
+		double2* const o = rows[threadIdx.x];
+		o[0] = make_double2(w.f0.re, w.f0.im);
+		o[1] = make_double2(f1.re, f1.im);
+		o[2] = make_double2(ws.re, ws.im);
+		o[3] = make_double2(m, err_bound(w));
+	}
+	__syncthreads();
+	// the points' rows side by side, a wave's store 1 KiB in one piece
+	const int i0 = blockIdx.x * EVAL_BLOCK, m = min(EVAL_BLOCK, n - i0);
+	for (int k = threadIdx.x; k < 4 * m; k += EVAL_BLOCK) out[(size_t)4 * i0 + k] = rows[k >> 2][k & 3];
 }
 
 // star positions and masses (generate_star_field_kernel, star.cuh:64-107) from
@@ -2308,6 +2339,22 @@ int tail_sweep(const int* track, int at, int R, int stars)
 	return at + 1;
 }
 
+// slices of one allocation (or of the no-allocation sweep's scratch array),
+// 256-byte aligned; with a null base it only adds up the bytes they take
+struct Carve
+{
+	unsigned char* base;
+	size_t used = 0;
+	template <class T>
+	bool operator()(T*& p, size_t count)
+	{
+		used = (used + 255) & ~size_t(255);
+		p = base ? reinterpret_cast<T*>(base + used) : nullptr;
+		used += count * sizeof(T);
+		return true;
+	}
+};
+
 // The sweep buffers of `rows` rows of R roots (and, when the root-sum FMM
 // applies, its grid over the field): take(p, count) provides each array of
 // count elements, from the context's device pool or from a slice of the
@@ -2370,42 +2417,45 @@ bool root_layout(ccf_ctx* ctx, SweepBufs& b, Take&& take)
 		take(b.mp, ce) && take(b.lcq, (size_t)rows * coarse_cells(g) * (g.order + 1));
 }
 
-// the root-sum FMM's arrays alone (ccf_root_sums), from the context's pool
-bool alloc_root_fmm(ccf_ctx* ctx, SweepBufs& b)
-{
-	auto take = [ctx](auto*& p, size_t count) { return CCF_HIP(ctx, ctx->dmalloc(&p, count * sizeof(*p))); };
-	return root_layout(ctx, b, take) &&
-		CCF_HIP(ctx, hipMemsetAsync(b.slot, 0xff, (size_t)b.rows * b.R * sizeof(int), ctx->stream)) &&
-		CCF_HIP(ctx, hipMemsetAsync(b.rmode, 0, b.rows * sizeof(int), ctx->stream)) &&
-		CCF_HIP(ctx, hipStreamSynchronize(ctx->stream));
-}
-
 } // namespace
 
 void free_sweep(ccf_ctx* ctx, SweepBufs& b)
 {
-	auto F = [ctx](auto*& p) { ctx->dfree(p); p = nullptr; };
-	F(b.act); F(b.cnt); F(b.fl); F(b.fcnt); F(b.f0); F(b.f1); F(b.ex); F(b.tile_off); F(b.plan); F(b.ticket);
-	F(b.part);
-	F(b.slot); F(b.rmode); F(b.rsum); F(b.ccnt); F(b.cstart); F(b.ccur); F(b.cell); F(b.bidx); F(b.sidx); F(b.spos);
-	F(b.ocnt); F(b.oidx); F(b.mp); F(b.lcq);
+	ctx->dfree(b.mem);
 	b = SweepBufs{};
 }
 
-bool alloc_sweep(ccf_ctx* ctx, SweepBufs& b, int rows, int R)
+// what a phase expects of its buffers before the first k_prepare: no root
+// listed anywhere, the ticket at 0 (a kernel: nothing waits for it but what
+// follows on its stream)
+__global__ __launch_bounds__(BLOCK) void k_clear_sweep(SweepBufs B)
+{
+	const size_t i = (size_t)blockIdx.x * BLOCK + threadIdx.x;
+	if (i < (size_t)2 * B.rows) B.cnt[i] = B.fcnt[i] = 0;
+	if (i == 0) *B.ticket = 0;
+	if (!B.slot) return;
+	if (i < (size_t)B.rows) B.rmode[i] = 0;
+	if (i < (size_t)B.rows * B.R) B.slot[i] = -1;
+}
+
+// The buffers are slices of one allocation: a new context pays for one
+// hipMalloc, not for a dozen (two dozen with the FMM's arrays). clear: set as
+// a phase finds them (else the caller's first kernel does)
+bool alloc_sweep(ccf_ctx* ctx, SweepBufs& b, int rows, int R, bool clear)
 {
 	free_sweep(ctx, b);
-	auto take = [ctx](auto*& p, size_t count) { return CCF_HIP(ctx, ctx->dmalloc(&p, count * sizeof(*p))); };
-	if (!sweep_layout(ctx, b, rows, R, take)) return false;
-	const size_t list = (size_t)rows * R;
-	if (!CCF_HIP(ctx, hipMemsetAsync(b.cnt, 0, 2 * rows * sizeof(int), ctx->stream)) ||
-		!CCF_HIP(ctx, hipMemsetAsync(b.fcnt, 0, 2 * rows * sizeof(int), ctx->stream)) ||
-		!CCF_HIP(ctx, hipMemsetAsync(b.ticket, 0, sizeof(int), ctx->stream)))
-		return false;
-	if (!b.slot) return true;
-	return CCF_HIP(ctx, hipMemsetAsync(b.slot, 0xff, list * sizeof(int), ctx->stream)) &&
-		CCF_HIP(ctx, hipMemsetAsync(b.rmode, 0, rows * sizeof(int), ctx->stream)) &&
-		CCF_HIP(ctx, hipStreamSynchronize(ctx->stream));
+	Carve size{nullptr};
+	if (!sweep_layout(ctx, b, rows, R, size)) return false;
+	b = SweepBufs{};
+	unsigned char* mem = nullptr;
+	if (!CCF_HIP(ctx, ctx->dmalloc(&mem, size.used))) return false;
+	Carve carve{mem};
+	const bool ok = sweep_layout(ctx, b, rows, R, carve);
+	b.mem = mem;
+	if (!ok || !clear) return ok;
+	const size_t n = b.slot ? std::max((size_t)2 * rows, (size_t)rows * R) : (size_t)2 * rows;
+	k_clear_sweep<<<grid((long long)n), BLOCK, 0, ctx->stream>>>(b);
+	return CCF_LAUNCH(ctx, "sweep buffers");
 }
 
 // the seeds in the rows of branch centres c0 .. c0 + gridDim.y - 1
@@ -2479,19 +2529,26 @@ bool alloc_groups(ccf_ctx* ctx)
 	return true;
 }
 
-// the pinned host slots of the read-backs and of the tracked counts
+// most bytes of a call's points or roots, and of its results, that go through
+// pinned memory (call_slots); above, a copy is as fast
+constexpr size_t CALL_BYTES = size_t(128) << 10;
+
+// the pinned host memory of a context, one allocation: the slots of the read-
+// backs and of the tracked counts, then the calls' buffer
 bool host_slots(ccf_ctx* ctx)
 {
 	const size_t counts = (size_t)ctx->max_rows + 6 * CONT_GROUPS, track = (size_t)CONT_GROUPS * TRACK_STEPS * 2 * TRACK_SWEEPS;
-	if (ctx->host_counts_size < counts + track)
+	const size_t slots = ((counts + track) * sizeof(int) + 4095) / 4096 * 4096;
+	if (ctx->host_size < slots + 2 * CALL_BYTES)
 	{
 		if (ctx->host_counts) (void)hipHostFree(ctx->host_counts);
 		ctx->host_counts = nullptr;
-		ctx->host_counts_size = 0;
-		if (!CCF_HIP(ctx, hipHostMalloc((void**)&ctx->host_counts, (counts + track) * sizeof(int), hipHostMallocCoherent))) return false;
-		ctx->host_counts_size = counts + track;
+		ctx->host_size = 0;
+		if (!CCF_HIP(ctx, hipHostMalloc((void**)&ctx->host_counts, slots + 2 * CALL_BYTES, hipHostMallocCoherent))) return false;
+		ctx->host_size = slots + 2 * CALL_BYTES;
 	}
 	ctx->host_track = ctx->host_counts + counts;
+	ctx->call_host = (char*)ctx->host_counts + slots;
 	return true;
 }
 
@@ -3049,39 +3106,120 @@ bool generate_stars_dev(ccf_ctx* ctx)
 	return CCF_LAUNCH(ctx, "generate_star_field_kernel") && CCF_HIP(ctx, hipStreamSynchronize(ctx->stream));
 }
 
+// The calls that take a few points or roots from the host (ccf_eval_points,
+// ccf_aberth_sweep, ccf_root_sums) are bound by latency: a copy from or to
+// pageable memory costs 16 to 33 us in the stream, a launch 2. Up to
+// CALL_BYTES each way they go through a pinned buffer of the context that the
+// kernels read and write themselves: 1000 points of a 100-star field 48 -> 27
+// us, a sweep over 1000 roots 218 -> 67, their root sums 159 -> 102.
+
+// that buffer (in: its first half, out: its second), or null
+char* call_slots(ccf_ctx* ctx, size_t in, size_t out)
+{
+	return in <= CALL_BYTES && out <= CALL_BYTES ? ctx->call_host : nullptr;
+}
+
+// a single row of n roots for a sweep or the root-sum FMM: copied from src
+// (or already in place: null), every root active, the counts and the ticket
+// clear; every root listed for the FMM's sums at its own index (fmm 1), or
+// none (0)
+__global__ __launch_bounds__(BLOCK) void k_call_row(double2* __restrict__ row, const double2* __restrict__ src, int n, SweepBufs B, int fmm)
+{
+	const int a = blockIdx.x * BLOCK + threadIdx.x;
+	if (a < n)
+	{
+		if (src) row[a] = src[a];
+		if (B.act) B.act[a] = a;
+		if (B.slot) B.slot[a] = fmm ? a : -1;
+	}
+	if (a == 0)
+	{
+		if (B.rmode) B.rmode[0] = fmm;
+		if (B.cnt)
+		{
+			B.cnt[0] = n;
+			B.cnt[1] = B.fcnt[0] = B.fcnt[1] = 0;
+			*B.ticket = 0;
+			B.plan[2] = B.plan[3] = 0;
+		}
+	}
+}
+
+// a call's result times sign, to device or pinned host memory
+__global__ __launch_bounds__(BLOCK) void k_call_out(const double2* __restrict__ v, int n, double sign, double2* __restrict__ out)
+{
+	const int i = blockIdx.x * BLOCK + threadIdx.x;
+	if (i < n) out[i] = make_double2(sign * v[i].x, sign * v[i].y);
+}
+
 bool eval_points_dev(ccf_ctx* ctx, const double* z, int n, double phi, double* out)
 {
 	if (n <= 0) return true;
+	const size_t nin = (size_t)n * sizeof(double2), nout = (size_t)n * 8 * sizeof(double);
+	hipStream_t s = ctx->stream;
+	if (char* h = call_slots(ctx, nin, nout))
+	{
+		std::memcpy(h, z, nin);
+		k_eval<<<grid(n, EVAL_BLOCK), EVAL_BLOCK, 0, s>>>(ctx->lens(), (const double2*)h, n, phi, (double2*)(h + CALL_BYTES));
+		if (!CCF_LAUNCH(ctx, "eval kernel") || !CCF_HIP(ctx, hipStreamSynchronize(s))) return false;
+		std::memcpy(out, h + CALL_BYTES, nout);
+		return true;
+	}
 	double2* dz = nullptr;
 	double* dout = nullptr;
-	hipStream_t s = ctx->stream;
-	bool ok = CCF_HIP(ctx, ctx->dmalloc(&dz, (size_t)n * sizeof(double2))) && CCF_HIP(ctx, ctx->dmalloc(&dout, (size_t)n * 8 * sizeof(double))) &&
-		CCF_HIP(ctx, hipMemcpyAsync(dz, z, (size_t)n * sizeof(double2), hipMemcpyHostToDevice, s));
+	bool ok = CCF_HIP(ctx, ctx->dmalloc(&dz, nin)) && CCF_HIP(ctx, ctx->dmalloc(&dout, nout)) &&
+		CCF_HIP(ctx, hipMemcpyAsync(dz, z, nin, hipMemcpyHostToDevice, s));
 	if (ok)
 	{
-		k_eval<<<grid(n), BLOCK, 0, s>>>(ctx->lens(), dz, n, phi, dout);
-		ok = CCF_LAUNCH(ctx, "eval kernel") && CCF_HIP(ctx, copy_out(ctx, out, dout, (size_t)n * 8 * sizeof(double)));
+		k_eval<<<grid(n, EVAL_BLOCK), EVAL_BLOCK, 0, s>>>(ctx->lens(), dz, n, phi, (double2*)dout);
+		ok = CCF_LAUNCH(ctx, "eval kernel") && CCF_HIP(ctx, copy_out(ctx, out, dout, nout));
 	}
 	ctx->dfree(dz);
 	ctx->dfree(dout);
 	return ok;
 }
 
+// the rows' way in and out of a call: roots to `row` with the buffers'
+// start values (k_call_row), and n results times sign to the host
+bool call_in(ccf_ctx* ctx, const double* roots, double2* row, int n, const SweepBufs& B, int fmm)
+{
+	const size_t bytes = (size_t)n * sizeof(double2);
+	hipStream_t s = ctx->stream;
+	char* h = call_slots(ctx, bytes, bytes);
+	if (h) std::memcpy(h, roots, bytes);
+	else if (!CCF_HIP(ctx, hipMemcpyAsync(row, roots, bytes, hipMemcpyHostToDevice, s))) return false;
+	k_call_row<<<grid(n), BLOCK, 0, s>>>(row, (const double2*)h, n, B, fmm);
+	return CCF_LAUNCH(ctx, "row of a call");
+}
+
+bool call_out(ccf_ctx* ctx, double2* v, int n, double sign, double* out)
+{
+	const size_t bytes = (size_t)n * sizeof(double2);
+	hipStream_t s = ctx->stream;
+	char* h = call_slots(ctx, bytes, bytes);
+	double2* dst = h ? (double2*)(h + CALL_BYTES) : v;
+	if (h || sign != 1)
+	{
+		k_call_out<<<grid(n), BLOCK, 0, s>>>(v, n, sign, dst); // (in place without the slots: a thread's own entry)
+		if (!CCF_LAUNCH(ctx, "result of a call")) return false;
+	}
+	if (!h) return CCF_HIP(ctx, copy_out(ctx, out, v, bytes));
+	if (!CCF_HIP(ctx, hipStreamSynchronize(s))) return false;
+	std::memcpy(out, dst, bytes);
+	return true;
+}
+
 bool aberth_sweep_dev(ccf_ctx* ctx, const double* roots, int n, double phi, double* out)
 {
 	if (n <= 0) return true;
-	hipStream_t s = ctx->stream;
 	double2* row = nullptr;
 	SweepBufs B;
-	bool ok = CCF_HIP(ctx, ctx->dmalloc(&row, (size_t)n * sizeof(double2))) && alloc_sweep(ctx, B, 1, n) &&
-		CCF_HIP(ctx, hipMemcpyAsync(row, roots, (size_t)n * sizeof(double2), hipMemcpyHostToDevice, s));
+	bool ok = CCF_HIP(ctx, ctx->dmalloc(&row, (size_t)n * sizeof(double2))) && alloc_sweep(ctx, B, 1, n, false) &&
+		call_in(ctx, roots, row, n, B, 0);
 	if (ok)
 	{
 		const RowMap M{n, 2, 1, 0, 0, phi};
-		k_prepare<<<dim3(grid(n), 1), BLOCK, 0, s>>>(row, M, B, 0, nullptr, nullptr);
-		ok = CCF_LAUNCH(ctx, "prepare") && run_sweeps(ctx, B, row, M, 1, 1, 1) &&
-			CCF_HIP(ctx, hipMemcpyAsync(out, row, (size_t)n * sizeof(double2), hipMemcpyDeviceToHost, s)) &&
-			CCF_HIP(ctx, hipStreamSynchronize(s));
+		ok = run_sweeps(ctx, B, row, M, 1, 1, 1) && call_out(ctx, row, n, 1, out);
 	}
 	ctx->dfree(row);
 	free_sweep(ctx, B);
@@ -3108,22 +3246,6 @@ constexpr int SCRATCH_DEVICES = 64;
 std::mutex scratch_mu;
 unsigned char* scratch_addr[SCRATCH_DEVICES] = {};
 hipError_t scratch_err[SCRATCH_DEVICES] = {}; // a failed look-up of the address, reported by the sweep
-
-// slices of the scratch array, 256-byte aligned; with a null base it only
-// adds up the bytes the slices take
-struct ScratchCarve
-{
-	unsigned char* base;
-	size_t used = 0;
-	template <class T>
-	bool operator()(T*& p, size_t count)
-	{
-		used = (used + 255) & ~size_t(255);
-		p = base ? reinterpret_cast<T*>(base + used) : nullptr;
-		used += count * sizeof(T);
-		return true;
-	}
-};
 
 __global__ void k_fill_int(int* __restrict__ p, size_t n, int v)
 {
@@ -3184,7 +3306,7 @@ bool aberth_sweep_noalloc_dev(ccf_ctx* ctx, const double* roots, int n, double p
 	// FMM's when the context takes it)
 	SweepBufs B;
 	double2* row = nullptr;
-	ScratchCarve size{nullptr};
+	Carve size{nullptr};
 	size(row, (size_t)n);
 	if (!sweep_layout(ctx, B, 1, n, size)) return false;
 	if (size.used > NOALLOC_SCRATCH_BYTES)
@@ -3194,7 +3316,7 @@ bool aberth_sweep_noalloc_dev(ccf_ctx* ctx, const double* roots, int n, double p
 		return false;
 	}
 	B = SweepBufs{};
-	ScratchCarve carve{base};
+	Carve carve{base};
 	carve(row, (size_t)n);
 	if (!sweep_layout(ctx, B, 1, n, carve)) return false;
 	hipStream_t s = ctx->stream;
@@ -3219,37 +3341,26 @@ bool aberth_sweep_noalloc_dev(ccf_ctx* ctx, const double* roots, int n, double p
 bool root_sums_dev(ccf_ctx* ctx, const double* roots, int n, double* out)
 {
 	if (n <= 0) return true;
-	hipStream_t s = ctx->stream;
 	double2* row = nullptr;
 	unsigned long long* stats = nullptr;
 	SweepBufs B;
 	B.rows = 1;
 	B.R = n;
-	std::vector<int> iota(n), one{1};
-	for (int i = 0; i < n; i++) iota[i] = i;
-	std::vector<double2> res(n);
-	bool ok = CCF_HIP(ctx, ctx->dmalloc(&row, (size_t)n * sizeof(double2))) && alloc_root_fmm(ctx, B) &&
-		CCF_HIP(ctx, ctx->dmalloc(&stats, STAT_WORDS * sizeof(unsigned long long))) &&
-		CCF_HIP(ctx, hipMemcpyAsync(row, roots, (size_t)n * sizeof(double2), hipMemcpyHostToDevice, s)) &&
-		CCF_HIP(ctx, hipMemcpyAsync(B.slot, iota.data(), (size_t)n * sizeof(int), hipMemcpyHostToDevice, s)) &&
-		CCF_HIP(ctx, hipMemcpyAsync(B.rmode, one.data(), sizeof(int), hipMemcpyHostToDevice, s));
+	// every root listed at its own index, the row in FMM mode; the pass's
+	// statistics go to a buffer that nothing reads
+	const auto layout = [&](Carve& take) { return take(row, (size_t)n) && take(stats, STAT_WORDS) && root_layout(ctx, B, take); };
+	Carve size{nullptr};
+	unsigned char* mem = nullptr;
+	if (!layout(size) || !CCF_HIP(ctx, ctx->dmalloc(&mem, size.used))) return false;
+	Carve carve{mem};
+	bool ok = layout(carve) && call_in(ctx, roots, row, n, B, 1);
 	if (ok)
 	{
 		const RowMap M{n, 2, 1, 0, 0, 0.0};
-		root_fmm_pass(B, row, M, 1, stats, s);
-		ok = CCF_LAUNCH(ctx, "root-sum FMM") &&
-			CCF_HIP(ctx, hipMemcpyAsync(res.data(), B.rsum, (size_t)n * sizeof(double2), hipMemcpyDeviceToHost, s)) &&
-			CCF_HIP(ctx, hipStreamSynchronize(s));
+		root_fmm_pass(B, row, M, 1, stats, ctx->stream);
+		ok = CCF_LAUNCH(ctx, "root-sum FMM") && call_out(ctx, B.rsum, n, -1, out); // rsum holds -S
 	}
-	if (ok)
-		for (int i = 0; i < n; i++)
-		{
-			out[2 * i] = -res[i].x;
-			out[2 * i + 1] = -res[i].y;
-		}
-	ctx->dfree(row);
-	ctx->dfree(stats);
-	free_sweep(ctx, B);
+	ctx->dfree(mem);
 	return ok;
 }
 
