@@ -23,9 +23,13 @@
 //    the Aberth update and the |dz| / theta < 1e-9 test (ccf_functions.cuh:
 //    379-389). Workgroups take tasks from the queue, largest rows first,
 //    until it is empty.
+//  * the phi chains of an FP64 batch's larger fields, whose sums would keep
+//    one CU each busy long after the others are done, go step by step over
+//    the whole device (k_batch_sweep, k_batch_step_tail);
 //  * the 1/mu error pass (which also forms the caustic map from the same
 //    field evaluation) and the transpose run once over all fields;
-//  * the launches of a solve are captured in a HIP graph and replayed.
+//  * the launches of a solve without such steps are captured in a HIP graph
+//    and replayed.
 // An autotuner picks the workgroup size of each phase by timing the phase's
 // launch on the batch itself.
 #include "chain.hpp"
@@ -469,13 +473,14 @@ __global__ __launch_bounds__(BS, BATCH_WAVES_PER_SIMD) void k_batch(const BField
 	}
 }
 
-// The phi chains of the FP64 form (phase 1): the tasks and the row's place of
-// k_batch, the sweeps of chain_row (sums with shared reciprocals, lanes
-// shared by the roots a sweep lists). A field with the exact sheets takes
-// solve_row's sweeps: at their edge a root can hop until the cap and follows
-// the last bit of its evaluation. 24 fields of 50 to 1000 stars at num_phi
-// 504: 69 ms, 120 ms with solve_row's serial and wave-wide sums; the longest
-// chains (2000 roots) run at about three quarters of a CU's FP64 rate.
+// The phi chains of the FP64 form's small fields (phase 1; the larger ones
+// take k_batch_sweep's steps): the tasks and the row's place of k_batch, the
+// sweeps of chain_row (sums with shared reciprocals, lanes shared by the
+// roots a sweep lists). A workgroup's sweep of a small row is shorter than
+// a launch over the device (CHAIN_ROOTS), and a field's route, so that its
+// bits do not depend on the batch around it, follows from its own size. A
+// field with the exact sheets takes solve_row's sweeps: at their edge a root
+// can hop until the cap and follows the last bit of its evaluation.
 template <int BS>
 __global__ __launch_bounds__(BS, BATCH_WAVES_PER_SIMD) void k_batch_chains(const BField* __restrict__ fields,
 	const BTask* __restrict__ tasks, int ntasks, int* __restrict__ next, int, int rmax, int rlds, int nlds, ListSlice lists)
@@ -549,10 +554,349 @@ __global__ __launch_bounds__(BS, BATCH_WAVES_PER_SIMD) void k_batch_chains(const
 	}
 }
 
+// ---------------------------------------------------------------------------
+// The phi chains of the FP64 form's larger fields, step by step over the
+// whole device: the rows of all fields, branches and sides move on together.
+// A workgroup that runs a chain by itself (k_batch_chains) is bound by the
+// FP64 rate of its one CU, so a batch lasts as long as its largest field
+// (69 ms for 24 fields of 50 to 1000 stars, of which the device's FP64 rate
+// asks 15). Here a step is
+//  - SWEEPS launches of k_batch_sweep, one Jacobi sweep each, a workgroup for
+//    64 roots of a row;
+//  - k_batch_step_tail, one workgroup for a row: the sweeps that are left
+//    (few roots each), the row written out and the next one predicted.
+// The same batch: 25 ms, the dense sweeps at 3.2e12 terms/s.
+
+// a row that takes its steps together with the others'
+struct BRow
+{
+	int field, branch, side;
+	int group;       // its first group of 64 roots
+	long long off;   // its slots of the row buffers
+};
+
+// what a group of 64 roots counts: full updates, early exits, converged, near-field stars
+struct GroupStat
+{
+	unsigned full, early, conv;
+	unsigned long long near;
+};
+
+constexpr int SWEEP_ROOTS = 64;
+// the device-wide sweeps of a step at most (the first two sum over every
+// root, the third evaluates every root; a row with at most TAIL_ROOTS active
+// roots leaves the rest to its tail)
+constexpr int SWEEPS = 4;
+constexpr int TAIL_ROOTS = 64;
+
+// Positions are in the rows' processing order (slot q holds the root
+// order[q]), so a group's roots are neighbours.
+struct RowBufs
+{
+	double2* pos[2];          // start-of-sweep positions of sweep s in pos[s & 1]
+	double2* f1;              // the tails' lists
+	int *la, *lb, *fl;
+	unsigned long long* mask; // active roots of a group, entering the next sweep
+	int* act;                 // [rows][SWEEPS + 1] active roots entering a sweep (from the second on)
+	GroupStat* stat;          // of a group
+};
+
+// whether sweep s of a step runs over the device for a row
+__device__ inline bool device_sweep(const int* act, int s, int cap)
+{
+	return s < min(SWEEPS, cap) && (s == 0 || act[s] > TAIL_ROOTS);
+}
+
+// One Jacobi sweep of a group: four lanes a root for the Witt function and
+// the 1/mu exit, then the Cauchy sums, lanes over the roots and the four
+// waves over quarters of the sources (read through scalar loads); a group
+// with at most SWEEP_SPARSE roots to sum has a wave's lanes over the sources.
+// Every root is written to the other buffer, moved or not, so a sweep reads
+// start-of-sweep positions only, and a root's arithmetic depends on its row
+// and group alone. Bound by the FP64 VALU in the dense sweeps.
+constexpr int SWEEP_SPARSE = 24;
+
+__global__ __launch_bounds__(BLOCK, 4) void k_batch_sweep(const BField* __restrict__ fields, const BRow* __restrict__ rows,
+	const int2* __restrict__ items, RowBufs B, int j, int s)
+{
+	const int2 it = items[blockIdx.x];
+	const BRow W = rows[it.x];
+	const BField& F = fields[W.field];
+	if (j > F.np / (2 * F.nb)) return;
+	int* const act = B.act + (size_t)it.x * (SWEEPS + 1);
+	// (act[s] <= TAIL_ROOTS holds for every later sweep too: it is 0 there)
+	if (!device_sweep(act, s, F.cap_step)) return;
+	const LensView& L = F.L;
+	const int R = F.R, N = F.N, q0 = it.y * SWEEP_ROOTS, nq = min(SWEEP_ROOTS, R - q0);
+	const double2* __restrict__ zr = B.pos[s & 1] + W.off;
+	double2* __restrict__ zn = B.pos[(s + 1) & 1] + W.off;
+	const int g = W.group + it.y;
+	const unsigned long long all = nq == 64 ? ~0ull : (1ull << nq) - 1;
+	const unsigned long long active = s == 0 ? all : B.mask[g];
+	__shared__ unsigned long long s_full, s_early;
+	__shared__ unsigned s_near;
+	__shared__ double2 s_f0[SWEEP_ROOTS], s_f1[SWEEP_ROOTS], s_p[BLOCK / 64][SWEEP_ROOTS];
+	const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	if (threadIdx.x == 0)
+	{
+		s_full = s_early = 0;
+		s_near = 0;
+	}
+	__syncthreads();
+	if (active)
+	{
+		const double2 e = F.cs[centre_row(F, W.branch) + (W.side ? j : -j)];
+		constexpr int EL = BLOCK / SWEEP_ROOTS;
+		const int l = threadIdx.x / EL, sub = threadIdx.x & (EL - 1);
+		const bool valid = (active >> l) & 1;
+		cd z;
+		int node = 0;
+		if (valid)
+		{
+			const double2 v = zr[q0 + l];
+			z = cd(v.x, v.y);
+			node = nearest_node(L, z);
+		}
+		const bool outside = valid && L.nf_off[node] < 0;
+		Near nr;
+		for (unsigned long long m = __ballot(outside && sub == 0); m; m &= m - 1)
+		{
+			const int src = __ffsll(m) - 1;
+			const Near t = wave_near(L, __shfl(node, src, 64), cd(__shfl(z.re, src, 64), __shfl(z.im, src, 64)));
+			if ((lane & ~(EL - 1)) == src) nr = t;
+		}
+		if (valid)
+		{
+			if (!outside) nr = chain_near(L, node, z, sub, EL);
+			const Witt w = witt_from(L, z, e.x, e.y, node, nr);
+			if (sub == 0)
+			{
+				if (w.early) atomicOr(&s_early, 1ull << l);
+				else
+				{
+					const cd f1 = witt_f1(L, z, w);
+					s_f0[l] = make_double2(w.f0.re, w.f0.im);
+					s_f1[l] = make_double2(f1.re, f1.im);
+					atomicOr(&s_full, 1ull << l);
+					atomicAdd(&s_near, (unsigned)w.nr.count);
+				}
+			}
+		}
+	}
+	__syncthreads();
+	const unsigned long long full = s_full;
+	const int nf = __popcll(full);
+	const double2* __restrict__ st = F.stars;
+	if (nf > SWEEP_SPARSE)
+	{
+		constexpr int NW = BLOCK / 64;
+		const double2 z = zr[q0 + min(lane, nq - 1)];
+		const int s0 = (int)((long long)wv * N / NW), s1 = (int)((long long)(wv + 1) * N / NW);
+		const int r0 = (int)((long long)wv * R / NW), r1 = (int)((long long)(wv + 1) * R / NW);
+		double ax = 0, ay = 0;
+		cauchy_run<1>(st, s0, s1, z.x, z.y, ax, ay); // ccf_functions.cuh:218-227
+		ax *= 2;
+		ay *= 2;
+		cauchy_run<-1>(zr, r0, r1, z.x, z.y, ax, ay); // ccf_functions.cuh:232-239
+		if (!(isfinite(ax) && isfinite(ay)))
+		{
+			// out of cauchy4's range: the terms one by one
+			ax = ay = 0;
+			for (int q = s0; q < s1; q++) cauchy1<1>(z.x, z.y, st[q], ax, ay);
+			ax *= 2;
+			ay *= 2;
+			for (int q = r0; q < r1; q++) cauchy1<-1>(z.x, z.y, zr[q], ax, ay);
+		}
+		s_p[wv][lane] = make_double2(ax, -ay);
+	}
+	else
+	{
+		// wave w takes every fourth listed root
+		int k = 0;
+		for (unsigned long long m = full; m; m &= m - 1, k++)
+		{
+			if ((k & (BLOCK / 64 - 1)) != wv) continue;
+			const int l = __ffsll(m) - 1;
+			const double2 z = zr[q0 + l];
+			double ax = 0, ay = 0;
+			cauchy_lanes<1>(st, 0, N, z.x, z.y, ax, ay);
+			ax *= 2;
+			ay *= 2;
+			cauchy_lanes<-1>(zr, 0, R, z.x, z.y, ax, ay);
+			if (!(isfinite(ax) && isfinite(ay)))
+			{
+				ax = ay = 0;
+				for (int q = lane; q < N; q += 64) cauchy1<1>(z.x, z.y, st[q], ax, ay);
+				ax *= 2;
+				ay *= 2;
+				for (int q = lane; q < R; q += 64) cauchy1<-1>(z.x, z.y, zr[q], ax, ay);
+			}
+			for (int o = 32; o >= 1; o >>= 1)
+			{
+				ax += __shfl_xor(ax, o, 64);
+				ay += __shfl_xor(ay, o, 64);
+			}
+			if (lane == 0) s_p[0][l] = make_double2(ax, -ay);
+		}
+	}
+	__syncthreads();
+	if (wv != 0) return;
+	// the update, a lane a root
+	bool left = false;
+	if (lane < nq)
+	{
+		double2 v = zr[q0 + lane];
+		if ((full >> lane) & 1)
+		{
+			double2 t = s_p[0][lane];
+			if (nf > SWEEP_SPARSE)
+				for (int k = 1; k < BLOCK / 64; k++)
+				{
+					t.x += s_p[k][lane].x;
+					t.y += s_p[k][lane].y;
+				}
+			const double2 a0 = s_f0[lane], a1 = s_f1[lane];
+			const cd z(v.x, v.y), f0(a0.x, a0.y), f1(a1.x, a1.y);
+			const cd q = z - f0 / (f1 + f0 * cd(t.x, t.y));
+			left = !((q - z).abs() / L.theta < CONV_TOL); // a non-finite step stays active
+			v = make_double2(q.re, q.im);
+		}
+		zn[q0 + lane] = v;
+	}
+	const unsigned long long next = __ballot(left);
+	if (lane == 0)
+	{
+		const unsigned nearly = __popcll(s_early), n = __popcll(next);
+		B.mask[g] = next;
+		if (n) atomicAdd(&act[s + 1], (int)n);
+		GroupStat c = B.stat[g];
+		c.full += nf;
+		c.early += nearly;
+		c.conv += nearly + nf - n;
+		c.near += s_near;
+		B.stat[g] = c;
+	}
+}
+
+// The end of step j of a row: the sweeps its device-wide ones left, the row
+// to the output in root order, and the start of step j + 1
+// (prepare_roots_kernel, ccf_functions.cuh:261-295); j = 0 only predicts.
+// Bound by the latency of a few sweeps of few roots. The row and the stars
+// are staged in LDS where they fit (a listed root's sums read all of them).
+constexpr int TAIL_BLOCK = 1024;
+constexpr int TAIL_LIST = 2 * TAIL_ROOTS; // active roots whose lists fit in LDS
+
+__global__ __launch_bounds__(TAIL_BLOCK) void k_batch_step_tail(const BField* __restrict__ fields, const BRow* __restrict__ rows,
+	int first, RowBufs B, int j, int rlds, int nlds)
+{
+	extern __shared__ double2 smem[];
+	__shared__ int s_n[2];
+	__shared__ int s_list[3][TAIL_LIST];
+	__shared__ double2 s_f[2][TAIL_LIST];
+	__shared__ unsigned long long s_red[CHAIN_COUNTS];
+	const int r = first + blockIdx.x;
+	const BRow W = rows[r];
+	const BField& F = fields[W.field];
+	const int steps = F.np / (2 * F.nb);
+	if (j > steps) return;
+	const int R = F.R, N = F.N, sgn = W.side ? 1 : -1, row = centre_row(F, W.branch) + sgn * j;
+	double2* const out = F.roots + (size_t)row * R;
+	if (j > 0)
+	{
+		int* const act = B.act + (size_t)r * (SWEEPS + 1);
+		int done = 0;
+		while (device_sweep(act, done, F.cap_step)) done++;
+		const int n = done > 0 ? act[done] : R;
+		double2* const zr = B.pos[done & 1] + W.off;
+		if (threadIdx.x == 0) s_n[0] = s_n[1] = 0;
+		if (threadIdx.x < CHAIN_COUNTS) s_red[threadIdx.x] = 0;
+		__syncthreads();
+		int cc[CHAIN_COUNTS] = {0, 0, 0, 0, 0};
+		if (n > 0 && done < F.cap_step)
+		{
+			// the active roots from the groups' masks (their order does not matter)
+			const bool small = n <= TAIL_LIST;
+			ChainLists cl;
+			cl.la = small ? s_list[0] : B.la + W.off;
+			for (int q = threadIdx.x; q < R; q += TAIL_BLOCK)
+				if (done == 0 || (B.mask[W.group + q / SWEEP_ROOTS] >> (q % SWEEP_ROOTS) & 1)) cl.la[atomicAdd(&s_n[0], 1)] = q;
+			const double2 e = F.cs[row];
+			const bool staged = R <= rlds && N <= nlds;
+			double2* const sl = smem + rlds;
+			if (staged)
+			{
+				for (int q = threadIdx.x; q < R; q += TAIL_BLOCK) smem[q] = zr[q];
+				for (int q = threadIdx.x; q < N; q += TAIL_BLOCK) sl[q] = F.stars[q];
+			}
+			__syncthreads();
+			if (threadIdx.x == 0) s_n[0] = 0;
+			__syncthreads();
+			if (small && staged)
+			{
+				const ChainLists c{s_list[0], s_list[1], s_list[2], s_f[0], s_f[1]};
+				chain_row<TAIL_BLOCK>(F.L, R, N, 0, F.cap_step - done, e.x, e.y, smem, sl, c, n, s_n, cc);
+			}
+			else
+			{
+				cl.lb = small ? s_list[1] : B.lb + W.off;
+				cl.fl = small ? s_list[2] : B.fl + W.off;
+				// (the other buffer's row is free until the next step is predicted)
+				cl.f0 = small ? s_f[0] : B.pos[(done + 1) & 1] + W.off;
+				cl.f1 = small ? s_f[1] : B.f1 + W.off;
+				chain_row<TAIL_BLOCK>(F.L, R, N, 0, F.cap_step - done, e.x, e.y, staged ? smem : zr, staged ? sl : F.stars, cl, n, s_n, cc);
+			}
+			if (staged)
+				for (int q = threadIdx.x; q < R; q += TAIL_BLOCK) out[F.order[q]] = smem[q];
+		}
+		if (!(n > 0 && done < F.cap_step && R <= rlds && N <= nlds))
+			for (int q = threadIdx.x; q < R; q += TAIL_BLOCK) out[F.order[q]] = zr[q];
+		// the counts: the tail's own now, the groups' with the last step
+		unsigned long long v[CHAIN_COUNTS];
+		for (int k = 0; k < CHAIN_COUNTS; k++) v[k] = (unsigned long long)cc[k];
+		if (threadIdx.x == 0) v[4] += (unsigned long long)done;
+		if (j == steps)
+			for (int g = threadIdx.x; g < (R + SWEEP_ROOTS - 1) / SWEEP_ROOTS; g += TAIL_BLOCK)
+			{
+				const GroupStat c = B.stat[W.group + g];
+				v[0] += c.full;
+				v[1] += c.early;
+				v[2] += c.conv;
+				v[3] += c.near;
+			}
+#pragma unroll
+		for (int k = 0; k < CHAIN_COUNTS; k++)
+			if (__any(v[k] != 0))
+			{
+				const unsigned long long t = wave_sum(v[k]);
+				if ((threadIdx.x & 63) == 0) atomicAdd(&s_red[k], t);
+			}
+		__syncthreads(); // (and act has been read)
+		if (threadIdx.x < CHAIN_COUNTS)
+		{
+			const int which[CHAIN_COUNTS] = {B_FULL, B_EARLY, B_CONV, B_NEAR, B_SWEEPS};
+			if (s_red[threadIdx.x]) atomicAdd(&F.stats[which[threadIdx.x]], s_red[threadIdx.x]);
+		}
+		if (j == steps) return;
+		if (threadIdx.x <= SWEEPS) act[threadIdx.x] = 0;
+	}
+	// (a thread reads what it wrote in this step and the ones before)
+	const int q1 = min(F.predictor, j);
+	for (int q = threadIdx.x; q < R; q += TAIL_BLOCK)
+		B.pos[0][W.off + q] = predict_root(out + F.order[q], (long long)sgn * R, q1);
+}
+
 __global__ void k_zero_int(int* p, int n)
 {
 	const int i = blockIdx.x * blockDim.x + threadIdx.x;
 	if (i < n) p[i] = 0;
+}
+
+// the counters of the rows and groups (words ints and words2 8-byte words)
+__global__ void k_zero_rows(int* act, int words, unsigned long long* stat, int words2)
+{
+	const int i = blockIdx.x * blockDim.x + threadIdx.x;
+	if (i < words) act[i] = 0;
+	if (i < words2) stat[i] = 0;
 }
 
 __global__ void k_zero_u64(unsigned long long* p, int n)
@@ -740,7 +1084,16 @@ struct BatchDevice
 	int* next = nullptr;
 	unsigned long long* stats = nullptr;
 	int n0 = 0, n1 = 0, nf = 0;
-	int rmax = 0, rlds = 0, nlds = 0, maxrows = 0; // roots of the largest row, rows held in LDS, stars in LDS
+	int rmax = 0, maxrows = 0;             // roots of the largest row, phi rows of the longest field
+	int rlds[2] = {0, 0}, nlds[2] = {0, 0}; // of the centres' and the chains' tasks: row held in LDS, stars in LDS
+	// the rows that take their steps together (FP64)
+	BRow* rows = nullptr;
+	int2* items = nullptr;   // (row, group of SWEEP_ROOTS roots), largest rows first
+	RowBufs rb{};
+	char* row_mem = nullptr;
+	int nrows = 0, ngroups = 0, steps = 0;
+	int row_half = 0, item_half = 0; // the rows and items of the first of two streams
+	int trlds = 0, tnlds = 0; // row and stars that a tail stages in LDS
 	long long maxpts = 0;
 };
 
@@ -750,7 +1103,7 @@ namespace
 void free_bdev(ccf_ctx* m, BatchDevice& d)
 {
 	auto F = [m](auto*& p) { m->dfree(p); p = nullptr; };
-	F(d.slices); F(d.eoff); F(d.list_mem); F(d.fields); F(d.tasks0); F(d.tasks1); F(d.next); F(d.stats);
+	F(d.slices); F(d.eoff); F(d.list_mem); F(d.fields); F(d.tasks0); F(d.tasks1); F(d.next); F(d.stats); F(d.rows); F(d.items); F(d.row_mem);
 	d = BatchDevice{};
 }
 
@@ -766,7 +1119,8 @@ int batch_grid(ccf_batch* b, int phase, int bs)
 	const bool mixed = m->P.precision == 1;
 	const BatchKernel fn = pick_kernel(phase, mixed, bs);
 	int per_cu = 0;
-	if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)fn, bs, batch_lds(d.rlds, d.nlds)) != hipSuccess || per_cu < 1)
+	if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)fn, bs, batch_lds(d.rlds[phase], d.nlds[phase])) != hipSuccess ||
+		per_cu < 1)
 		per_cu = 1;
 	const int cus = m->num_cus > 0 ? m->num_cus : 256;
 	// the list buffers hold d.list_wgs workgroups
@@ -779,8 +1133,9 @@ bool launch_batch_phase(ccf_batch* b, int phase, int bs, int g, hipStream_t s)
 	BatchDevice& d = *b->dev;
 	const bool mixed = m->P.precision == 1;
 	const BatchKernel fn = pick_kernel(phase, mixed, bs);
-	const size_t lds = batch_lds(d.rlds, d.nlds);
+	const size_t lds = batch_lds(d.rlds[phase], d.nlds[phase]);
 	const int ntasks = phase == 0 ? d.n0 : d.n1;
+	if (ntasks == 0) return true;
 	if (g > d.list_wgs)
 	{
 		m->fail("Error. The batched grid exceeds its list buffers\n");
@@ -788,7 +1143,7 @@ bool launch_batch_phase(ccf_batch* b, int phase, int bs, int g, hipStream_t s)
 	}
 	k_zero_int<<<1, 64, 0, s>>>(d.next, 1);
 	hipLaunchKernelGGL(fn, dim3(g), dim3(bs), lds, s, (const BField*)d.fields, (const BTask*)(phase == 0 ? d.tasks0 : d.tasks1),
-		ntasks, d.next, phase, d.rmax, d.rlds, d.nlds, d.lists);
+		ntasks, d.next, phase, d.rmax, d.rlds[phase], d.nlds[phase], d.lists);
 	return CCF_LAUNCH(m, "batched Aberth solve");
 }
 
@@ -801,13 +1156,58 @@ bool launch_post(ccf_batch* b, hipStream_t s)
 	return CCF_LAUNCH(m, "batched errors, transpose, caustics");
 }
 
+// the steps of the rows that move on together
+bool launch_steps(ccf_batch* b, hipStream_t s)
+{
+	ccf_ctx* m = b->master;
+	BatchDevice& d = *b->dev;
+	const int words = d.nrows * (SWEEPS + 1), words2 = (int)(d.ngroups * (sizeof(GroupStat) / sizeof(unsigned long long)));
+	k_zero_rows<<<grid(std::max(words, words2)), BLOCK, 0, s>>>(d.rb.act, words, (unsigned long long*)d.rb.stat, words2);
+	const size_t lds = batch_lds(d.trlds, d.tnlds);
+	// Two halves of the rows on two streams: one's tails and last workgroups
+	// leave most of the device to the other's dense sweeps.
+	if (!group_streams_start(m, 2)) return false;
+	const hipStream_t st[2] = {s, m->group_streams[0]};
+	const int r0[3] = {0, d.row_half, d.nrows}, i0[3] = {0, d.item_half, d.ngroups};
+	for (int j = 0; j <= d.steps; j++)
+		for (int h = 0; h < 2; h++)
+		{
+			const int nr = r0[h + 1] - r0[h], ni = i0[h + 1] - i0[h];
+			if (nr == 0) continue;
+			for (int q = 0; q < SWEEPS && j > 0; q++)
+				k_batch_sweep<<<ni, BLOCK, 0, st[h]>>>(d.fields, d.rows, d.items + i0[h], d.rb, j, q);
+			k_batch_step_tail<<<nr, TAIL_BLOCK, lds, st[h]>>>(d.fields, d.rows, r0[h], d.rb, j, d.trlds, d.tnlds);
+		}
+	return CCF_LAUNCH(m, "batched phi steps") && group_streams_join(m, 2);
+}
+
+// the chains: a workgroup each for small fields, beside the steps of the
+// larger ones
+bool launch_chains(ccf_batch* b, hipStream_t s)
+{
+	ccf_ctx* m = b->master;
+	BatchDevice& d = *b->dev;
+	if (d.nrows == 0) return launch_batch_phase(b, 1, b->block1, b->grid1, s);
+	hipStream_t side = s;
+	if (d.n1 > 0)
+	{
+		if (!m->err_stream && !CCF_HIP(m, hipStreamCreateWithFlags(&m->err_stream, hipStreamNonBlocking))) return false;
+		if (!m->err_event && !CCF_HIP(m, hipEventCreateWithFlags(&m->err_event, hipEventDisableTiming))) return false;
+		side = m->err_stream;
+		if (!CCF_HIP(m, hipEventRecord(m->err_event, s)) || !CCF_HIP(m, hipStreamWaitEvent(side, m->err_event, 0)) ||
+			!launch_batch_phase(b, 1, b->block1, b->grid1, side))
+			return false;
+	}
+	if (!launch_steps(b, s)) return false;
+	return d.n1 == 0 || (CCF_HIP(m, hipEventRecord(m->err_event, side)) && CCF_HIP(m, hipStreamWaitEvent(s, m->err_event, 0)));
+}
+
 // the whole solve of a loaded and built batch, on stream s
 bool enqueue_solve(ccf_batch* b, hipStream_t s)
 {
 	BatchDevice& d = *b->dev;
 	k_zero_u64<<<grid((long long)d.nf * BSTAT), BLOCK, 0, s>>>(d.stats, d.nf * BSTAT);
-	return launch_batch_phase(b, 0, b->block, b->grid0, s) && launch_batch_phase(b, 1, b->block1, b->grid1, s) &&
-		launch_post(b, s);
+	return launch_batch_phase(b, 0, b->block, b->grid0, s) && launch_chains(b, s) && launch_post(b, s);
 }
 
 } // namespace
@@ -948,7 +1348,7 @@ bool batch_build(ccf_batch* b, int verbose)
 	lap("result arena");
 	// device tables
 	std::vector<BField> hf(nf);
-	std::vector<BTask> t0, t1;
+	std::vector<BTask> t0, t1, t2; // centres, chains, rows that take their steps together
 	for (int f = 0; f < nf; f++)
 	{
 		ccf_ctx* c = b->fields[f];
@@ -1015,29 +1415,36 @@ bool batch_build(ccf_batch* b, int verbose)
 		for (int br = 0; br < nb; br++)
 		{
 			t0.push_back(BTask{f, br, 0, cost});
-			t1.push_back(BTask{f, br, 0, cost});
-			t1.push_back(BTask{f, br, 1, cost});
+			std::vector<BTask>& t = m->P.precision == 0 && F.chained && R > CHAIN_ROOTS ? t2 : t1;
+			t.push_back(BTask{f, br, 0, cost});
+			t.push_back(BTask{f, br, 1, cost});
 		}
 	}
-	// LDS of a workgroup: the largest row that fits (larger rows are solved
-	// in place in global memory), then as many stars as fit
-	const long long lim = batch_lds_limit(m);
-	for (const BField& F : hf)
-		if ((long long)batch_lds(F.R, 0) <= lim) d.rlds = std::max(d.rlds, F.R);
 	// largest rows first (longest-processing-time order of the queue)
 	auto by_cost = [](const BTask& a, const BTask& b2) { return a.cost > b2.cost; };
-	std::stable_sort(t0.begin(), t0.end(), by_cost);
-	std::stable_sort(t1.begin(), t1.end(), by_cost);
+	for (std::vector<BTask>* t : {&t0, &t1, &t2}) std::stable_sort(t->begin(), t->end(), by_cost);
 	d.n0 = (int)t0.size();
 	d.n1 = (int)t1.size();
-	const long long room = lim - (long long)batch_lds(d.rlds, 0);
-	int nmax = 0;
-	for (ccf_ctx* c : b->fields) nmax = std::max(nmax, c->num_stars);
-	d.nlds = (int)std::max(0LL, std::min<long long>(nmax, room / (long long)sizeof(double2)));
-	// the mixed form takes the pole sum from the star FMM, or else its FP32
-	// terms from the FP32 star copy: no star is read from LDS, which then
-	// holds only the row (more workgroups per CU)
-	if (m->P.precision == 1) d.nlds = 0;
+	// LDS of a workgroup: the largest row that fits (larger rows are solved
+	// in place in global memory), then as many stars as fit. The mixed form
+	// takes the pole sum from the star FMM, or else its FP32 terms from the
+	// FP32 star copy: no star is read from LDS, which then holds only the row
+	// (more workgroups per CU)
+	const long long lim = batch_lds_limit(m);
+	auto lds_of = [&](const std::vector<BTask>& t, long long limit, int& rl, int& nl) {
+		int nmax = 0;
+		rl = 0;
+		for (const BTask& k : t)
+		{
+			const BField& F = hf[k.field];
+			if ((long long)batch_lds(F.R, 0) <= limit) rl = std::max(rl, F.R);
+			nmax = std::max(nmax, F.N);
+		}
+		const long long room = limit - (long long)batch_lds(rl, 0);
+		nl = m->P.precision == 1 ? 0 : (int)std::max(0LL, std::min<long long>(nmax, room / (long long)sizeof(double2)));
+	};
+	lds_of(t0, lim, d.rlds[0], d.nlds[0]);
+	lds_of(t1, lim, d.rlds[1], d.nlds[1]);
 	// list buffers for the largest persistent grid (no more workgroups than
 	// tasks): rmax slots per workgroup
 	{
@@ -1053,6 +1460,46 @@ bool batch_build(ccf_batch* b, int verbose)
 		d.lists.lb = d.lists.la + slots;
 	}
 	lap("field tables");
+	if (!t2.empty())
+	{
+		lds_of(t2, lim, d.trlds, d.tnlds);
+		std::vector<BRow> rows;
+		std::vector<int2> items;
+		long long slots = 0;
+		// (side by side: the halves have the same work)
+		std::stable_partition(t2.begin(), t2.end(), [](const BTask& t) { return t.side == 0; });
+		for (const BTask& t : t2)
+		{
+			const BField& F = hf[t.field];
+			if (t.side == 0) d.row_half = (int)rows.size() + 1;
+			const int groups = grid(F.R, SWEEP_ROOTS);
+			for (int g = 0; g < groups; g++) items.push_back(make_int2((int)rows.size(), g));
+			rows.push_back(BRow{t.field, t.branch, t.side, (int)items.size() - groups, slots});
+			if (t.side == 0) d.item_half = (int)items.size();
+			slots += (long long)groups * SWEEP_ROOTS;
+			d.steps = std::max(d.steps, F.np / (2 * F.nb));
+		}
+		d.nrows = (int)rows.size();
+		d.ngroups = (int)items.size();
+		const size_t bytes = (size_t)slots * (3 * sizeof(double2) + 3 * sizeof(int)) +
+			(size_t)d.ngroups * (sizeof(GroupStat) + sizeof(unsigned long long)) + (size_t)d.nrows * (SWEEPS + 1) * sizeof(int);
+		if (!CCF_HIP(m, m->dmalloc(&d.row_mem, bytes)) || !CCF_HIP(m, m->dmalloc(&d.rows, sizeof(BRow) * rows.size())) ||
+			!CCF_HIP(m, m->dmalloc(&d.items, sizeof(int2) * items.size())) ||
+			!CCF_HIP(m, hipMemcpyAsync(d.rows, rows.data(), sizeof(BRow) * rows.size(), hipMemcpyHostToDevice, s)) ||
+			!CCF_HIP(m, hipMemcpyAsync(d.items, items.data(), sizeof(int2) * items.size(), hipMemcpyHostToDevice, s)) ||
+			!CCF_HIP(m, hipStreamSynchronize(s)))
+			return false;
+		RowBufs& B = d.rb;
+		B.pos[0] = (double2*)d.row_mem;
+		B.pos[1] = B.pos[0] + slots;
+		B.f1 = B.pos[1] + slots;
+		B.stat = (GroupStat*)(B.f1 + slots);
+		B.mask = (unsigned long long*)(B.stat + d.ngroups);
+		B.la = (int*)(B.mask + d.ngroups);
+		B.lb = B.la + slots;
+		B.fl = B.lb + slots;
+		B.act = B.fl + slots;
+	}
 	// error-pass blocks of each field (fewer than 2^31 points per field and blocks in all)
 	std::vector<int> eoff(nf);
 	long long eb = 0;
@@ -1079,7 +1526,7 @@ bool batch_build(ccf_batch* b, int verbose)
 	if (!CCF_HIP(m, m->dmalloc(&d.stats, sizeof(unsigned long long) * nf * BSTAT))) return false;
 	for (int f = 0; f < nf; f++) hf[f].stats = d.stats + (size_t)f * BSTAT;
 	return CCF_HIP(m, m->dmalloc(&d.fields, sizeof(BField) * nf)) && CCF_HIP(m, m->dmalloc(&d.tasks0, sizeof(BTask) * d.n0)) &&
-		CCF_HIP(m, m->dmalloc(&d.tasks1, sizeof(BTask) * d.n1)) && CCF_HIP(m, m->dmalloc(&d.next, sizeof(int))) &&
+		CCF_HIP(m, m->dmalloc(&d.tasks1, sizeof(BTask) * std::max(1, d.n1))) && CCF_HIP(m, m->dmalloc(&d.next, sizeof(int))) &&
 		CCF_HIP(m, hipMemcpyAsync(d.fields, hf.data(), sizeof(BField) * nf, hipMemcpyHostToDevice, s)) &&
 		CCF_HIP(m, hipMemcpyAsync(d.tasks0, t0.data(), sizeof(BTask) * d.n0, hipMemcpyHostToDevice, s)) &&
 		CCF_HIP(m, hipMemcpyAsync(d.tasks1, t1.data(), sizeof(BTask) * d.n1, hipMemcpyHostToDevice, s)) &&
@@ -1154,7 +1601,13 @@ bool batch_solve(ccf_batch* b, int verbose)
 	b->grid0 = batch_grid(b, 0, b->block);
 	b->grid1 = batch_grid(b, 1, b->block1);
 	auto t0 = std::chrono::steady_clock::now();
-	if (!b->graph_exec)
+	// (hundreds of launches of a few microseconds: the host queues them while
+	// the device works, and recording them would cost a rebuilt batch more)
+	if (d.nrows > 0)
+	{
+		if (!enqueue_solve(b, s)) return false;
+	}
+	else if (!b->graph_exec)
 	{
 		if (!CCF_HIP(m, hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal))) return false;
 		const bool ok = enqueue_solve(b, s);
@@ -1167,7 +1620,8 @@ bool batch_solve(ccf_batch* b, int verbose)
 			std::cout << "batch solve: graph captured and instantiated in "
 					  << std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count() << " ms\n";
 	}
-	if (!CCF_HIP(m, hipGraphLaunch(b->graph_exec, s)) || !CCF_HIP(m, hipStreamSynchronize(s))) return false;
+	if (d.nrows == 0 && !CCF_HIP(m, hipGraphLaunch(b->graph_exec, s))) return false;
+	if (!CCF_HIP(m, hipStreamSynchronize(s))) return false;
 	auto t1 = std::chrono::steady_clock::now();
 	const double dt = std::chrono::duration<double>(t1 - t0).count();
 	std::vector<unsigned long long> st((size_t)d.nf * BSTAT);

@@ -76,6 +76,40 @@ __device__ __forceinline__ void cauchy1(double zx, double zy, double2 w, double&
 	ay = fma(dy, iv, ay);
 }
 
+// the terms of src[lo, hi) for a lane's target: every lane of the wave reads
+// the same source, so the sources come through scalar loads
+template <int SIGN>
+__device__ __forceinline__ void cauchy_run(const double2* __restrict__ src, int lo, int hi, double zx, double zy, double& ax,
+	double& ay)
+{
+	int q = lo;
+#pragma unroll 2
+	for (; q + 4 <= hi; q += 4)
+	{
+		const double2 w[4] = {src[q], src[q + 1], src[q + 2], src[q + 3]};
+		cauchy4<SIGN>(zx, zy, w, ax, ay);
+	}
+	for (; q < hi; q++) cauchy1<SIGN>(zx, zy, src[q], ax, ay);
+}
+
+// the same terms of one target, the wave's lanes over the sources (four of
+// its own at a time): the lane's part of the sum
+template <int SIGN>
+__device__ __forceinline__ void cauchy_lanes(const double2* __restrict__ src, int lo, int hi, double zx, double zy, double& ax,
+	double& ay)
+{
+	const int lane = threadIdx.x & 63;
+	int q0 = lo;
+#pragma unroll 1
+	for (; q0 + 256 <= hi; q0 += 256)
+	{
+		const double2 w[4] = {src[q0 + lane], src[q0 + 64 + lane], src[q0 + 128 + lane], src[q0 + 192 + lane]};
+		cauchy4<SIGN>(zx, zy, w, ax, ay);
+	}
+#pragma unroll 1
+	for (int q = q0 + lane; q < hi; q += 64) cauchy1<SIGN>(zx, zy, src[q], ax, ay);
+}
+
 // The near-field sums of a root outside the tree (its node is not a leaf:
 // every star of the node's ranges), by the lanes of one wave: lane l sums
 // the stars l, l + 64, ... of the ranges (p2p's terms), and a butterfly of
@@ -233,6 +267,9 @@ __device__ __forceinline__ void chain_terms(const double2* src, int m, double2 z
 // what a workgroup counts of its rows: full updates, early exits, converged,
 // near-field stars (of updates that formed f1), sweeps
 constexpr int CHAIN_COUNTS = 5;
+
+// rows of at most this many roots run their phi chain as one workgroup
+constexpr int CHAIN_ROOTS = 480;
 
 struct ChainLists
 {

@@ -350,6 +350,8 @@ hipError_t copy_out(ccf_ctx* c, void* dst, const void* src, size_t bytes);
 bool alloc_sweep(ccf_ctx* ctx, SweepBufs& b, int rows, int R, bool clear = true);
 void free_sweep(ccf_ctx* ctx, SweepBufs& b);
 bool alloc_solver(ccf_ctx* ctx);
+bool group_streams_start(ccf_ctx* ctx, int G);
+bool group_streams_join(ccf_ctx* ctx, int G);
 bool find_initial_roots_dev(ccf_ctx* ctx, int verbose);
 bool find_ccs_dev(ccf_ctx* ctx, int verbose);
 bool find_caustics_dev(ccf_ctx* ctx, bool caustics, bool mu);

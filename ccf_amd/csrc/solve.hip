@@ -805,40 +805,6 @@ __global__ __launch_bounds__(BLOCK) void k_sums64(const double2* __restrict__ sp
 // continuation step's sparse sweeps gain more: waves as items, lanes over the
 // sources.
 
-// the terms of src[lo, hi) for a lane's target: every lane of the wave reads
-// the same source, so the sources come through scalar loads
-template <int SIGN>
-__device__ __forceinline__ void cauchy_run(const double2* __restrict__ src, int lo, int hi, double zx, double zy, double& ax,
-	double& ay)
-{
-	int q = lo;
-#pragma unroll 2
-	for (; q + 4 <= hi; q += 4)
-	{
-		const double2 w[4] = {src[q], src[q + 1], src[q + 2], src[q + 3]};
-		cauchy4<SIGN>(zx, zy, w, ax, ay);
-	}
-	for (; q < hi; q++) cauchy1<SIGN>(zx, zy, src[q], ax, ay);
-}
-
-// the same terms of one target, the wave's lanes over the sources (four of
-// its own at a time): the lane's part of the sum
-template <int SIGN>
-__device__ __forceinline__ void cauchy_lanes(const double2* __restrict__ src, int lo, int hi, double zx, double zy, double& ax,
-	double& ay)
-{
-	const int lane = threadIdx.x & 63;
-	int q0 = lo;
-#pragma unroll 1
-	for (; q0 + 256 <= hi; q0 += 256)
-	{
-		const double2 w[4] = {src[q0 + lane], src[q0 + 64 + lane], src[q0 + 128 + lane], src[q0 + 192 + lane]};
-		cauchy4<SIGN>(zx, zy, w, ax, ay);
-	}
-#pragma unroll 1
-	for (int q = q0 + lane; q < hi; q += 64) cauchy1<SIGN>(zx, zy, src[q], ax, ay);
-}
-
 // One wave takes an item, a tile of QUAD_TILE listed roots and a slice of
 // the terms, by itself: no LDS and no barrier. A row with at most QUAD_SPARSE
 // listed roots has the wave's lanes over the slice's sources instead of over
@@ -1645,7 +1611,6 @@ __global__ __launch_bounds__(TAIL_BLOCK) void k_tail(LensView L, double2* __rest
 // wide step of so few roots takes about 145 us whatever they are: the chains
 // are faster up to CHAIN_ROOTS (400 roots: 112 us a step; 600: 184).
 constexpr int CHAIN_BLOCK = 1024;
-constexpr int CHAIN_ROOTS = 480;
 
 inline size_t chain_lds(int R, int N)
 {
