@@ -658,40 +658,48 @@ double ms_seconds(double s) { return std::floor(s * 1000.0) / 1000.0; } // stopw
 // 57. So the array is cut into a part per thread, and each thread takes its
 // part through two pinned slots of its own: the device fills one while the
 // thread copies (and first touches) the pages of the other. 646 MB: 61 -> 17
-// ms with 8 threads.
+// ms with 8 threads. Arrays of less than a part take one thread, none of
+// them started: above about 256 KiB the runtime pins the caller's pages for
+// a copy (320 KB: 150 -> 40 us, 3 MB: 740 -> 290).
 //
-// The pinned slots (COPY_THREADS x 2 x COPY_CHUNK = 32 MiB) and their events
-// are shared by the process's contexts: made by the first large copy, used by
+// The pinned slots (two of COPY_CHUNK for each of COPY_THREADS threads: 32
+// MiB at most) and their events are shared by the process's contexts: a
+// thread's are made by the first copy that takes as many threads, used by
 // one copy at a time (a copy that finds them taken goes through hipMemcpy),
 // and given back when the last context is destroyed.
 constexpr int COPY_THREADS = 8;
 constexpr size_t COPY_CHUNK = size_t(2) << 20;
-constexpr size_t COPY_MIN = size_t(4) << 20; // smaller arrays: hipMemcpy (a thread's start costs what they would save)
+constexpr size_t COPY_PART = size_t(512) << 10; // least bytes of a thread's part (a thread's start is about 20 us)
+constexpr size_t COPY_MIN = size_t(256) << 10;  // smaller arrays: hipMemcpy
 
 struct CopySlots
 {
 	std::mutex use;  // held by the copy that uses the slots
 	std::mutex life; // guards contexts
 	long contexts = 0;
-	char* mem = nullptr;
+	char* mem[COPY_THREADS] = {};
 	hipEvent_t event[2 * COPY_THREADS] = {};
 
-	bool ready()
+	// the slots of the first T threads
+	bool ready(int T)
 	{
-		if (mem) return true;
-		for (hipEvent_t& e : event)
-			if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess)
+		for (int t = 0; t < T; t++)
+		{
+			for (int k = 2 * t; k < 2 * t + 2; k++)
+				if (!event[k] && hipEventCreateWithFlags(&event[k], hipEventDisableTiming) != hipSuccess)
+				{
+					event[k] = nullptr;
+					(void)hipGetLastError();
+					return false;
+				}
+			if (!mem[t] && hipHostMalloc((void**)&mem[t], 2 * COPY_CHUNK, hipHostMallocDefault) != hipSuccess)
 			{
-				e = nullptr;
+				mem[t] = nullptr;
 				(void)hipGetLastError();
 				return false;
 			}
-		if (hipHostMalloc((void**)&mem, 2 * COPY_THREADS * COPY_CHUNK, hipHostMallocDefault) != hipSuccess)
-		{
-			mem = nullptr;
-			(void)hipGetLastError();
 		}
-		return mem != nullptr;
+		return true;
 	}
 	void release()
 	{
@@ -701,8 +709,11 @@ struct CopySlots
 			if (e) (void)hipEventDestroy(e);
 			e = nullptr;
 		}
-		if (mem) (void)hipHostFree(mem);
-		mem = nullptr;
+		for (char*& p : mem)
+		{
+			if (p) (void)hipHostFree(p);
+			p = nullptr;
+		}
 	}
 };
 
@@ -772,9 +783,9 @@ int guarded(ccf_ctx* c, F&& f)
 hipError_t ccf::copy_out(ccf_ctx* c, void* dst, const void* src, size_t bytes)
 {
 	CopySlots& cs = copy_slots();
-	const int T = bytes >= COPY_MIN && c->stream ? std::min<size_t>(copy_threads(), bytes / COPY_CHUNK) : 1;
+	const int T = bytes >= COPY_MIN && c->stream ? (int)std::max<size_t>(1, std::min<size_t>(copy_threads(), bytes / COPY_PART)) : 0;
 	std::unique_lock<std::mutex> lock(cs.use, std::defer_lock);
-	if (T < 2 || !lock.try_lock() || !cs.ready())
+	if (T < 1 || !lock.try_lock() || !cs.ready(T))
 	{
 		if (!c->stream) return hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost);
 		const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream);
@@ -783,7 +794,7 @@ hipError_t ccf::copy_out(ccf_ctx* c, void* dst, const void* src, size_t bytes)
 	std::atomic<int> bad{hipSuccess};
 	auto part = [&](int t) noexcept {
 		const size_t lo = bytes / T * t, hi = t + 1 == T ? bytes : bytes / T * (t + 1);
-		char* const slot[2] = {cs.mem + 2 * t * COPY_CHUNK, cs.mem + (2 * t + 1) * COPY_CHUNK};
+		char* const slot[2] = {cs.mem[t], cs.mem[t] + COPY_CHUNK};
 		hipEvent_t const event[2] = {cs.event[2 * t], cs.event[2 * t + 1]};
 		const hipError_t e = copy_part((char*)dst, (const char*)src, lo, hi, slot, event, c->stream);
 		if (e != hipSuccess) bad = e;

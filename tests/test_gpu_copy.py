@@ -13,8 +13,11 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("n,num_phi,nb", [
-    (64, 2046, 1),    # 2047 x 128 points: 4 192 256 B, just below the slots' smallest array
-    (64, 2048, 2),    # 2050 x 128 points: 4 198 400 B, two parts
+    (64, 124, 2),     # 126 x 128 points: 258 048 B, just below the slots' smallest array
+    (64, 128, 1),     # 129 x 128 points: 264 192 B, one part
+    (64, 512, 1),     # 513 x 128 points: 1 050 624 B, two parts
+    (64, 2046, 1),    # 2047 x 128 points: 4 192 256 B, seven parts
+    (64, 2048, 2),    # 2050 x 128 points: 4 198 400 B, eight parts
     (137, 2000, 4),   # 8.8 MB, odd parts
     (700, 1200, 6),   # 27 MB, more parts than threads
 ])
