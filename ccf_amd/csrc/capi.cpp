@@ -157,7 +157,8 @@ void ccf_ctx::free_device()
 	F(T.field); F(T.nf); F(T.nnf); F(T.nbox); F(T.nf_off); F(T.nf_cnt); F(T.nfs); F(T.mp); F(T.loc); F(T.loc32); F(T.mpu); F(T.locu); F(T.locu32); F(T.binom); F(T.lookup);
 	T = ccf::DeviceTree{};
 	F(spos); F(smass); F(spos_tmp); F(smass_tmp); F(spos32); F(ts_a); F(ts_b); F(ones);
-	F(ccs_init); F(phase); F(dseeds); F(dorder);
+	F(ccs_init); F(phase); F(dseeds); F(dorder); F(chain_mem);
+	chain_bytes = 0;
 	if (results_borrowed)
 	{
 		ccs = caustics = nullptr;
@@ -902,6 +903,13 @@ int ccf_set_params(ccf_ctx* c, const ccf_params* p)
 	ccf_params a = before, b = c->P_in;
 	a.timing = b.timing = 0;
 	if (std::memcmp(&a, &b, sizeof(a)) != 0) c->tuned = false;
+	return 0;
+}
+
+int ccf_set_team_wait(ccf_ctx* c, long long ticks)
+{
+	if (!c) return 1;
+	c->team_wait = ticks;
 	return 0;
 }
 

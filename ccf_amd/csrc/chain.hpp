@@ -268,7 +268,9 @@ __device__ __forceinline__ void chain_terms(const double2* src, int m, double2 z
 // near-field stars (of updates that formed f1), sweeps
 constexpr int CHAIN_COUNTS = 5;
 
-// rows of at most this many roots run their phi chain as one workgroup
+// A batch's rows of at most this many roots run their phi chain as one
+// workgroup, whose time grows with the square of its roots (400 roots: 112
+// us a step; 600: 184); a step over the device takes 70 us and more.
 constexpr int CHAIN_ROOTS = 480;
 
 struct ChainLists
@@ -280,128 +282,150 @@ struct ChainLists
 	double2* f1; // its derivative; then the moved root
 };
 
+// A sweep's three phases, between barriers, as in the batched form's
+// solve_row (batch.hip): zc holds the row's roots, st the stars.
+
+// Witt function and 1/mu exit of the n roots listed in cur, chain_eval_lanes
+// lanes a root (a root outside the tree, whose near field is every star, by
+// its whole wave); the roots that take the Cauchy sums are appended to ls.fl
+// (*nf their count, zero before)
+template <int BS>
+__device__ __forceinline__ void chain_evaluate(const LensView& L, double cp, double sp, const double2* zc, const int* cur, int n,
+	const ChainLists& ls, int* nf, int (&cnt)[CHAIN_COUNTS])
+{
+	const int lane = threadIdx.x & 63;
+	const unsigned long long below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+	const int W = chain_eval_lanes(n), sub = threadIdx.x & (W - 1), step = BS / W;
+	// whole waves go round together (the last round's idle lanes help
+	// with the roots outside the tree)
+	for (int q0 = 0; q0 < n; q0 += step)
+	{
+		const int q = q0 + threadIdx.x / W;
+		const bool valid = q < n;
+		if (__ballot(valid) == 0) continue;
+		const int i = valid ? cur[q] : 0;
+		cd z;
+		int node = 0;
+		if (valid)
+		{
+			z = cd(zc[i].x, zc[i].y);
+			node = nearest_node(L, z);
+		}
+		const bool outside = valid && L.nf_off[node] < 0;
+		Near nr;
+		for (unsigned long long m = __ballot(outside && sub == 0); m; m &= m - 1)
+		{
+			const int src = __ffsll(m) - 1;
+			const Near t = wave_near(L, __shfl(node, src, 64), cd(__shfl(z.re, src, 64), __shfl(z.im, src, 64)));
+			if ((lane & ~(W - 1)) == src) nr = t;
+		}
+		bool full = false;
+		Witt w;
+		cd f1;
+		if (valid)
+		{
+			if (!outside) nr = chain_near(L, node, z, sub, W);
+			w = witt_from(L, z, cp, sp, node, nr);
+			if (!w.early) f1 = witt_f1(L, z, w);
+			full = !w.early && sub == 0;
+			cnt[0] += full;
+			cnt[1] += w.early && sub == 0;
+			cnt[2] += w.early && sub == 0;
+			cnt[3] += full ? w.nr.count : 0;
+		}
+		const unsigned long long m = __ballot(full);
+		if (m)
+		{
+			int base = 0;
+			if (lane == 0) base = atomicAdd(nf, (int)__popcll(m));
+			base = __shfl(base, 0, 64);
+			if (full)
+			{
+				const int k = base + (int)__popcll(m & below);
+				ls.fl[k] = i;
+				ls.f0[k] = make_double2(w.f0.re, w.f0.im);
+				ls.f1[k] = make_double2(f1.re, f1.im);
+			}
+		}
+	}
+}
+
+// the Cauchy sums of the nf listed roots, chain_sum_lanes lanes each, and
+// where they move to (in ls.f1)
+template <int BS>
+__device__ __forceinline__ void chain_sums(int R, int N, int circ_exact, const double2* zc, const double2* st, const ChainLists& ls, int nf)
+{
+	const int W = chain_sum_lanes(nf, N + R), sub = threadIdx.x & (W - 1);
+	for (int g = threadIdx.x / W; g < nf; g += BS / W)
+	{
+		const double2 z = zc[ls.fl[g]];
+		double ax = 0, ay = 0;
+		chain_terms<1>(st, N, z, sub, W, ax, ay);
+		ax *= 2;
+		ay *= 2;
+		chain_terms<-1>(zc, R, z, sub, W, ax, ay);
+		if (!(isfinite(ax) && isfinite(ay)))
+		{
+			// out of cauchy4's range: the lane's terms one by one
+			ax = ay = 0;
+			for (int q = sub; q < N; q += W) cauchy1<1>(z.x, z.y, st[q], ax, ay);
+			ax *= 2;
+			ay *= 2;
+			for (int q = sub; q < R; q += W) cauchy1<-1>(z.x, z.y, zc[q], ax, ay);
+		}
+		for (int o = 1; o < W; o <<= 1)
+		{
+			ax += __shfl_xor(ax, o, 64);
+			ay += __shfl_xor(ay, o, 64);
+		}
+		if (sub == 0)
+		{
+			const double2 a0 = ls.f0[g], a1 = ls.f1[g];
+			const cd zz(z.x, z.y), f0(a0.x, a0.y), f1(a1.x, a1.y);
+			cd sum(ax, -ay);
+			if (circ_exact) sum += 2.0 * zz.inv(); // ccf_functions.cuh:223-227
+			const cd zn = zz - f0 / (f1 + f0 * sum);
+			ls.f1[g] = make_double2(zn.re, zn.im);
+		}
+	}
+}
+
+// the nf updates written and tested, the roots that are left in nxt (*left
+// their count)
+template <int BS>
+__device__ __forceinline__ void chain_update(const LensView& L, double2* zc, const ChainLists& ls, int nf, int* nxt, int* left,
+	int (&cnt)[CHAIN_COUNTS])
+{
+	for (int g = threadIdx.x; g < nf; g += BS)
+	{
+		const int i = ls.fl[g];
+		const double2 v = ls.f1[g];
+		const cd dz(v.x - zc[i].x, v.y - zc[i].y);
+		zc[i] = v;
+		if (dz.abs() / L.theta < CONV_TOL) cnt[2]++;
+		else nxt[atomicAdd(left, 1)] = i; // a non-finite step stays active
+	}
+}
+
 // The sweeps of one row (at most cap) from the n active roots in ls.la (as
 // written before a barrier): zc holds its roots, st the stars, ls room for
-// the row's lists. s_cnt: two ints of LDS, zero. Three barrier-separated
-// phases a sweep, as in the batched form's solve_row (batch.hip):
-//  - Witt function and 1/mu exit, chain_eval_lanes lanes a root (a root
-//    outside the tree, whose near field is every star, by its whole wave);
-//  - Cauchy sums, chain_sum_lanes lanes a listed root, and its update;
-//  - the updates written and tested once every sum is formed.
+// the row's lists. s_cnt: two ints of LDS, zero.
 template <int BS>
 __device__ __forceinline__ void chain_row(const LensView& L, int R, int N, int circ_exact, int cap, double cp, double sp, double2* zc,
 	const double2* st, const ChainLists& ls, int n, int* s_cnt, int (&cnt)[CHAIN_COUNTS])
 {
-	const int lane = threadIdx.x & 63;
-	const unsigned long long below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
 	int* cur = ls.la;
 	int* nxt = ls.lb;
 	// s_cnt: listed this sweep, active next
 	for (int it = 0; it < cap && n > 0; it++)
 	{
 		cnt[4] += threadIdx.x == 0;
-		{
-			const int W = chain_eval_lanes(n), sub = threadIdx.x & (W - 1), step = BS / W;
-			// whole waves go round together (the last round's idle lanes help
-			// with the roots outside the tree)
-			for (int q0 = 0; q0 < n; q0 += step)
-			{
-				const int q = q0 + threadIdx.x / W;
-				const bool valid = q < n;
-				if (__ballot(valid) == 0) continue;
-				const int i = valid ? cur[q] : 0;
-				cd z;
-				int node = 0;
-				if (valid)
-				{
-					z = cd(zc[i].x, zc[i].y);
-					node = nearest_node(L, z);
-				}
-				const bool outside = valid && L.nf_off[node] < 0;
-				Near nr;
-				for (unsigned long long m = __ballot(outside && sub == 0); m; m &= m - 1)
-				{
-					const int src = __ffsll(m) - 1;
-					const Near t = wave_near(L, __shfl(node, src, 64), cd(__shfl(z.re, src, 64), __shfl(z.im, src, 64)));
-					if ((lane & ~(W - 1)) == src) nr = t;
-				}
-				bool full = false;
-				Witt w;
-				cd f1;
-				if (valid)
-				{
-					if (!outside) nr = chain_near(L, node, z, sub, W);
-					w = witt_from(L, z, cp, sp, node, nr);
-					if (!w.early) f1 = witt_f1(L, z, w);
-					full = !w.early && sub == 0;
-					cnt[0] += full;
-					cnt[1] += w.early && sub == 0;
-					cnt[2] += w.early && sub == 0;
-					cnt[3] += full ? w.nr.count : 0;
-				}
-				const unsigned long long m = __ballot(full);
-				if (m)
-				{
-					int base = 0;
-					if (lane == 0) base = atomicAdd(&s_cnt[0], (int)__popcll(m));
-					base = __shfl(base, 0, 64);
-					if (full)
-					{
-						const int k = base + (int)__popcll(m & below);
-						ls.fl[k] = i;
-						ls.f0[k] = make_double2(w.f0.re, w.f0.im);
-						ls.f1[k] = make_double2(f1.re, f1.im);
-					}
-				}
-			}
-		}
+		chain_evaluate<BS>(L, cp, sp, zc, cur, n, ls, &s_cnt[0], cnt);
 		__syncthreads();
 		const int nf = s_cnt[0];
-		{
-			const int W = chain_sum_lanes(nf, N + R), sub = threadIdx.x & (W - 1);
-			for (int g = threadIdx.x / W; g < nf; g += BS / W)
-			{
-				const double2 z = zc[ls.fl[g]];
-				double ax = 0, ay = 0;
-				chain_terms<1>(st, N, z, sub, W, ax, ay);
-				ax *= 2;
-				ay *= 2;
-				chain_terms<-1>(zc, R, z, sub, W, ax, ay);
-				if (!(isfinite(ax) && isfinite(ay)))
-				{
-					// out of cauchy4's range: the lane's terms one by one
-					ax = ay = 0;
-					for (int q = sub; q < N; q += W) cauchy1<1>(z.x, z.y, st[q], ax, ay);
-					ax *= 2;
-					ay *= 2;
-					for (int q = sub; q < R; q += W) cauchy1<-1>(z.x, z.y, zc[q], ax, ay);
-				}
-				for (int o = 1; o < W; o <<= 1)
-				{
-					ax += __shfl_xor(ax, o, 64);
-					ay += __shfl_xor(ay, o, 64);
-				}
-				if (sub == 0)
-				{
-					const double2 a0 = ls.f0[g], a1 = ls.f1[g];
-					const cd zz(z.x, z.y), f0(a0.x, a0.y), f1(a1.x, a1.y);
-					cd sum(ax, -ay);
-					if (circ_exact) sum += 2.0 * zz.inv(); // ccf_functions.cuh:223-227
-					const cd zn = zz - f0 / (f1 + f0 * sum);
-					ls.f1[g] = make_double2(zn.re, zn.im);
-				}
-			}
-		}
+		chain_sums<BS>(R, N, circ_exact, zc, st, ls, nf);
 		__syncthreads();
-		for (int g = threadIdx.x; g < nf; g += BS)
-		{
-			const int i = ls.fl[g];
-			const double2 v = ls.f1[g];
-			const cd dz(v.x - zc[i].x, v.y - zc[i].y);
-			zc[i] = v;
-			if (dz.abs() / L.theta < CONV_TOL) cnt[2]++;
-			else nxt[atomicAdd(&s_cnt[1], 1)] = i; // a non-finite step stays active
-		}
+		chain_update<BS>(L, zc, ls, nf, nxt, &s_cnt[1], cnt);
 		__syncthreads();
 		n = s_cnt[1];
 		int* const t = cur;

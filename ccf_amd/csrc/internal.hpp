@@ -236,6 +236,9 @@ struct ccf_ctx
 	std::vector<ccf::Timer> witt_timers;
 	std::vector<ccf::Timer> tail_timers;
 	// the timers' events, created once and reused once the timers are read
+	char* chain_mem = nullptr;    // FP64 chains of small fields: see ChainTeams (solve.hip)
+	size_t chain_bytes = 0;
+	long long team_wait = -1;     // ccf_set_team_wait
 	std::vector<hipEvent_t> events;
 	size_t events_used = 0;
 	hipEvent_t next_event()

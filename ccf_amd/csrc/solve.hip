@@ -1600,62 +1600,219 @@ __global__ __launch_bounds__(TAIL_BLOCK) void k_tail(LensView L, double2* __rest
 	block_stats<8, TAIL_BLOCK>(stats, which, v);
 }
 
-// The FP64 continuation of a small field in one launch: a workgroup per
-// (branch, side) takes its whole chain of phi steps, the row, its stars and
-// its lists in LDS (chain_row). A step's sweeps over a few hundred roots are
-// bound by the latency of their launches (and were by their read-backs: 9.4
-// ms for the 50 steps of 200 roots at num_phi 100, 2.9 ms in one launch).
-// 1024 threads, though they spill 12 bytes at 128 VGPRs: four waves a SIMD
-// keep the FP64 pipe busier than two do (3.4 ms with 512 threads and no
-// spill). A workgroup's time grows with the square of its roots, a device-
-// wide step of so few roots takes about 145 us whatever they are: the chains
-// are faster up to CHAIN_ROOTS (400 roots: 112 us a step; 600: 184).
+// The FP64 continuation of a small field in one launch: a team of K
+// workgroups per (branch, side) takes its whole chain of phi steps, the row,
+// its stars and its lists in LDS. A step's sweeps over a few hundred roots
+// are bound by the latency of their launches when they run over the device
+// (and were by their read-backs: 9.4 ms for the 50 steps of 200 roots at
+// num_phi 100); one workgroup (2.9 ms) is bound by its CU's FP64 rate in two
+// sweeps a step and by the latency of an evaluation. As teams of 32: 1.7 ms;
+// 1000 roots: 2.7 ms against 7.7 in sweeps over the device.
+//
+// A member owns the roots lo .. hi of the processing order: it evaluates,
+// sums and moves them as chain_row does, and after a sweep every member
+// publishes its roots' positions and takes in the others'. 1024 threads,
+// though they spill a few bytes at 128 VGPRs: four waves a SIMD keep the
+// FP64 pipe busier than two do.
+//
+// The members meet in memory once a sweep: positions and arrivals are
+// agent-scope atomic accesses, which are coherent between the XCDs' L2s, and
+// a wave's stores have been acknowledged (vmcnt 0) before its workgroup
+// arrives, so no cache needs writing back or invalidating. They run at the
+// same time as long as the device has room for all (at most TEAM_WGS
+// workgroups, a quarter of the CUs, so the process's four hardware queues
+// may each hold such a launch). Should a member wait for longer than `wait`
+// all the same, it raises the flag, every member leaves, and the launch that
+// follows (RETRY, one workgroup per row, which otherwise only hands the
+// counts on) does the members' work in turn, with the same arithmetic.
 constexpr int CHAIN_BLOCK = 1024;
+constexpr int TEAM_WGS = 64;
+constexpr int TEAM_MAX = 32;
+constexpr int TEAM_ROOTS = 8;                     // fewest roots of a member
+constexpr long long TEAM_WAIT = 20 * 1000 * 1000; // 0.2 s of the 100 MHz clock
 
-inline size_t chain_lds(int R, int N)
+// one team's meeting point, in a line of its own: arrivals (high word) and
+// active roots (low word) of the last four sweeps
+struct alignas(128) TeamSlot
 {
-	return (size_t)R * (3 * sizeof(double2) + 3 * sizeof(int)) + (size_t)N * sizeof(double2) + sizeof(int);
+	unsigned long long arrived[4];
+};
+
+struct ChainTeams
+{
+	TeamSlot* slots;              // [rows]
+	unsigned long long* counts;   // [CHAIN_COUNTS] of the members, handed on by the second launch
+	int* flag;                    // a member gave up waiting
+	double2* pos;                 // [rows][2][R] published positions, by sweep parity
+	long long wait;
+	int K;
+};
+
+// LDS of a member (lists of n roots: its own, or the row's in the second launch)
+inline size_t chain_lds(int R, int N, int n)
+{
+	return (size_t)(R + N) * sizeof(double2) + (size_t)n * (2 * sizeof(double2) + 3 * sizeof(int));
 }
 
+inline int chain_team(int R, int rows) { return std::max(1, std::min(std::min(TEAM_MAX, TEAM_WGS / rows), R / TEAM_ROOTS)); }
+
+// Whether a field's chains run as teams. A step of theirs takes 30 to 90 us
+// (3.6 sweeps of 7 us, and a member's share of the sums), one over the
+// device about 150 us and more with more rows: measured with one to ten
+// branches, the two meet where a member sums 0.7 to 0.9 million terms a
+// sweep (500 stars, 10 branches, teams of 2: 187 us either way). The launch
+// that stands in for the teams holds a row and all its lists in LDS (about
+// 2280 roots).
+constexpr long long TEAM_TERMS = 600 * 1000;
+constexpr size_t CHAIN_LDS = 152 * 1024;
+
+inline bool chain_fits(int R, int N, int rows)
+{
+	return chain_lds(R, N, R) <= CHAIN_LDS && (long long)R * (R + N) / chain_team(R, rows) <= TEAM_TERMS;
+}
+
+__global__ void k_clear_teams(ChainTeams T, int rows)
+{
+	for (int i = threadIdx.x; i < rows; i += blockDim.x)
+		for (int k = 0; k < 4; k++) T.slots[i].arrived[k] = 0;
+	if (threadIdx.x < CHAIN_COUNTS) T.counts[threadIdx.x] = 0;
+	if (threadIdx.x == 0) *T.flag = 0;
+}
+
+// what thread 0 of a member does between publishing and taking in: arrives
+// with its active roots and waits for the others; the team's active roots,
+// or -1 once a member has given up
+__device__ inline int team_meet(const ChainTeams& T, TeamSlot& slot, unsigned epoch, int member, int active)
+{
+	unsigned long long* const a = &slot.arrived[epoch & 3];
+	__hip_atomic_fetch_add(a, (1ull << 32) | (unsigned)active, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+	const long long t0 = wall_clock64();
+	unsigned long long v;
+	while ((int)((v = __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) >> 32) < T.K)
+	{
+		if (wall_clock64() - t0 >= T.wait) __hip_atomic_store(T.flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+		if (__hip_atomic_load(T.flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return -1;
+		__builtin_amdgcn_s_sleep(1);
+	}
+	// every member has left the sweep before this one: its slot serves the
+	// sweep three on (no member reaches that one before this store, which
+	// completes before the member's next arrival)
+	if (member == 0) __hip_atomic_store(&slot.arrived[(epoch + 3) & 3], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+	return (int)(unsigned)v;
+}
+
+// a member's roots lo .. hi published and the others' taken in; false once a
+// member has given up. Every thread of the workgroup calls it.
+__device__ __forceinline__ bool team_exchange(const ChainTeams& T, int r, unsigned& epoch, int member, int R, int lo, int hi, double2* zc,
+	int& active, int* s_meet)
+{
+	unsigned long long* const p = reinterpret_cast<unsigned long long*>(T.pos + (size_t)(2 * r + (epoch & 1)) * R);
+	for (int k = 2 * lo + threadIdx.x; k < 2 * hi; k += CHAIN_BLOCK)
+		__hip_atomic_store(p + k, reinterpret_cast<const unsigned long long*>(zc)[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+	asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+	__syncthreads();
+	if (threadIdx.x == 0) *s_meet = team_meet(T, T.slots[r], epoch, member, active);
+	__syncthreads();
+	active = *s_meet;
+	if (active < 0) return false;
+	const int other = 2 * (R - (hi - lo));
+	for (int q = threadIdx.x; q < other; q += CHAIN_BLOCK)
+	{
+		const int k = q < 2 * lo ? q : q + 2 * (hi - lo);
+		reinterpret_cast<unsigned long long*>(zc)[k] = __hip_atomic_load(p + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+	}
+	epoch++;
+	__syncthreads();
+	return true;
+}
+
+template <bool RETRY>
 __global__ __launch_bounds__(CHAIN_BLOCK) void k_chains(LensView L, double2* __restrict__ roots, const double2* __restrict__ cs, int R,
-	int N, int np, int nb, int steps, int cap, int predictor, int circ_exact, const int* __restrict__ order,
+	int N, int np, int nb, int steps, int cap, int predictor, const int* __restrict__ order, ChainTeams T,
 	unsigned long long* __restrict__ stats)
 {
 	extern __shared__ double2 chain_mem[];
-	__shared__ int s_cnt[2];
-	double2* const zc = chain_mem;
+	__shared__ int s_nf[TEAM_MAX], s_left[TEAM_MAX], s_meet;
+	const int rows = 2 * nb, r = RETRY ? blockIdx.x : blockIdx.x % rows;
+	const int K = T.K;
+	const int m0 = RETRY ? 0 : blockIdx.x / rows, m1 = RETRY ? K : m0 + 1; // the members this workgroup is
+	const auto first = [&](int m) { return (int)((long long)R * m / K); };
+	const int lo = first(m0), hi = first(m1);
+	const int which[CHAIN_COUNTS] = {C_TAIL_FULL, C_TAIL_EARLY, C_CONV, C_TAIL_NEAR, C_TAIL_SWEEPS};
+	if (RETRY && *T.flag == 0)
+	{
+		if (r == 0 && threadIdx.x < CHAIN_COUNTS) atomicAdd(stat_slot(stats, which[threadIdx.x]), T.counts[threadIdx.x]);
+		return;
+	}
+	double2* const zc = chain_mem; // in processing order
 	double2* const st = zc + R;
-	ChainLists ls;
-	ls.f0 = st + N;
-	ls.f1 = ls.f0 + R;
-	ls.la = reinterpret_cast<int*>(ls.f1 + R);
-	ls.lb = ls.la + R;
-	ls.fl = ls.lb + R;
-	const int c = blockIdx.x >> 1, sgn = (blockIdx.x & 1) == 0 ? -1 : 1;
+	double2* const f0 = st + N;
+	double2* const f1 = f0 + (hi - lo);
+	int* cur = reinterpret_cast<int*>(f1 + (hi - lo));
+	int* nxt = cur + (hi - lo);
+	int* const fl = nxt + (hi - lo);
+	const int c = r >> 1, sgn = (r & 1) == 0 ? -1 : 1;
 	const int center = np / (2 * nb) + c * (np / nb + 1);
 	int cnt[CHAIN_COUNTS] = {0, 0, 0, 0, 0};
+	unsigned epoch = 0;
 	for (int s = threadIdx.x; s < N; s += CHAIN_BLOCK) st[s] = L.spos[s];
+	for (int p = threadIdx.x; p < R; p += CHAIN_BLOCK) zc[p] = roots[(size_t)center * R + order[p]];
+	if (threadIdx.x < TEAM_MAX) s_nf[threadIdx.x] = s_left[threadIdx.x] = 0;
 	for (int j = 1; j <= steps; j++)
 	{
-		const int row = center + sgn * j;
+		const int row = center + sgn * j, q = min(predictor, j - 1);
 		const double2 e = cs[row];
-		double2* const out = roots + (size_t)row * R;
-		const int q = min(predictor, j - 1);
-		// (a thread reads what it wrote in the earlier steps)
-		for (int i = threadIdx.x; i < R; i += CHAIN_BLOCK)
+		if (q > 0)
 		{
-			zc[i] = predict_root(roots + (size_t)(row - sgn) * R + i, (long long)sgn * R, q);
-			ls.la[i] = order[i];
+			// (a thread reads what it wrote in the earlier steps)
+			for (int p = lo + threadIdx.x; p < hi; p += CHAIN_BLOCK)
+				zc[p] = predict_root(roots + (size_t)(row - sgn) * R + order[p], (long long)sgn * R, q);
+			__syncthreads(); // (a position is published by another thread)
+			int none = 0;
+			if (!RETRY && K > 1 && !team_exchange(T, r, epoch, m0, R, lo, hi, zc, none, &s_meet)) return;
 		}
-		if (threadIdx.x == 0) s_cnt[0] = s_cnt[1] = 0;
+		for (int p = lo + threadIdx.x; p < hi; p += CHAIN_BLOCK) cur[p - lo] = p;
 		__syncthreads();
-		chain_row<CHAIN_BLOCK>(L, R, N, circ_exact, cap, e.x, e.y, zc, st, ls, R, s_cnt, cnt);
-		for (int i = threadIdx.x; i < R; i += CHAIN_BLOCK) out[i] = zc[i];
+		int n[RETRY ? TEAM_MAX : 1];
+		for (int m = m0; m < m1; m++) n[m - m0] = first(m + 1) - first(m);
+		int active = R;
+		for (int it = 0; it < cap && active > 0; it++)
+		{
+			cnt[4] += threadIdx.x == 0 && m0 == 0;
+			const auto lists = [&](int m) {
+				const int o = first(m) - lo;
+				return ChainLists{cur + o, nxt + o, fl + o, f0 + o, f1 + o};
+			};
+			for (int m = m0; m < m1; m++) chain_evaluate<CHAIN_BLOCK>(L, e.x, e.y, zc, lists(m).la, n[m - m0], lists(m), &s_nf[m - m0], cnt);
+			__syncthreads();
+			for (int m = m0; m < m1; m++) chain_sums<CHAIN_BLOCK>(R, N, 0, zc, st, lists(m), s_nf[m - m0]);
+			__syncthreads();
+			for (int m = m0; m < m1; m++) chain_update<CHAIN_BLOCK>(L, zc, lists(m), s_nf[m - m0], lists(m).lb, &s_left[m - m0], cnt);
+			__syncthreads();
+			active = 0;
+			for (int m = m0; m < m1; m++) active += n[m - m0] = s_left[m - m0];
+			__syncthreads();
+			if (threadIdx.x < TEAM_MAX) s_nf[threadIdx.x] = s_left[threadIdx.x] = 0;
+			if (!RETRY && K > 1)
+			{
+				if (!team_exchange(T, r, epoch, m0, R, lo, hi, zc, active, &s_meet)) return;
+			}
+			else __syncthreads();
+			int* const t = cur;
+			cur = nxt;
+			nxt = t;
+		}
+		for (int p = lo + threadIdx.x; p < hi; p += CHAIN_BLOCK) roots[(size_t)row * R + order[p]] = zc[p];
 	}
-	const int which[CHAIN_COUNTS] = {C_TAIL_FULL, C_TAIL_EARLY, C_CONV, C_TAIL_NEAR, C_TAIL_SWEEPS};
 	unsigned long long v[CHAIN_COUNTS];
 	for (int t = 0; t < CHAIN_COUNTS; t++) v[t] = (unsigned long long)cnt[t];
-	block_stats<CHAIN_COUNTS, CHAIN_BLOCK>(stats, which, v);
+	if (RETRY) block_stats<CHAIN_COUNTS, CHAIN_BLOCK>(stats, which, v);
+	else
+		for (int t = 0; t < CHAIN_COUNTS; t++)
+		{
+			const unsigned long long w = wave_sum(v[t]);
+			if ((threadIdx.x & 63) == 0 && w) atomicAdd(&T.counts[t], w);
+		}
 }
 
 // The FP64 form's tail: the sweeps of a continuation step after its device-
@@ -2706,12 +2863,35 @@ bool find_initial_roots_dev(ccf_ctx* ctx, int verbose)
 }
 
 // whether a field's continuation runs as k_chains: FP64 with direct sums, and
-// rows of at most CHAIN_ROOTS roots, above which the sweeps over the whole
-// device are faster. Not with the exact sheets, at whose edge a root can hop
+// rows for which that is faster (chain_fits). Not with the exact sheets, at whose edge a root can hop
 // until the cap and follows the last bit of its evaluation.
 bool chain_field(const ccf_ctx* ctx)
 {
-	return ctx->P.precision == 0 && ctx->P.approx && ctx->P.root_fmm != 1 && ctx->num_roots <= CHAIN_ROOTS;
+	return ctx->P.precision == 0 && ctx->P.approx && ctx->P.root_fmm != 1 &&
+		chain_fits(ctx->num_roots, ctx->num_stars, 2 * ctx->P.num_branches);
+}
+
+// the teams' meeting points and published positions, kept with the field
+bool chain_teams(ccf_ctx* ctx, ChainTeams& T, int K)
+{
+	const int R = ctx->num_roots, rows = 2 * ctx->P.num_branches;
+	const size_t slots = sizeof(TeamSlot) * (rows + 1);
+	const size_t bytes = slots + (size_t)rows * 2 * R * sizeof(double2);
+	if (bytes > ctx->chain_bytes)
+	{
+		ctx->dfree(ctx->chain_mem);
+		ctx->chain_mem = nullptr;
+		ctx->chain_bytes = 0;
+		if (!CCF_HIP(ctx, ctx->dmalloc(&ctx->chain_mem, bytes))) return false;
+		ctx->chain_bytes = bytes;
+	}
+	T.slots = (TeamSlot*)ctx->chain_mem;
+	T.counts = (unsigned long long*)(T.slots + rows);
+	T.flag = (int*)(T.counts + CHAIN_COUNTS);
+	T.pos = (double2*)(ctx->chain_mem + slots);
+	T.wait = ctx->team_wait >= 0 ? ctx->team_wait : TEAM_WAIT;
+	T.K = K;
+	return true;
 }
 
 bool find_ccs_dev(ccf_ctx* ctx, int verbose)
@@ -2807,8 +2987,14 @@ bool find_ccs_dev(ccf_ctx* ctx, int verbose)
 			tt.b = ctx->next_event();
 			if (tt.a && tt.b) (void)hipEventRecord(tt.a, s);
 		}
-		k_chains<<<2 * nb, CHAIN_BLOCK, chain_lds(R, ctx->num_stars), s>>>(L, ctx->ccs_init, ctx->phase, R, ctx->num_stars, np, nb, steps,
-			cap, ctx->P.predictor, 0, ctx->dorder, ctx->counters);
+		const int K = chain_team(R, 2 * nb), N = ctx->num_stars;
+		ChainTeams T;
+		if (!chain_teams(ctx, T, K)) return false;
+		k_clear_teams<<<1, 64, 0, s>>>(T, 2 * nb);
+		k_chains<false><<<2 * nb * K, CHAIN_BLOCK, chain_lds(R, N, (R + K - 1) / K), s>>>(L, ctx->ccs_init, ctx->phase, R, N, np, nb, steps,
+			cap, ctx->P.predictor, ctx->dorder, T, ctx->counters);
+		k_chains<true><<<2 * nb, CHAIN_BLOCK, chain_lds(R, N, R), s>>>(L, ctx->ccs_init, ctx->phase, R, N, np, nb, steps, cap,
+			ctx->P.predictor, ctx->dorder, T, ctx->counters);
 		if (ctx->P.timing && tt.a && tt.b)
 		{
 			(void)hipEventRecord(tt.b, s);

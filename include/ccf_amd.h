@@ -151,6 +151,12 @@ void ccf_default_params(ccf_params* p);
 int ccf_set_params(ccf_ctx* ctx, const ccf_params* p);
 int ccf_get_params(const ccf_ctx* ctx, ccf_params* p);
 
+/* How long, in units of 10 ns, the workgroups that solve a small field's phi
+   chains together (FP64) wait for each other before one workgroup per chain
+   does their work instead, with the same results: 0.2 s unless set, which a
+   device with room for all of them does not come near; negative: the default. */
+int ccf_set_team_wait(ccf_ctx* ctx, long long ticks);
+
 /* bool CCF::run(int verbose) (ccf.cuh:1265-1280) */
 int ccf_run(ccf_ctx* ctx, int verbose);
 

@@ -1,8 +1,10 @@
-"""The FP64 continuation of small fields in one launch (k_chains) and the FP64
-tail launch (k_tail64): whole runs against the oracle, within 1e-9 relative
-at every point, at the sizes where they change over (480 roots), with the
-smallest fields, one and several branches, points outside the tree, and
-sweep caps that end a step before, at and after its tail."""
+"""The FP64 continuation of small fields in one launch (k_chains, teams of
+workgroups) and the FP64 tail launch (k_tail64): whole runs against the
+oracle, within 1e-9 relative at every point, at the sizes where they change
+over (a row and its lists in LDS; a member's terms), with the smallest
+fields, one and several branches, points outside the tree, and sweep caps
+that end a step before, at and after its tail."""
+import ctypes
 import os
 
 import numpy as np
@@ -29,10 +31,13 @@ def _stars(workdir, n, **kw):
     (33, {}, dict(num_phi=24, num_branches=2)),
     (128, {}, dict(num_phi=20, num_branches=1, direct=1)),
     (64, dict(rectangular=1), dict(num_phi=24, num_branches=2)),
-    (240, {}, dict(num_phi=16, num_branches=1)),       # the last rows of k_chains
-    (241, {}, dict(num_phi=16, num_branches=1)),       # the first of the sweeps with k_tail64
+    (241, {}, dict(num_phi=16, num_branches=1)),
     (300, dict(rectangular=1), dict(num_phi=36, num_branches=3)),
     (700, {}, dict(num_phi=16, num_branches=2)),
+    (1144, {}, dict(num_phi=4, num_branches=1)),       # the largest row that fits
+    (1145, {}, dict(num_phi=4, num_branches=1)),       # the sweeps with k_tail64
+    (400, {}, dict(num_phi=72, num_branches=18)),      # teams of one, 960 000 terms: the sweeps
+    (300, {}, dict(num_phi=64, num_branches=16)),      # teams of two, 270 000 terms a member
 ])
 @pytest.mark.parametrize("predictor", [0, 3])
 def test_fp64_continuation_matches_oracle(workdir, n, field, grid, predictor):
@@ -54,7 +59,25 @@ def test_fp64_continuation_matches_oracle(workdir, n, field, grid, predictor):
         assert worst < 1e-6 and nbad <= max(5, 1e-3 * R * (np_ + nb)), (worst, nbad)
     assert info["points_converged"] == info["points_total"] == R * (np_ + nb)
     # one launch for the chains; else a tail for each step and side
-    assert info["tail_launches"] == (1 if R <= 480 else 2 * (np_ // (2 * nb)))
+    assert info["tail_launches"] == (2 * (np_ // (2 * nb)) if (n, nb) in ((1145, 1), (400, 18)) else 1)
+
+
+@pytest.mark.parametrize("n,nb", [(1, 1), (17, 1), (100, 1), (137, 2), (240, 3), (60, 40), (1000, 1)])
+@pytest.mark.parametrize("predictor", [0, 2])
+def test_chains_without_teams_are_the_same_bits(workdir, n, nb, predictor):
+    """members that give up at once: one workgroup per chain does their work,
+    and the counts are those of one solve"""
+    kw = dict(starfile=_stars(workdir, n), outfile_prefix="./", kappa_tot=0.45, shear=0.3, num_phi=8 * nb, num_branches=nb,
+              predictor=predictor)
+    with ccf_amd.Context(**kw) as c, ccf_amd.Context(**kw) as d:
+        assert c.run(0), c.last_error()
+        assert d.lib.ccf_set_team_wait(ctypes.c_void_p(d.ptr), ctypes.c_longlong(0)) == 0
+        assert d.run(0) and d.run(0), d.last_error()
+        assert np.array_equal(c.array(ccf_amd.ARRAY_CCS), d.array(ccf_amd.ARRAY_CCS))
+        assert np.array_equal(c.array(ccf_amd.ARRAY_CAUSTICS), d.array(ccf_amd.ARRAY_CAUSTICS))
+        a, b = c.info(), d.info()
+    for k in ("points_converged", "points_total", "updates_full", "updates_early", "tail_sweeps", "flops_tail"):
+        assert a[k] == b[k], k
 
 
 @pytest.mark.parametrize("n", [100, 300])
