@@ -453,6 +453,7 @@ __device__ __forceinline__ void direct_term(cd z, double2 u, double& ax, double&
 // b of nb takes the row's outliers b, b + nb, ..., OUT_GROUP at a time, so
 // that each pass over the row's roots serves a group of them.
 constexpr int OUT_GROUP = 8;
+constexpr int OUT_BATCH = 8;
 constexpr int RSUM_OUT_BLOCKS = 16;
 
 template <int P>
@@ -478,12 +479,22 @@ __device__ void rsum_outliers(const RootView& V, const double2* __restrict__ zr,
 			z[k] = cd(v.x, v.y);
 			ax[k] = ay[k] = 0;
 		}
-		for (int q = threadIdx.x; q < R; q += NT)
+		// (OUT_BATCH loads in flight: a row's few outliers are otherwise the
+		// longest part of the launch, one load's latency after the other)
+		for (int q0 = threadIdx.x; q0 < R; q0 += OUT_BATCH * NT)
 		{
-			const double2 u = zr[q];
+			double2 u[OUT_BATCH];
 #pragma unroll
-			for (int k = 0; k < OUT_GROUP; k++)
-				if (sl[k] >= 0 && q != j[k]) direct_term<P>(z[k], u, ax[k], ay[k]);
+			for (int i = 0; i < OUT_BATCH; i++) u[i] = zr[min(q0 + i * NT, R - 1)];
+#pragma unroll
+			for (int i = 0; i < OUT_BATCH; i++)
+			{
+				const int q = q0 + i * NT;
+				if (q < R)
+#pragma unroll
+					for (int k = 0; k < OUT_GROUP; k++)
+						if (sl[k] >= 0 && q != j[k]) direct_term<P>(z[k], u[i], ax[k], ay[k]);
+			}
 		}
 #pragma unroll
 		for (int k = 0; k < OUT_GROUP; k++)
