@@ -76,7 +76,6 @@ namespace
 {
 
 constexpr int BLOCK = 256;
-constexpr int CHUNK64 = 1024;         // FP64 complex values per LDS chunk (16 KiB)
 constexpr int CHUNK32 = 2048;         // FP32 complex values per LDS chunk (16 KiB)
 constexpr int ROOTS_PER_THREAD = 2;   // of k_sums32 and k_sums64 unless given or tuned
 constexpr int MAX_SLICES = 64;
@@ -715,85 +714,61 @@ __device__ inline int row_of_tile(const int* __restrict__ tile_off, int nrows, i
 // which index takes which root (the sweeps before they settle are chaotic;
 // a continuation step starts next to its roots and is not), so the order
 // and form of the terms stay as they are here and a field keeps its indices.
-template <int RPT>
-__global__ __launch_bounds__(BLOCK) void k_sums64(const double2* __restrict__ spos, int Np, const double2* __restrict__ roots,
+//
+// A wave takes 64 listed roots of a tile and a slice of the terms by itself,
+// every lane the same source (scalar loads), no LDS and no barrier: the
+// plan's tiles of up to 512 roots and its slices fix each root's partial
+// sums, not who forms them. Bound by the FP64 VALU when the device is full
+// and by one wave's chain of terms in a small field, where a workgroup with
+// two roots a thread took longer: 274 roots x 411 terms 21 -> 18 us, the 25
+// launches of a 10 000-star field 125 -> 114 on average.
+__global__ __launch_bounds__(BLOCK, 8) void k_sums64(const double2* __restrict__ spos, int Np, const double2* __restrict__ roots,
 	RowMap M, SweepView V, int nrows)
 {
-	__shared__ double2 buf[CHUNK64];
 	const int tiles = V.plan[0], S = V.plan[1];
-	const long long items = (long long)tiles * S;
-	const int R = M.R, T = BLOCK * RPT;
+	const int R = M.R, T = V.tile, subs = T / 64;
+	const long long items = (long long)tiles * S * subs;
+	const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 	const long long Lt = (long long)Np + R;
-	for (long long item = blockIdx.x; item < items; item += gridDim.x)
+	for (long long w = (long long)blockIdx.x * (BLOCK / 64) + wv; w < items; w += (long long)gridDim.x * (BLOCK / 64))
 	{
+		const long long item = w / subs;
+		const int sub = (int)(w % subs);
 		const int g = (int)(item / S), s = (int)(item % S);
 		const int r = row_of_tile(V.tile_off, nrows, g);
-		const int t = g - V.tile_off[r];
-		const int nfr = V.fcnt[r];
+		const int i0 = (g - V.tile_off[r]) * T + sub * 64, nt = V.fcnt[r] - i0;
+		if (nt <= 0) continue;
 		int row;
 		double phi;
 		M.get(r, row, phi);
 		const double2* __restrict__ xrow = roots + (size_t)row * R;
-		double zx[RPT], zy[RPT], ax[RPT], ay[RPT], bx[RPT], by[RPT];
-#pragma unroll
-		for (int k = 0; k < RPT; k++)
-		{
-			const int i = t * T + k * BLOCK + threadIdx.x;
-			const int a = V.fl[(size_t)r * R + (i < nfr ? i : t * T)];
-			const double2 v = xrow[a];
-			zx[k] = v.x;
-			zy[k] = v.y;
-			ax[k] = ay[k] = bx[k] = by[k] = 0;
-		}
+		const double2 z = xrow[V.fl[(size_t)r * R + i0 + (lane < nt ? lane : 0)]];
+		double ax = 0, ay = 0, bx = 0, by = 0;
 		const long long lo = s * Lt / S, hi = (s + 1) * Lt / S;
 		// star terms (ccf_functions.cuh:218-227)
-		const int s1 = (int)min(hi, (long long)Np);
-		for (int c0 = (int)lo; c0 < s1; c0 += CHUNK64)
-		{
-			const int m = min(CHUNK64, s1 - c0);
-			for (int q = threadIdx.x; q < m; q += BLOCK) buf[q] = spos[c0 + q];
-			__syncthreads();
+		const int s0 = (int)lo, s1 = (int)min(hi, (long long)Np);
 #pragma unroll 4
-			for (int q = 0; q < m; q++)
-			{
-				const double2 w = buf[q];
-#pragma unroll
-				for (int k = 0; k < RPT; k++)
-				{
-					const double dx = zx[k] - w.x, dy = zy[k] - w.y;
-					const double iv = rcp64(fma(dx, dx, dy * dy));
-					ax[k] = fma(dx, iv, ax[k]);
-					ay[k] = fma(dy, iv, ay[k]);
-				}
-			}
-			__syncthreads();
+		for (int q = s0; q < s1; q++)
+		{
+			const double2 u = spos[q];
+			const double dx = z.x - u.x, dy = z.y - u.y;
+			const double iv = rcp64(fma(dx, dx, dy * dy));
+			ax = fma(dx, iv, ax);
+			ay = fma(dy, iv, ay);
 		}
 		// root terms (ccf_functions.cuh:232-239); the own root gives dx = dy = 0
 		// exactly and the floor on |d|^2 turns its term into 0
 		const int r0 = (int)(max(lo, (long long)Np) - Np), r1 = (int)(hi - Np);
-		for (int c0 = r0; c0 < r1; c0 += CHUNK64)
-		{
-			const int m = min(CHUNK64, r1 - c0);
-			for (int q = threadIdx.x; q < m; q += BLOCK) buf[q] = xrow[c0 + q];
-			__syncthreads();
 #pragma unroll 4
-			for (int q = 0; q < m; q++)
-			{
-				const double2 w = buf[q];
-#pragma unroll
-				for (int k = 0; k < RPT; k++)
-				{
-					const double dx = zx[k] - w.x, dy = zy[k] - w.y;
-					const double iv = rcp64(fmax(fma(dx, dx, dy * dy), 1e-300));
-					bx[k] = fma(dx, iv, bx[k]);
-					by[k] = fma(dy, iv, by[k]);
-				}
-			}
-			__syncthreads();
+		for (int q = r0; q < r1; q++)
+		{
+			const double2 u = xrow[q];
+			const double dx = z.x - u.x, dy = z.y - u.y;
+			const double iv = rcp64(fmax(fma(dx, dx, dy * dy), 1e-300));
+			bx = fma(dx, iv, bx);
+			by = fma(dy, iv, by);
 		}
-#pragma unroll
-		for (int k = 0; k < RPT; k++)
-			V.part[(size_t)item * T + k * BLOCK + threadIdx.x] = make_double2(2 * ax[k] - bx[k], -(2 * ay[k] - by[k]));
+		V.part[(size_t)item * T + sub * 64 + lane] = make_double2(2 * ax - bx, -(2 * ay - by));
 	}
 }
 
@@ -2099,7 +2074,7 @@ SumsLaunch sums_launch(ccf_ctx* ctx, SumsForm form)
 	const void* fn;
 	if (form == SUMS_64_QUAD) fn = (const void*)k_sums64_quad;
 	else if (form == SUMS_32) fn = l.rpt == 1 ? (const void*)k_sums32<1> : (l.rpt == 4 ? (const void*)k_sums32<4> : (const void*)k_sums32<2>);
-	else fn = l.rpt == 1 ? (const void*)k_sums64<1> : (l.rpt == 4 ? (const void*)k_sums64<4> : (const void*)k_sums64<2>);
+	else fn = (const void*)k_sums64;
 	if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, BLOCK, 0) != hipSuccess || per_cu < 1) per_cu = 2;
 	const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
 	l.grid = cus * per_cu;
@@ -2113,7 +2088,8 @@ SumsLaunch sums_launch(ccf_ctx* ctx, SumsForm form)
 	{
 		l.tile = BLOCK * l.rpt;
 		l.min_slice = MIN_SLICE;
-		l.target = 4 * l.grid;
+		// (SUMS_64: a constant of the form, for its slices decide the last bits)
+		l.target = form == SUMS_64 ? 4 * cus * (l.rpt == 1 ? 8 : 4) : 4 * l.grid;
 	}
 	return l;
 }
@@ -2308,9 +2284,7 @@ bool run_sweeps_groups(ccf_ctx* ctx, SweepGroup* gs, int G, double2* roots, int 
 			}
 			else
 			{
-				if (sl.rpt == 1) k_sums64<1><<<sl.grid, BLOCK, 0, s>>>(ctx->spos, Np, roots, M, V, nrows);
-				else if (sl.rpt == 4) k_sums64<4><<<sl.grid, BLOCK, 0, s>>>(ctx->spos, Np, roots, M, V, nrows);
-				else k_sums64<2><<<sl.grid, BLOCK, 0, s>>>(ctx->spos, Np, roots, M, V, nrows);
+				k_sums64<<<sl.grid, BLOCK, 0, s>>>(ctx->spos, Np, roots, M, V, nrows);
 			}
 			if (ctx->P.timing && tm.a && tm.b)
 			{
