@@ -1588,7 +1588,9 @@ __global__ __launch_bounds__(TAIL_BLOCK) void k_tail(LensView L, double2* __rest
 // sums and moves them as chain_row does, and after a sweep every member
 // publishes its roots' positions and takes in the others'. 1024 threads,
 // though they spill a few bytes at 128 VGPRs: four waves a SIMD keep the
-// FP64 pipe busier than two do.
+// FP64 pipe busier than two do. Members of few roots (TEAM_SMALL) have 512,
+// whose barriers are shorter: 100 stars 1.56 -> 1.44 ms, 300 stars 2.16 ->
+// 2.06; 1000 stars 4.45 -> 4.67, so not there. The bits are the same.
 //
 // The members meet in memory once a sweep: positions and arrivals are
 // agent-scope atomic accesses, which are coherent between the XCDs' L2s, and
@@ -1601,6 +1603,7 @@ __global__ __launch_bounds__(TAIL_BLOCK) void k_tail(LensView L, double2* __rest
 // follows (RETRY, one workgroup per row, which otherwise only hands the
 // counts on) does the members' work in turn, with the same arithmetic.
 constexpr int CHAIN_BLOCK = 1024;
+constexpr int TEAM_SMALL = 24;
 constexpr int TEAM_WGS = 64;
 constexpr int TEAM_MAX = 32;
 constexpr int TEAM_ROOTS = 8;                     // fewest roots of a member
@@ -1678,11 +1681,12 @@ __device__ inline int team_meet(const ChainTeams& T, TeamSlot& slot, unsigned ep
 
 // a member's roots lo .. hi published and the others' taken in; false once a
 // member has given up. Every thread of the workgroup calls it.
+template <int BS>
 __device__ __forceinline__ bool team_exchange(const ChainTeams& T, int r, unsigned& epoch, int member, int R, int lo, int hi, double2* zc,
 	int& active, int* s_meet)
 {
 	unsigned long long* const p = reinterpret_cast<unsigned long long*>(T.pos + (size_t)(2 * r + (epoch & 1)) * R);
-	for (int k = 2 * lo + threadIdx.x; k < 2 * hi; k += CHAIN_BLOCK)
+	for (int k = 2 * lo + threadIdx.x; k < 2 * hi; k += BS)
 		__hip_atomic_store(p + k, reinterpret_cast<const unsigned long long*>(zc)[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 	asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 	__syncthreads();
@@ -1691,7 +1695,7 @@ __device__ __forceinline__ bool team_exchange(const ChainTeams& T, int r, unsign
 	active = *s_meet;
 	if (active < 0) return false;
 	const int other = 2 * (R - (hi - lo));
-	for (int q = threadIdx.x; q < other; q += CHAIN_BLOCK)
+	for (int q = threadIdx.x; q < other; q += BS)
 	{
 		const int k = q < 2 * lo ? q : q + 2 * (hi - lo);
 		reinterpret_cast<unsigned long long*>(zc)[k] = __hip_atomic_load(p + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1701,8 +1705,8 @@ __device__ __forceinline__ bool team_exchange(const ChainTeams& T, int r, unsign
 	return true;
 }
 
-template <bool RETRY>
-__global__ __launch_bounds__(CHAIN_BLOCK) void k_chains(LensView L, double2* __restrict__ roots, const double2* __restrict__ cs, int R,
+template <bool RETRY, int BS>
+__global__ __launch_bounds__(BS) void k_chains(LensView L, double2* __restrict__ roots, const double2* __restrict__ cs, int R,
 	int N, int np, int nb, int steps, int cap, int predictor, const int* __restrict__ order, ChainTeams T,
 	unsigned long long* __restrict__ stats)
 {
@@ -1730,8 +1734,8 @@ __global__ __launch_bounds__(CHAIN_BLOCK) void k_chains(LensView L, double2* __r
 	const int center = np / (2 * nb) + c * (np / nb + 1);
 	int cnt[CHAIN_COUNTS] = {0, 0, 0, 0, 0};
 	unsigned epoch = 0;
-	for (int s = threadIdx.x; s < N; s += CHAIN_BLOCK) st[s] = L.spos[s];
-	for (int p = threadIdx.x; p < R; p += CHAIN_BLOCK) zc[p] = roots[(size_t)center * R + order[p]];
+	for (int s = threadIdx.x; s < N; s += BS) st[s] = L.spos[s];
+	for (int p = threadIdx.x; p < R; p += BS) zc[p] = roots[(size_t)center * R + order[p]];
 	if (threadIdx.x < TEAM_MAX) s_nf[threadIdx.x] = s_left[threadIdx.x] = 0;
 	for (int j = 1; j <= steps; j++)
 	{
@@ -1740,13 +1744,13 @@ __global__ __launch_bounds__(CHAIN_BLOCK) void k_chains(LensView L, double2* __r
 		if (q > 0)
 		{
 			// (a thread reads what it wrote in the earlier steps)
-			for (int p = lo + threadIdx.x; p < hi; p += CHAIN_BLOCK)
+			for (int p = lo + threadIdx.x; p < hi; p += BS)
 				zc[p] = predict_root(roots + (size_t)(row - sgn) * R + order[p], (long long)sgn * R, q);
 			__syncthreads(); // (a position is published by another thread)
 			int none = 0;
-			if (!RETRY && K > 1 && !team_exchange(T, r, epoch, m0, R, lo, hi, zc, none, &s_meet)) return;
+			if (!RETRY && K > 1 && !team_exchange<BS>(T, r, epoch, m0, R, lo, hi, zc, none, &s_meet)) return;
 		}
-		for (int p = lo + threadIdx.x; p < hi; p += CHAIN_BLOCK) cur[p - lo] = p;
+		for (int p = lo + threadIdx.x; p < hi; p += BS) cur[p - lo] = p;
 		__syncthreads();
 		int n[RETRY ? TEAM_MAX : 1];
 		for (int m = m0; m < m1; m++) n[m - m0] = first(m + 1) - first(m);
@@ -1758,11 +1762,11 @@ __global__ __launch_bounds__(CHAIN_BLOCK) void k_chains(LensView L, double2* __r
 				const int o = first(m) - lo;
 				return ChainLists{cur + o, nxt + o, fl + o, f0 + o, f1 + o};
 			};
-			for (int m = m0; m < m1; m++) chain_evaluate<CHAIN_BLOCK>(L, e.x, e.y, zc, lists(m).la, n[m - m0], lists(m), &s_nf[m - m0], cnt);
+			for (int m = m0; m < m1; m++) chain_evaluate<BS>(L, e.x, e.y, zc, lists(m).la, n[m - m0], lists(m), &s_nf[m - m0], cnt);
 			__syncthreads();
-			for (int m = m0; m < m1; m++) chain_sums<CHAIN_BLOCK>(R, N, 0, zc, st, lists(m), s_nf[m - m0]);
+			for (int m = m0; m < m1; m++) chain_sums<BS>(R, N, 0, zc, st, lists(m), s_nf[m - m0]);
 			__syncthreads();
-			for (int m = m0; m < m1; m++) chain_update<CHAIN_BLOCK>(L, zc, lists(m), s_nf[m - m0], lists(m).lb, &s_left[m - m0], cnt);
+			for (int m = m0; m < m1; m++) chain_update<BS>(L, zc, lists(m), s_nf[m - m0], lists(m).lb, &s_left[m - m0], cnt);
 			__syncthreads();
 			active = 0;
 			for (int m = m0; m < m1; m++) active += n[m - m0] = s_left[m - m0];
@@ -1770,18 +1774,18 @@ __global__ __launch_bounds__(CHAIN_BLOCK) void k_chains(LensView L, double2* __r
 			if (threadIdx.x < TEAM_MAX) s_nf[threadIdx.x] = s_left[threadIdx.x] = 0;
 			if (!RETRY && K > 1)
 			{
-				if (!team_exchange(T, r, epoch, m0, R, lo, hi, zc, active, &s_meet)) return;
+				if (!team_exchange<BS>(T, r, epoch, m0, R, lo, hi, zc, active, &s_meet)) return;
 			}
 			else __syncthreads();
 			int* const t = cur;
 			cur = nxt;
 			nxt = t;
 		}
-		for (int p = lo + threadIdx.x; p < hi; p += CHAIN_BLOCK) roots[(size_t)row * R + order[p]] = zc[p];
+		for (int p = lo + threadIdx.x; p < hi; p += BS) roots[(size_t)row * R + order[p]] = zc[p];
 	}
 	unsigned long long v[CHAIN_COUNTS];
 	for (int t = 0; t < CHAIN_COUNTS; t++) v[t] = (unsigned long long)cnt[t];
-	if (RETRY) block_stats<CHAIN_COUNTS, CHAIN_BLOCK>(stats, which, v);
+	if (RETRY) block_stats<CHAIN_COUNTS, BS>(stats, which, v);
 	else
 		for (int t = 0; t < CHAIN_COUNTS; t++)
 		{
@@ -2965,9 +2969,11 @@ bool find_ccs_dev(ccf_ctx* ctx, int verbose)
 		ChainTeams T;
 		if (!chain_teams(ctx, T, K)) return false;
 		k_clear_teams<<<1, 64, 0, s>>>(T, 2 * nb);
-		k_chains<false><<<2 * nb * K, CHAIN_BLOCK, chain_lds(R, N, (R + K - 1) / K), s>>>(L, ctx->ccs_init, ctx->phase, R, N, np, nb, steps,
-			cap, ctx->P.predictor, ctx->dorder, T, ctx->counters);
-		k_chains<true><<<2 * nb, CHAIN_BLOCK, chain_lds(R, N, R), s>>>(L, ctx->ccs_init, ctx->phase, R, N, np, nb, steps, cap,
+		const bool small = R <= TEAM_SMALL * K;
+		(small ? k_chains<false, CHAIN_BLOCK / 2> : k_chains<false, CHAIN_BLOCK>)<<<2 * nb * K, small ? CHAIN_BLOCK / 2 : CHAIN_BLOCK,
+			chain_lds(R, N, (R + K - 1) / K), s>>>(L, ctx->ccs_init, ctx->phase, R, N, np, nb, steps, cap, ctx->P.predictor, ctx->dorder,
+			T, ctx->counters);
+		k_chains<true, CHAIN_BLOCK><<<2 * nb, CHAIN_BLOCK, chain_lds(R, N, R), s>>>(L, ctx->ccs_init, ctx->phase, R, N, np, nb, steps, cap,
 			ctx->P.predictor, ctx->dorder, T, ctx->counters);
 		if (ctx->P.timing && tt.a && tt.b)
 		{
