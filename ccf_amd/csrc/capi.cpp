@@ -674,13 +674,17 @@ double ms_seconds(double s) { return std::floor(s * 1000.0) / 1000.0; } // stopw
 // them started: above about 256 KiB the runtime pins the caller's pages for
 // a copy (320 KB: 150 -> 40 us, 3 MB: 740 -> 290).
 //
-// The pinned slots (two of COPY_CHUNK for each of COPY_THREADS threads: 32
+// The pinned slots (two of COPY_CHUNK for each of COPY_THREADS threads: 64
 // MiB at most) and their events are shared by the process's contexts: a
 // thread's are made by the first copy that takes as many threads, used by
 // one copy at a time (a copy that finds them taken goes through hipMemcpy),
 // and given back when the last context is destroyed.
 constexpr int COPY_THREADS = 8;
-constexpr size_t COPY_CHUNK = size_t(2) << 20;
+constexpr size_t COPY_CHUNK = size_t(4) << 20;
+// Arrays below this go in half chunks, which the threads start on sooner
+// (64 MB: 3.6 ms against 4.1); above, the gaps between the device's copies
+// count (646 MB: 14.3 ms against 16.2)
+constexpr size_t COPY_LARGE = size_t(128) << 20;
 constexpr size_t COPY_PART = size_t(512) << 10; // least bytes of a thread's part (a thread's start is about 20 us)
 constexpr size_t COPY_MIN = size_t(256) << 10;  // smaller arrays: hipMemcpy
 
@@ -745,20 +749,21 @@ int copy_threads()
 }
 
 // the part [lo, hi) of src to dst through slots a and b, filled on stream s
-hipError_t copy_part(char* dst, const char* src, size_t lo, size_t hi, char* const (&slot)[2], hipEvent_t const (&event)[2], hipStream_t s)
+hipError_t copy_part(char* dst, const char* src, size_t lo, size_t hi, size_t chunk, char* const (&slot)[2], hipEvent_t const (&event)[2],
+	hipStream_t s)
 {
 	auto fill = [&](size_t at, int k) {
-		const hipError_t e = hipMemcpyAsync(slot[k], src + at, std::min(COPY_CHUNK, hi - at), hipMemcpyDeviceToHost, s);
+		const hipError_t e = hipMemcpyAsync(slot[k], src + at, std::min(chunk, hi - at), hipMemcpyDeviceToHost, s);
 		return e != hipSuccess ? e : hipEventRecord(event[k], s);
 	};
 	hipError_t e = lo < hi ? fill(lo, 0) : hipSuccess;
-	for (size_t at = lo, n = 0; e == hipSuccess && at < hi; at += COPY_CHUNK, n++)
+	for (size_t at = lo, n = 0; e == hipSuccess && at < hi; at += chunk, n++)
 	{
 		const int k = (int)(n & 1);
 		hipError_t next = hipSuccess;
-		if (at + COPY_CHUNK < hi) next = fill(at + COPY_CHUNK, k ^ 1);
+		if (at + chunk < hi) next = fill(at + chunk, k ^ 1);
 		e = hipEventSynchronize(event[k]);
-		if (e == hipSuccess) std::memcpy(dst + at, slot[k], std::min(COPY_CHUNK, hi - at));
+		if (e == hipSuccess) std::memcpy(dst + at, slot[k], std::min(chunk, hi - at));
 		if (e == hipSuccess) e = next;
 	}
 	return e;
@@ -808,7 +813,7 @@ hipError_t ccf::copy_out(ccf_ctx* c, void* dst, const void* src, size_t bytes)
 		const size_t lo = bytes / T * t, hi = t + 1 == T ? bytes : bytes / T * (t + 1);
 		char* const slot[2] = {cs.mem[t], cs.mem[t] + COPY_CHUNK};
 		hipEvent_t const event[2] = {cs.event[2 * t], cs.event[2 * t + 1]};
-		const hipError_t e = copy_part((char*)dst, (const char*)src, lo, hi, slot, event, c->stream);
+		const hipError_t e = copy_part((char*)dst, (const char*)src, lo, hi, bytes >= COPY_LARGE ? COPY_CHUNK : COPY_CHUNK / 2, slot, event, c->stream);
 		if (e != hipSuccess) bad = e;
 	};
 	std::vector<std::thread> threads;

@@ -20,6 +20,7 @@ pytestmark = pytest.mark.gpu
     (64, 2048, 2),    # 2050 x 128 points: 4 198 400 B, eight parts
     (137, 2000, 4),   # 8.8 MB, odd parts
     (700, 1200, 6),   # 27 MB, more parts than threads
+    (700, 6000, 6),   # 134.5 MB: whole chunks
 ])
 def test_concurrent_copies_agree(n, num_phi, nb):
     kw = dict(num_stars=n, kappa_tot=0.4, kappa_star=0.4, shear=0.2, num_phi=num_phi, num_branches=nb, random_seed=7,
