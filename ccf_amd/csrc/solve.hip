@@ -773,7 +773,7 @@ __global__ __launch_bounds__(BLOCK, 8) void k_sums64(const double2* __restrict__
 }
 
 // K3 in FP64 of the continuation steps and of single sweeps: the same partial
-// sums with the reciprocals shared (cauchy4).
+// sums with the reciprocals shared (cauchy8).
 //
 // Bound by the FP64 VALU: 20 000 roots against 30 000 terms take 0.22 ms
 // (2.7e12 terms/s; the loop alone reaches 3.2e12), 0.33 ms in k_sums64. A

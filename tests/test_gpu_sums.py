@@ -57,3 +57,30 @@ def test_quad_sums_far_roots(workdir, n):
     roots[1], roots[2], roots[3] = 1e60, 2e60j, -3e59 + 1e59j
     print(f"# quad sums, {n} roots, three of them far off", flush=True)
     _check(sf, roots, dict(kappa_tot=0.3, shear=0.1, direct=1, num_phi=10))
+
+
+@pytest.mark.parametrize("copies", [2, 5, 6, 8])
+def test_quad_sums_coincident_roots(workdir, copies):
+    """positions that coincide add nothing to each other's sums, also where a
+    group's product of squared distances underflows"""
+    sf = make_field(workdir, "cfg1")
+    rng = np.random.default_rng(copies)
+    roots = 18 * (rng.uniform(-1, 1, 48) + 1j * rng.uniform(-1, 1, 48))
+    roots[8:8 + copies] = roots[8]
+    phi, kw = 2.1, dict(kappa_tot=0.3, shear=0.1, direct=1, num_phi=10)
+    _, _, _, _, st = io.read_stars(sf)
+    s = st[:, 0] + 1j * st[:, 1]
+    with ccf_amd.Context(starfile=sf, outfile_prefix="./", **kw) as c:
+        c.prepare()
+        g = c.aberth_sweep(roots, phi)
+        e = c.eval_points(roots, phi)
+    f0, f1 = e[:, 0] + 1j * e[:, 1], e[:, 2] + 1j * e[:, 3]
+    d = roots[:, None] - roots[None, :]
+    t = np.where(d == 0, 0, 1 / np.where(d == 0, 1, d))
+    u = 1 / (roots[:, None] - s[None, :])
+    o = roots - f0 / (f1 + f0 * (2 * u.sum(1) - t.sum(1)))
+    step = np.abs(o - roots)
+    scale = 2 * np.abs(u).sum(1) + np.abs(t).sum(1)
+    # (as in _check: roundings of the terms, and of f0 and f1)
+    tol = 64 * EPS * (np.maximum(np.abs(roots), 1) + step * step * scale) + 1e-12 * step
+    assert step.max() > 0 and np.all(np.abs(g - o) <= tol), (np.abs(g - o) / tol).max()
