@@ -6,6 +6,7 @@ fields, one and several branches, points outside the tree, and sweep caps
 that end a step before, at and after its tail."""
 import ctypes
 import os
+import threading
 
 import numpy as np
 import pytest
@@ -78,6 +79,35 @@ def test_chains_without_teams_are_the_same_bits(workdir, n, nb, predictor):
         a, b = c.info(), d.info()
     for k in ("points_converged", "points_total", "updates_full", "updates_early", "tail_sweeps", "flops_tail"):
         assert a[k] == b[k], k
+
+
+def test_teams_of_several_contexts_at_once(workdir):
+    """chains of contexts that run side by side from their own threads (teams
+    of 32, 30 and 64 workgroups a launch) give the bits of each alone"""
+    fields = [(100, 1), (400, 1), (137, 3), (240, 1)]
+    kws = [dict(starfile=_stars(workdir, n), outfile_prefix="./", kappa_tot=0.45, shear=0.3, num_phi=40 * nb, num_branches=nb)
+           for n, nb in fields]
+    alone = []
+    for kw in kws:
+        with ccf_amd.Context(**kw) as c:
+            assert c.run(0), c.last_error()
+            alone.append(c.array(ccf_amd.ARRAY_CCS))
+    got = [[] for _ in kws]
+    start = threading.Barrier(len(kws))
+
+    def work(k):
+        with ccf_amd.Context(**kws[k]) as c:
+            start.wait()
+            for _ in range(3):
+                got[k].append(c.array(ccf_amd.ARRAY_CCS) if c.run(0) else None)
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(len(kws))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for k, a in enumerate(alone):
+        assert len(got[k]) == 3 and all(np.array_equal(a, g) for g in got[k]), fields[k]
 
 
 @pytest.mark.parametrize("n", [100, 300])
