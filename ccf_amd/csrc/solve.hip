@@ -205,8 +205,8 @@ __device__ inline int block_append(int* counter, bool pred)
 
 // phi-row index and angle of solved row r of a phase (ccf_functions.cuh:338-374).
 // rows_per_branch 1: the branch centres (j = 0); 2: both sides of step j;
-// 0: row r of a caller-supplied array, all at angle phi_fixed; -1: row r of
-// the output, whose phase comes from cs.
+// 0: row r of a caller-supplied array, all at angle phi_fixed; -1: row
+// c0 + r of the output, whose phase comes from cs.
 // angle of phi step j on side sgn of branch c (ccf_functions.cuh:338-374)
 __device__ inline double branch_phi(int c, int sgn, int j, int np, int nb)
 {
@@ -220,7 +220,7 @@ struct RowMap
 	int R, np, nb, j, rows_per_branch;
 	double phi_fixed;
 	const double2* cs = nullptr; // (cos phi, sin phi) of every phi row, or null
-	int c0 = 0;                  // the first branch of the rows (a group of branches solved on its own stream)
+	int c0 = 0;                  // the first branch of the rows (a group of branches solved on its own stream), or the first row
 	int side = 0;                // rows_per_branch 1: step j's rows of this side (-1 or 1), or the centres (0)
 	__device__ inline int sgn(int r) const
 	{
@@ -230,7 +230,7 @@ struct RowMap
 	{
 		if (rows_per_branch <= 0)
 		{
-			row = r;
+			row = c0 + r;
 			phi = phi_fixed;
 			return;
 		}
@@ -1644,6 +1644,10 @@ inline int chain_team(int R, int rows) { return std::max(1, std::min(std::min(TE
 constexpr long long TEAM_TERMS = 600 * 1000;
 constexpr size_t CHAIN_LDS = 152 * 1024;
 
+// rows of a launch of the error pass after the chains (a launch holds 65 536
+// in y; a run has num_phi + num_branches)
+constexpr int ERROR_ROWS = 32768;
+
 inline bool chain_fits(int R, int N, int rows)
 {
 	return chain_lds(R, N, R) <= CHAIN_LDS && (long long)R * (R + N) / chain_team(R, rows) <= TEAM_TERMS;
@@ -2955,7 +2959,7 @@ bool find_ccs_dev(ccf_ctx* ctx, int verbose)
 		if (sides) return j == 0 && g > 0 ? 0 : nb; // the centres with the first side
 		return (j == 0 ? 1 : 2) * (gb[g + 1] - gb[g]);
 	};
-	// the chains, then one error pass over all rows
+	// the chains, then the error pass over all rows
 	if (chained)
 	{
 		ccf::Timer tt;
@@ -2980,9 +2984,9 @@ bool find_ccs_dev(ccf_ctx* ctx, int verbose)
 			(void)hipEventRecord(tt.b, s);
 			ctx->tail_timers.push_back(tt);
 		}
-		if (!CCF_LAUNCH(ctx, "find_critical_curve_roots_kernel") ||
-			!errors(RowMap{R, np, nb, 0, -1, 0.0, ctx->phase, 0}, np + nb, s, ctx->err_event))
-			return false;
+		if (!CCF_LAUNCH(ctx, "find_critical_curve_roots_kernel")) return false;
+		for (int r0 = 0; r0 < np + nb; r0 += ERROR_ROWS)
+			if (!errors(RowMap{R, np, nb, 0, -1, 0.0, ctx->phase, r0}, std::min(ERROR_ROWS, np + nb - r0), s, ctx->err_event)) return false;
 		ctx->info.tail_launches++;
 		if (verbose >= 1)
 		{

@@ -123,3 +123,16 @@ def test_fp64_sweep_caps(workdir, n, cap):
     assert np.all(np.isfinite(z)) and np.all(z != 0)
     assert info["tail_sweeps"] <= 32 * 2 * cap
     assert info["updates_full"] + info["updates_early"] <= 2 * n * (60 + 64 * cap)
+
+
+def test_error_pass_in_blocks_of_rows(workdir):
+    """a phi grid of more rows than a launch of the error pass takes: the
+    caustics it forms are the lens map of every row's roots"""
+    sf = _stars(workdir, 17)
+    with ccf_amd.Context(starfile=sf, outfile_prefix="./", kappa_tot=0.45, shear=0.3, num_phi=32780, num_branches=1) as c:
+        assert c.run(0), c.last_error()
+        z, w, info = c.array(ccf_amd.ARRAY_CCS).ravel(), c.array(ccf_amd.ARRAY_CAUSTICS).ravel(), c.info()
+        e = c.eval_points(z, 0.0)
+    assert info["points_converged"] == info["points_total"] == z.size
+    g = e[:, 4] + 1j * e[:, 5]
+    assert (np.abs(w - g) / np.maximum(np.abs(g), 1.0)).max() < 1e-11

@@ -1,0 +1,47 @@
+"""What the host code asks of the device, on the CPU: a stand-in for the HIP
+runtime (hip_stub.cpp) takes its place in a process of its own, runs no
+kernel and writes down the launches, copies and synchronisations, which the
+tests read back."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+FIELD = "kappa_tot=0.4, kappa_star=0.4, shear=0.2, direct=1, random_seed=3, outfile_prefix='./'"
+
+
+@pytest.fixture(scope="module")
+def stub(tmp_path_factory):
+    path = str(tmp_path_factory.mktemp("stub") / "libhip_stub.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    "-o", path, os.path.join(HERE, "hip_stub.cpp")], check=True)
+    return path
+
+
+def _log(stub, tmp_path, code):
+    """the stand-in's lines for a program (Context and Batch of ccf_amd; `stub` the stand-in)"""
+    log = str(tmp_path / "log")
+    program = (f"import ctypes, sys\nstub = ctypes.CDLL({stub!r}, mode=ctypes.RTLD_GLOBAL)\nsys.path.insert(0, {ROOT!r})\n"
+               f"import numpy as np\nimport ccf_amd\nstub.stub_log({log.encode()!r})\n" + code)
+    r = subprocess.run([sys.executable, "-c", program], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr[-2000:]
+    return [line.split() for line in open(log)]
+
+
+def _launches(lines, kernel):
+    """(grid x, y, z, workgroup) of a kernel's launches"""
+    return [tuple(int(v) for v in w[2:6]) for w in lines if w[0] == "launch" and kernel in w[1]]
+
+
+@pytest.mark.parametrize("num_phi,blocks", [(32766, 1), (32768, 2), (65600, 3)])
+def test_error_pass_of_a_fine_phi_grid_fits_a_launch(stub, tmp_path, num_phi, blocks):
+    """a launch holds 65 536 workgroups in y; the rows of a small field's run are num_phi + num_branches"""
+    lines = _log(stub, tmp_path, f"c = ccf_amd.Context(num_stars=20, num_phi={num_phi}, num_branches=1, {FIELD})\nassert c.run(0)\n")
+    assert _launches(lines, "k_chains")
+    passes = _launches(lines, "k_errors")
+    assert len(passes) == blocks and sum(g[1] for g in passes) == num_phi + 1
+    assert all(int(v) <= 65536 for w in lines if w[0] == "launch" for v in w[3:5])
