@@ -1605,7 +1605,13 @@ bool batch_solve(ccf_batch* b, int verbose)
 	// the device works, and recording them would cost a rebuilt batch more)
 	if (d.nrows > 0)
 	{
-		if (!enqueue_solve(b, s)) return false;
+		if (!enqueue_solve(b, s))
+		{
+			// what was queued before the failure may be on streams that were
+			// not joined yet, and its buffers go back to the pool
+			m->sync_streams();
+			return false;
+		}
 	}
 	else if (!b->graph_exec)
 	{

@@ -127,14 +127,19 @@ void ccf_ctx::dfree(void* p)
 	pool.emplace(it->second, p);
 }
 
-void ccf_ctx::pool_release()
+void ccf_ctx::sync_streams()
 {
-	if (pool.empty()) return;
-	// work queued on the streams may still use a pooled buffer
 	if (stream) (void)hipStreamSynchronize(stream);
 	if (err_stream) (void)hipStreamSynchronize(err_stream);
 	for (hipStream_t g : group_streams)
 		if (g) (void)hipStreamSynchronize(g);
+}
+
+void ccf_ctx::pool_release()
+{
+	if (pool.empty()) return;
+	// work queued on the streams may still use a pooled buffer
+	sync_streams();
 	for (auto& [n, p] : pool)
 	{
 		owned.erase(p);

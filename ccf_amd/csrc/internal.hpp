@@ -302,6 +302,7 @@ struct ccf_ctx
 	}
 	void dfree(void* p);
 	void pool_release();
+	void sync_streams(); // waits for every stream of the context
 	std::multimap<size_t, void*> pool;        // free buffers by capacity
 	std::unordered_map<void*, size_t> owned;  // every buffer from dalloc, by capacity
 };

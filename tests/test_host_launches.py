@@ -45,3 +45,30 @@ def test_error_pass_of_a_fine_phi_grid_fits_a_launch(stub, tmp_path, num_phi, bl
     passes = _launches(lines, "k_errors")
     assert len(passes) == blocks and sum(g[1] for g in passes) == num_phi + 1
     assert all(int(v) <= 65536 for w in lines if w[0] == "launch" for v in w[3:5])
+
+
+@pytest.mark.parametrize("kernel,n", [("k_batch_step_tail", 1), ("k_batch_sweep", 6), ("k_batch_step_tail", 4)])
+def test_failed_batch_steps_leave_nothing_queued(stub, tmp_path, kernel, n):
+    """an FP64 batch works on three streams; a launch that fails in between leaves all of them waited for, since the
+    buffers that they use serve the next load"""
+    lines = _log(stub, tmp_path, f"""
+b = ccf_amd.Batch()
+for stars in (300, 60, 320):
+    b.add(num_stars=stars, num_phi=8, num_branches=1, {FIELD})
+b.load(0)
+b.build(0)
+stub.stub_fail({kernel.encode()!r}, {n})
+try:
+    b.solve(0)
+    raise SystemExit("the launch did not fail")
+except RuntimeError:
+    stub.stub_log(None)
+assert b.run(0), b.last_error()
+""")
+    used = {}
+    for k, w in enumerate(lines):
+        if w[0] in ("launch", "sync"):
+            used.setdefault(w[-1], {})[w[0]] = k
+    assert sum("launch" in v for v in used.values()) == 3
+    for s, v in used.items():
+        assert v.get("sync", -1) > v.get("launch", -1), (s, lines[-5:])
