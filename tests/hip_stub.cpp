@@ -20,6 +20,7 @@ namespace
 {
 std::mutex mu;
 std::map<const void*, std::string> names;
+std::map<const char*, size_t> pinned;
 FILE* out = nullptr;
 std::string fail_name;
 int fail_at = 0, cus = 256;
@@ -146,12 +147,25 @@ hipError_t hipHostMalloc(void** p, size_t n, unsigned)
 {
 	*p = std::calloc(1, n);
 	line("pin %zu\n", n);
+	std::lock_guard<std::mutex> l(mu);
+	pinned[(const char*)*p] = n;
 	return *p ? hipSuccess : hipErrorOutOfMemory;
 }
 hipError_t hipHostFree(void* p)
 {
 	line("unpin\n");
+	std::lock_guard<std::mutex> l(mu);
+	pinned.erase((const char*)p);
 	std::free(p);
+	return hipSuccess;
+}
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p)
+{
+	std::memset(a, 0, sizeof(*a));
+	a->type = hipMemoryTypeUnregistered;
+	std::lock_guard<std::mutex> l(mu);
+	const auto it = pinned.upper_bound((const char*)p);
+	if (it != pinned.begin() && (const char*)p < std::prev(it)->first + std::prev(it)->second) a->type = hipMemoryTypeHost;
 	return hipSuccess;
 }
 hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind)

@@ -2,10 +2,12 @@
 same time from several threads and contexts (one of them holds the slots, the
 others go through the runtime's own copy) give the same bytes, for sizes at
 and around the slots' boundaries."""
+import ctypes
 import threading
 
 import numpy as np
 import pytest
+import torch
 
 import ccf_amd
 
@@ -48,3 +50,18 @@ def test_concurrent_copies_agree(n, num_phi, nb):
     with ccf_amd.Context(**kw) as c:
         assert c.run(0)
         assert np.array_equal(c.array(ccf_amd.ARRAY_CCS), one)
+
+
+@pytest.mark.parametrize("offset", [0, 24])
+def test_copy_to_pinned_memory(offset):
+    """a destination that the runtime knows takes one copy, and the same bytes"""
+    buf = torch.empty(1 << 21, dtype=torch.float64, pin_memory=True)
+    with ccf_amd.Context(num_stars=137, kappa_tot=0.4, kappa_star=0.4, shear=0.2, num_phi=2000, num_branches=4, random_seed=7,
+                         outfile_prefix="./") as c:
+        assert c.run(0)
+        one = c.array(ccf_amd.ARRAY_CCS)
+        rows, cols = ctypes.c_int(), ctypes.c_int()
+        assert c.lib.ccf_get_array(c.ptr, ccf_amd.ARRAY_CCS, ctypes.c_void_p(buf.data_ptr() + 8 * offset), 8 * (buf.numel() - offset),
+                                   ctypes.byref(rows), ctypes.byref(cols)) == 0
+    got = buf[offset:offset + 2 * one.size].numpy().view(np.complex128)
+    assert one.nbytes >= 1 << 18 and np.array_equal(got, one.ravel())

@@ -72,3 +72,23 @@ assert b.run(0), b.last_error()
     assert sum("launch" in v for v in used.values()) == 3
     for s, v in used.items():
         assert v.get("sync", -1) > v.get("launch", -1), (s, lines[-5:])
+
+
+@pytest.mark.parametrize("pinned", [False, True])
+def test_copies_to_pinned_memory_go_there_at_once(stub, tmp_path, pinned):
+    """one copy of the whole array to memory that the runtime knows; to other memory, copies into the slots"""
+    lines = _log(stub, tmp_path, f"""
+p = ctypes.c_void_p()
+assert stub.hipHostMalloc(ctypes.byref(p), ctypes.c_size_t(1 << 23), 0) == 0
+c = ccf_amd.Context(num_stars=100, num_phi=1000, num_branches=1, {FIELD})
+assert c.run(0)
+plain = np.empty(1 << 20)
+base = (p.value if {pinned} else plain.ctypes.data) + 64
+stub.stub_log({str(tmp_path / 'log').encode()!r})
+r, k = ctypes.c_int(), ctypes.c_int()
+assert c.lib.ccf_get_array(c.ptr, 1, ctypes.c_void_p(base), 1 << 22, ctypes.byref(r), ctypes.byref(k)) == 0
+stub.stub_log(None)
+""")
+    copies = [int(w[1]) for w in lines if w[0] == "copy"]
+    assert sum(copies) == 200 * 1001 * 16
+    assert len(copies) == 1 if pinned else len(copies) > 1
