@@ -6,6 +6,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <bit>
 #include <chrono>
 #include <cmath>
 #include <cstdint>
@@ -679,11 +680,13 @@ double ms_seconds(double s) { return std::floor(s * 1000.0) / 1000.0; } // stopw
 // them started: above about 256 KiB the runtime pins the caller's pages for
 // a copy (320 KB: 150 -> 40 us, 3 MB: 740 -> 290).
 //
-// The pinned slots (two of COPY_CHUNK for each of COPY_THREADS threads: 64
-// MiB at most) and their events are shared by the process's contexts: a
-// thread's are made by the first copy that takes as many threads, used by
-// one copy at a time (a copy that finds them taken goes through hipMemcpy),
-// and given back when the last context is destroyed.
+// The pinned slots and their events are shared by the process's contexts:
+// made by the first copy, made anew by one that needs more, used by one copy
+// at a time (a copy that finds them taken goes through hipMemcpy), and given
+// back when the last context is destroyed. At most 64 MiB (two of COPY_CHUNK
+// for each of COPY_THREADS threads), and for a smaller array no more than
+// about twice its size, for pinning and freeing them costs about 30 us a MiB,
+// which a program that makes a context for each field pays every time.
 constexpr int COPY_THREADS = 8;
 constexpr size_t COPY_CHUNK = size_t(4) << 20;
 // Arrays below this go in half chunks, which the threads start on sooner
@@ -698,28 +701,31 @@ struct CopySlots
 	std::mutex use;  // held by the copy that uses the slots
 	std::mutex life; // guards contexts
 	long contexts = 0;
-	char* mem[COPY_THREADS] = {};
+	char* mem = nullptr;
+	size_t room = 0; // bytes of mem
 	hipEvent_t event[2 * COPY_THREADS] = {};
 
-	// the slots of the first T threads
-	bool ready(int T)
+	// the events of T threads and `bytes` of slots
+	bool ready(int T, size_t bytes)
 	{
-		for (int t = 0; t < T; t++)
-		{
-			for (int k = 2 * t; k < 2 * t + 2; k++)
-				if (!event[k] && hipEventCreateWithFlags(&event[k], hipEventDisableTiming) != hipSuccess)
-				{
-					event[k] = nullptr;
-					(void)hipGetLastError();
-					return false;
-				}
-			if (!mem[t] && hipHostMalloc((void**)&mem[t], 2 * COPY_CHUNK, hipHostMallocDefault) != hipSuccess)
+		for (int k = 0; k < 2 * T; k++)
+			if (!event[k] && hipEventCreateWithFlags(&event[k], hipEventDisableTiming) != hipSuccess)
 			{
-				mem[t] = nullptr;
+				event[k] = nullptr;
 				(void)hipGetLastError();
 				return false;
 			}
+		if (room >= bytes) return true;
+		if (mem) (void)hipHostFree(mem);
+		room = 0;
+		bytes = std::bit_ceil(bytes); // (arrays that grow little by little do not have them made anew each time)
+		if (hipHostMalloc((void**)&mem, bytes, hipHostMallocDefault) != hipSuccess)
+		{
+			mem = nullptr;
+			(void)hipGetLastError();
+			return false;
 		}
+		room = bytes;
 		return true;
 	}
 	void release()
@@ -730,11 +736,9 @@ struct CopySlots
 			if (e) (void)hipEventDestroy(e);
 			e = nullptr;
 		}
-		for (char*& p : mem)
-		{
-			if (p) (void)hipHostFree(p);
-			p = nullptr;
-		}
+		if (mem) (void)hipHostFree(mem);
+		mem = nullptr;
+		room = 0;
 	}
 };
 
@@ -822,8 +826,12 @@ hipError_t ccf::copy_out(ccf_ctx* c, void* dst, const void* src, size_t bytes)
 	CopySlots& cs = copy_slots();
 	const int T =
 		bytes >= COPY_MIN && c->stream && plain_memory(dst) ? (int)std::max<size_t>(1, std::min<size_t>(copy_threads(), bytes / COPY_PART)) : 0;
+	// a thread's part, and its two slots (one for a part that is a chunk or less)
+	const size_t share = T > 0 ? bytes / T : 0, part_max = T > 0 ? bytes - share * (T - 1) : 0;
+	const size_t chunk = bytes >= COPY_LARGE ? COPY_CHUNK : COPY_CHUNK / 2;
+	const size_t slot_size = (std::min(chunk, part_max) + 4095) / 4096 * 4096, slots = part_max > chunk ? 2 : 1;
 	std::unique_lock<std::mutex> lock(cs.use, std::defer_lock);
-	if (T < 1 || !lock.try_lock() || !cs.ready(T))
+	if (T < 1 || !lock.try_lock() || !cs.ready(T, T * slots * slot_size))
 	{
 		if (!c->stream) return hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost);
 		const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream);
@@ -831,10 +839,11 @@ hipError_t ccf::copy_out(ccf_ctx* c, void* dst, const void* src, size_t bytes)
 	}
 	std::atomic<int> bad{hipSuccess};
 	auto part = [&](int t) noexcept {
-		const size_t lo = bytes / T * t, hi = t + 1 == T ? bytes : bytes / T * (t + 1);
-		char* const slot[2] = {cs.mem[t], cs.mem[t] + COPY_CHUNK};
+		const size_t lo = share * t, hi = t + 1 == T ? bytes : share * (t + 1);
+		char* const first = cs.mem + t * slots * slot_size;
+		char* const slot[2] = {first, first + (slots - 1) * slot_size};
 		hipEvent_t const event[2] = {cs.event[2 * t], cs.event[2 * t + 1]};
-		const hipError_t e = copy_part((char*)dst, (const char*)src, lo, hi, bytes >= COPY_LARGE ? COPY_CHUNK : COPY_CHUNK / 2, slot, event, c->stream);
+		const hipError_t e = copy_part((char*)dst, (const char*)src, lo, hi, chunk, slot, event, c->stream);
 		if (e != hipSuccess) bad = e;
 	};
 	std::vector<std::thread> threads;

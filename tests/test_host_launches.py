@@ -92,3 +92,27 @@ stub.stub_log(None)
     copies = [int(w[1]) for w in lines if w[0] == "copy"]
     assert sum(copies) == 200 * 1001 * 16
     assert len(copies) == 1 if pinned else len(copies) > 1
+
+
+def test_copy_slots_are_as_large_as_the_arrays_need(stub, tmp_path):
+    """a program that makes a context for each field has the slots made and freed with each: one pinned allocation, for
+    a small array at most twice its size; a larger one when a copy needs more, none when it needs less"""
+    lines = _log(stub, tmp_path, f"""
+def run(num_phi):
+    c = ccf_amd.Context(num_stars=100, num_phi=num_phi, num_branches=1, {FIELD})
+    assert c.run(0)
+    return c
+a, b, d = run(200), run(3000), run(50000)
+stub.stub_log({str(tmp_path / 'log').encode()!r})
+for c in (a, b, a, b, d, a, b, d):
+    c.array(1)
+stub.stub_log(None)
+for c in (a, b, d):
+    c.close()
+""")
+    pins = [int(w[1]) for w in lines if w[0] == "pin"]
+    sizes = [200 * 201 * 16, 200 * 3001 * 16, 200 * 50001 * 16]
+    assert len(pins) <= len(sizes) and pins == sorted(set(pins))
+    assert pins[0] <= 2 * (sizes[0] + 4096) and pins[-1] <= 64 << 20
+    assert len(pins) == 1 or pins[1] <= 2 * (sizes[1] + 8 * 4096)
+    assert sum(w[0] == "unpin" for w in lines) == len(pins) - 1
