@@ -2482,9 +2482,12 @@ bool sweep_layout(ccf_ctx* ctx, SweepBufs& b, int rows, int R, Take&& take)
 	const size_t list = (size_t)rows * R;
 	if (!(take(b.act, 2 * list) && take(b.cnt, 2 * (size_t)rows) && take(b.fl, list) && take(b.fcnt, 2 * (size_t)rows) &&
 			take(b.f0, list) && take(b.f1, list) && take(b.ex, list) &&
-			take(b.tile_off, (size_t)rows + 1) && take(b.plan, 4 + 2 * TRACK_SWEEPS) && take(b.ticket, 1) &&
+			take(b.tile_off, (size_t)rows + 1) && take(b.plan, 4 + 2 * TRACK_SWEEPS + 1) &&
 			take(b.part, b.part_room)))
 		return false;
+	// (after the plan: a slice of its own would take 256 bytes more, 16 roots
+	// of the largest sweep in the fixed scratch array)
+	b.ticket = b.plan ? b.plan + 4 + 2 * TRACK_SWEEPS : nullptr;
 	if (ctx->P.root_fmm != 1 || R < ROOT_FMM_MIN_ROOTS) return true;
 	return root_layout(ctx, b, take);
 }

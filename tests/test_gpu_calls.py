@@ -66,3 +66,16 @@ def test_root_sum_sizes(workdir, n):
     # truncation at order 14 (3e-8 of the sum of moduli on uniform sets; the
     # bound that the 6000-root test of this order allows)
     assert np.all(np.abs(S[pick] - D) <= 2e-7 * scale)
+
+
+def test_noalloc_sweep_largest_row(workdir):
+    """the largest row that the no-allocation sweep's 32 MiB hold (mixed form, one root a thread)"""
+    sf = make_field(workdir, "salpeter300")
+    n = 194112
+    z = _points(sf, n, 5)
+    with ccf_amd.Context(starfile=sf, outfile_prefix="./", kappa_tot=0.45, shear=0.35, num_phi=10, precision=1, roots_per_thread=1) as c:
+        c.prepare()
+        g = c.aberth_sweep_noalloc(z, 0.7)
+        assert np.array_equal(g, c.aberth_sweep(z, 0.7)) and np.any(g != z)
+        with pytest.raises(RuntimeError, match="bytes of scratch"):
+            c.aberth_sweep_noalloc(np.append(z, 0.5 + 0.5j), 0.7)
