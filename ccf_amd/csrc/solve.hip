@@ -1632,7 +1632,12 @@ inline size_t chain_lds(int R, int N, int n)
 	return (size_t)(R + N) * sizeof(double2) + (size_t)n * (2 * sizeof(double2) + 3 * sizeof(int));
 }
 
-inline int chain_team(int R, int rows) { return std::max(1, std::min(std::min(TEAM_MAX, TEAM_WGS / rows), R / TEAM_ROOTS)); }
+// (a device of fewer CUs, such as a partition of one: a quarter of those)
+inline int chain_team(int R, int rows, int cus)
+{
+	const int wgs = std::min(TEAM_WGS, cus / 4);
+	return std::max(1, std::min(std::min(TEAM_MAX, wgs / rows), R / TEAM_ROOTS));
+}
 
 // Whether a field's chains run as teams. A step of theirs takes 30 to 90 us
 // (3.6 sweeps of 7 us, and a member's share of the sums), one over the
@@ -1648,9 +1653,9 @@ constexpr size_t CHAIN_LDS = 152 * 1024;
 // in y; a run has num_phi + num_branches)
 constexpr int ERROR_ROWS = 32768;
 
-inline bool chain_fits(int R, int N, int rows)
+inline bool chain_fits(int R, int N, int rows, int cus)
 {
-	return chain_lds(R, N, R) <= CHAIN_LDS && (long long)R * (R + N) / chain_team(R, rows) <= TEAM_TERMS;
+	return chain_lds(R, N, R) <= CHAIN_LDS && (long long)R * (R + N) / chain_team(R, rows, cus) <= TEAM_TERMS;
 }
 
 __global__ void k_clear_teams(ChainTeams T, int rows)
@@ -2853,7 +2858,7 @@ bool find_initial_roots_dev(ccf_ctx* ctx, int verbose)
 bool chain_field(const ccf_ctx* ctx)
 {
 	return ctx->P.precision == 0 && ctx->P.approx && ctx->P.root_fmm != 1 &&
-		chain_fits(ctx->num_roots, ctx->num_stars, 2 * ctx->P.num_branches);
+		chain_fits(ctx->num_roots, ctx->num_stars, 2 * ctx->P.num_branches, ctx->num_cus);
 }
 
 // the teams' meeting points and published positions, kept with the field
@@ -2972,7 +2977,7 @@ bool find_ccs_dev(ccf_ctx* ctx, int verbose)
 			tt.b = ctx->next_event();
 			if (tt.a && tt.b) (void)hipEventRecord(tt.a, s);
 		}
-		const int K = chain_team(R, 2 * nb), N = ctx->num_stars;
+		const int K = chain_team(R, 2 * nb, ctx->num_cus), N = ctx->num_stars;
 		ChainTeams T;
 		if (!chain_teams(ctx, T, K)) return false;
 		k_clear_teams<<<1, 64, 0, s>>>(T, 2 * nb);

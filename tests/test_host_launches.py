@@ -116,3 +116,18 @@ for c in (a, b, d):
     assert pins[0] <= 2 * (sizes[0] + 4096) and pins[-1] <= 64 << 20
     assert len(pins) == 1 or pins[1] <= 2 * (sizes[1] + 8 * 4096)
     assert sum(w[0] == "unpin" for w in lines) == len(pins) - 1
+
+
+@pytest.mark.parametrize("cus,branches,workgroups", [(256, 1, 24), (256, 4, 64), (256, 40, 80), (128, 1, 24), (128, 4, 32),
+                                                     (32, 1, 8), (32, 4, 8), (32, 8, 16), (4, 1, 2)])
+def test_teams_fit_a_quarter_of_the_device(stub, tmp_path, cus, branches, workgroups):
+    """the workgroups that wait for each other are at most a quarter of the CUs (a member takes a whole one); with more
+    rows than that none waits"""
+    lines = _log(stub, tmp_path, f"""
+stub.stub_cus({cus})
+c = ccf_amd.Context(num_stars=50, num_phi={8 * branches}, num_branches={branches}, {FIELD})
+assert c.run(0)
+""")
+    teams, alone = _launches(lines, "k_chains")
+    assert teams[0] == workgroups and alone[0] == 2 * branches
+    assert teams[0] <= max(cus // 4, 2 * branches)
