@@ -142,6 +142,7 @@ def load(path: str = LIB_PATH) -> ctypes.CDLL:
         "ccf_default_params": (None, [P]),
         "ccf_set_params": (ctypes.c_int, [vp, P]),
         "ccf_get_params": (ctypes.c_int, [vp, P]),
+        "ccf_team_retries": (ctypes.c_longlong, [vp]),
         "ccf_run": (ctypes.c_int, [vp, ctypes.c_int]),
         "ccf_save": (ctypes.c_int, [vp, ctypes.c_int]),
         "ccf_check_input_params": (ctypes.c_int, [vp, ctypes.c_int]),

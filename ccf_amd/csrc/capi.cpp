@@ -959,6 +959,8 @@ int ccf_set_team_wait(ccf_ctx* c, long long ticks)
 	return 0;
 }
 
+long long ccf_team_retries(const ccf_ctx* c) { return c ? c->team_retries : -1; }
+
 int ccf_get_params(const ccf_ctx* c, ccf_params* p)
 {
 	if (!c || !p) return 1;

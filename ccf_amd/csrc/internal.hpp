@@ -239,6 +239,7 @@ struct ccf_ctx
 	char* chain_mem = nullptr;    // FP64 chains of small fields: see ChainTeams (solve.hip)
 	size_t chain_bytes = 0;
 	long long team_wait = -1;     // ccf_set_team_wait
+	long long team_retries = 0;   // ccf_team_retries
 	std::vector<hipEvent_t> events;
 	size_t events_used = 0;
 	hipEvent_t next_event()

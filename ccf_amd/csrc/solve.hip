@@ -69,6 +69,7 @@ enum Counter
 	C_TAIL_NEAR = 17,  // k_tail: near-field stars of its evaluations
 	C_TAIL_SWEEPS = 18, // k_tail: sweeps, summed over rows
 	C_OUTSIDE = 19,     // error pass: points outside the tree (their near field is every star)
+	C_TEAM_RETRY = 20,  // k_chains: launches whose teams gave up waiting
 	C_COUNT = 24
 };
 
@@ -1732,6 +1733,7 @@ __global__ __launch_bounds__(BS) void k_chains(LensView L, double2* __restrict__
 		if (r == 0 && threadIdx.x < CHAIN_COUNTS) atomicAdd(stat_slot(stats, which[threadIdx.x]), T.counts[threadIdx.x]);
 		return;
 	}
+	if (RETRY && r == 0 && threadIdx.x == 0) atomicAdd(stat_slot(stats, C_TEAM_RETRY), 1ull);
 	double2* const zc = chain_mem; // in processing order
 	double2* const st = zc + R;
 	double2* const f0 = st + N;
@@ -3149,6 +3151,7 @@ bool find_ccs_dev(ccf_ctx* ctx, int verbose)
 	ctx->info.updates_early = (long long)(c[C_EARLY] + c[C_TAIL_EARLY]);
 	ctx->info.updates_newton = (long long)(c[C_NEWTON] + c[C_TAIL_NEWTON]);
 	ctx->info.tail_sweeps = (long long)c[C_TAIL_SWEEPS];
+	ctx->team_retries = (long long)c[C_TEAM_RETRY];
 	ctx->info.cluster_chunks = (long long)c[C_CLUSTER];
 	{
 		// algorithmic flops: 10 per Cauchy term of the sums; per Witt

@@ -156,6 +156,10 @@ int ccf_get_params(const ccf_ctx* ctx, ccf_params* p);
    does their work instead, with the same results: 0.2 s unless set, which a
    device with room for all of them does not come near; negative: the default. */
 int ccf_set_team_wait(ccf_ctx* ctx, long long ticks);
+/* How many of the continuations since the last initial solve (in general one)
+   had workgroups that gave up waiting, and so were solved by one workgroup per
+   chain. */
+long long ccf_team_retries(const ccf_ctx* ctx);
 
 /* bool CCF::run(int verbose) (ccf.cuh:1265-1280) */
 int ccf_run(ccf_ctx* ctx, int verbose);

@@ -136,3 +136,15 @@ def test_error_pass_in_blocks_of_rows(workdir):
     assert info["points_converged"] == info["points_total"] == z.size
     g = e[:, 4] + 1j * e[:, 5]
     assert (np.abs(w - g) / np.maximum(np.abs(g), 1.0)).max() < 1e-11
+
+
+@pytest.mark.parametrize("n,nb", [(17, 1), (100, 1), (137, 2), (240, 3), (1000, 1), (300, 16)])
+def test_teams_meet(workdir, n, nb):
+    """the teams of a run that has the device to itself meet, for every size
+    of team; members that may not wait give up"""
+    kw = dict(starfile=_stars(workdir, n), outfile_prefix="./", kappa_tot=0.45, shear=0.3, num_phi=8 * nb, num_branches=nb)
+    with ccf_amd.Context(**kw) as c:
+        for wait, retries in ((-1, 0), (0, 1), (-1, 0)):
+            assert c.lib.ccf_set_team_wait(ctypes.c_void_p(c.ptr), ctypes.c_longlong(wait)) == 0
+            assert c.run(0), c.last_error()
+            assert c.lib.ccf_team_retries(c.ptr) == retries, wait
