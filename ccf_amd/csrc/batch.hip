@@ -386,7 +386,8 @@ __device__ void solve_row(const BField& F, int row, int cap, bool newton, double
 	}
 }
 
-// The persistent solve of one phase (0: branch centres, 1: phi chains).
+// The persistent solve of one phase (0: branch centres, 1: phi chains, the
+// mixed form's; k_batch_chains has the FP64 form's).
 // Dynamic LDS: rlds roots and nlds stars (fields with more stars read them
 // from global memory; a field with more than rlds roots solves its rows in
 // place in global memory). lists: the active lists and the listed roots,
@@ -426,7 +427,7 @@ __global__ __launch_bounds__(BS, BATCH_WAVES_PER_SIMD) void k_batch(const BField
 		unsigned long long cnt[BCNT] = {0, 0, 0, 0, 0, 0};
 		// the row being solved: in LDS, or in place in the output rows
 		const bool lds_row = R <= rlds;
-		if (phase == 0)
+		if (!MIXED || phase == 0)
 		{
 			const int row = centre_row(F, tk.branch);
 			double2* zc = lds_row ? smem : F.roots + (size_t)row * R;
@@ -450,7 +451,7 @@ __global__ __launch_bounds__(BS, BATCH_WAVES_PER_SIMD) void k_batch(const BField
 				// (in place: row is written, the rows before it are read)
 				for (int i = threadIdx.x; i < R; i += BS)
 					zc[i] = predict_root(F.roots + (size_t)(row - sgn) * R + i, (long long)sgn * R, q);
-				solve_row<BS, MIXED>(F, row, F.cap_step, true, zc, st, la, lb, ls, s_n, cnt);
+				solve_row<BS, true>(F, row, F.cap_step, true, zc, st, la, lb, ls, s_n, cnt);
 				if (lds_row)
 					for (int i = threadIdx.x; i < R; i += BS) F.roots[(size_t)row * R + i] = zc[i];
 			}
