@@ -701,7 +701,7 @@ __global__ __launch_bounds__(BLOCK, 4) void k_batch_sweep(const BField* __restri
 		cauchy_run<-1>(zr, r0, r1, z.x, z.y, ax, ay); // ccf_functions.cuh:232-239
 		if (!(isfinite(ax) && isfinite(ay)))
 		{
-			// out of cauchy4's range: the terms one by one
+			// out of cauchy8's range: the terms one by one
 			ax = ay = 0;
 			for (int q = s0; q < s1; q++) cauchy1<1>(z.x, z.y, st[q], ax, ay);
 			ax *= 2;

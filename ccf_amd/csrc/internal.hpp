@@ -260,12 +260,12 @@ struct ccf_ctx
 	hipEvent_t err_event = nullptr;   // a row set's roots are final (no timing)
 	size_t host_size = 0;         // bytes of host_counts' allocation: kept from run to run, grown when one needs more
 	int* host_track = nullptr; // a part of it: [CONT_GROUPS][TRACK_STEPS][2 TRACK_SWEEPS] the tracked counts of a group's last steps
-	hipEvent_t step_event[2 * ccf::CONT_GROUPS] = {}; // mixed continuation: before a step's tail, per group and parity (no timing)
+	hipEvent_t step_event[2 * ccf::CONT_GROUPS] = {}; // tailed continuations: before a step's tail, per group and parity (no timing)
 	hipEvent_t fmm_rows_event[2 * ccf::CONT_GROUPS] = {}; // mixed continuation: after the copy of a step's FMM row count, per group (no timing)
 	hipEvent_t read_event[ccf::CONT_GROUPS] = {}; // after the copy of a sweep's active counts, per group (no timing)
-	hipStream_t group_streams[ccf::CONT_GROUPS - 1] = {}; // mixed form: the streams of the groups of branches after the first (default priority)
+	hipStream_t group_streams[ccf::CONT_GROUPS - 1] = {}; // the streams of the groups of rows after the first (default priority)
 	hipEvent_t group_event = nullptr;   // orders the group streams around the continuation (no timing)
-	ccf::SweepBufs swg[ccf::CONT_GROUPS - 1]; // mixed form: the sweep buffers of the groups after the first
+	ccf::SweepBufs swg[ccf::CONT_GROUPS - 1]; // the sweep buffers of the groups after the first
 	int fmm_rows_sweep[2] = {-1, -1}; // root-sum FMM rows of the last phase's first and second sweep (-1: unknown)
 	int phase_sweeps = 0;         // sweeps the last phase ran (its cap when no read-back saw it end)
 	// params.autotune: the choices the context's first solve timed fastest

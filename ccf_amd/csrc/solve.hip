@@ -13,12 +13,14 @@
 //                  appended to a per-row list (the few roots outside the
 //                  tree by their whole wave); its last workgroup runs
 //   K2 plan_sums   cuts the (stars + roots) term range of every tile of
-//                  RPT*256 listed roots into S slices so that dense and sparse
+//                  listed roots into S slices so that dense and sparse
 //                  sweeps alike give enough equal work items to fill the chip;
-//   K3 k_sums*     one work item = one tile x one slice: the slice's terms are
-//                  streamed through LDS and every lane accumulates
-//                  2 sum 1/(z - s_i) - sum 1/(z - z_j) for its RPT roots;
-//                  partials go to a buffer so the result is deterministic;
+//   K3 k_sums*     one work item = one tile x one slice: the partial sums
+//                  2 sum 1/(z - s_i) - sum 1/(z - z_j) of the tile's roots
+//                  over the slice's terms (FP32: through LDS, RPT roots a
+//                  lane; FP64: by single waves, a root a lane, the terms
+//                  through scalar loads); partials go to a buffer, which
+//                  k_finalize adds in a fixed order;
 //   K4 k_finalize  reduces the partials, forms z - f0 / (f1 + f0 S), tests
 //                  |dz| / theta < 1e-9, writes the root and appends the
 //                  unconverged ones to the next sweep's active list.
@@ -776,10 +778,10 @@ __global__ __launch_bounds__(BLOCK, 8) void k_sums64(const double2* __restrict__
 // K3 in FP64 of the continuation steps and of single sweeps: the same partial
 // sums with the reciprocals shared (cauchy8).
 //
-// Bound by the FP64 VALU: 20 000 roots against 30 000 terms take 0.22 ms
-// (2.7e12 terms/s; the loop alone reaches 3.2e12), 0.33 ms in k_sums64. A
-// continuation step's sparse sweeps gain more: waves as items, lanes over the
-// sources.
+// Bound by the FP64 VALU: 20 000 roots against 30 000 terms take 0.204 ms
+// (2.9e12 terms/s, 0.70 of what the issue slots allow), 0.33 ms in k_sums64.
+// A continuation step's sparse sweeps gain more: waves as items, lanes over
+// the sources.
 
 // One wave takes an item, a tile of QUAD_TILE listed roots and a slice of
 // the terms, by itself: no LDS and no barrier. A row with at most QUAD_SPARSE
@@ -827,7 +829,7 @@ __global__ __launch_bounds__(BLOCK, 8) void k_sums64_quad(const double2* __restr
 				cauchy_lanes<-1>(xrow, r0, r1, z.x, z.y, ax, ay);
 				if (!(isfinite(ax) && isfinite(ay)))
 				{
-					// out of cauchy4's range: the lane's terms one by one
+					// out of cauchy4's range (cauchy_lanes): the lane's terms one by one
 					ax = ay = 0;
 					for (int q = s0 + lane; q < s1; q += 64) cauchy1<1>(z.x, z.y, spos[q], ax, ay);
 					ax *= 2;
@@ -851,7 +853,7 @@ __global__ __launch_bounds__(BLOCK, 8) void k_sums64_quad(const double2* __restr
 		cauchy_run<-1>(xrow, r0, r1, z.x, z.y, ax, ay); // ccf_functions.cuh:232-239
 		if (!(isfinite(ax) && isfinite(ay)))
 		{
-			// out of cauchy4's range: the terms one by one
+			// out of cauchy8's range: the terms one by one
 			ax = ay = 0;
 			for (int q = s0; q < s1; q++) cauchy1<1>(z.x, z.y, spos[q], ax, ay);
 			ax *= 2;
@@ -1307,9 +1309,10 @@ __device__ __forceinline__ TailSum tail_sum(const double2* __restrict__ xrow, in
 
 // The sums of a continuation step's later sweeps over the whole device: an
 // item is the listed roots of a row that a workgroup takes at a time, each
-// summed exactly as k_tail sums it (tail_sum), the whole Aberth sum left in
-// ex. A step's roots so do not depend on where its tail starts, which the
-// counts of earlier steps decide. Bound by the latency of the row's loads
+// summed by the code that k_tail sums it with (tail_sum), the whole Aberth sum
+// left in ex. (Where the tail starts, which the counts of earlier steps
+// decide, may still move a last bit: k_witt and k_tail compile the evaluation
+// each for itself.) Bound by the latency of the row's loads
 // when few roots are listed (a wave a root): TAIL_LOADS of them in flight
 // took the launch from 561 to 228 us on rows of 100 060 roots, and k_tail,
 // which shares the loop, from 106 to 74 us on rows of 20 000.
@@ -2316,10 +2319,10 @@ bool run_sweeps_groups(ccf_ctx* ctx, SweepGroup* gs, int G, double2* roots, int 
 				for (int r = 0; r < nrows; r++) most = std::max(most, ctx->host_counts[q.row0 + r]);
 				if (most <= (f32 ? TAIL_ACTIVE : 64)) q.tail_at = it + 1;
 			}
-			// mixed form, continuation: the sweeps from tail_at on in one launch, with no read-back, which begins with
-			// this sweep's updates. The rows the root-sum FMM took in the
-			// step's first two sweeps go to the host for the choice two steps
-			// later.
+			// the sweeps from tail_at on in one launch, with no read-back (mixed
+			// form: it begins with this sweep's updates). The rows the root-sum
+			// FMM took in the step's first two sweeps go to the host for the
+			// choice two steps later.
 			const bool tail_now = q.tail_at > 0 && it + 1 == q.tail_at && it + 1 < cap;
 			if (!tail_now || !f32) k_finalize<<<g_rows, BLOCK, 0, s>>>(ctx->theta, roots, M, V, ctx->counters);
 			if (!CCF_LAUNCH(ctx, "find_critical_curve_roots_kernel")) return false;
@@ -2644,7 +2647,8 @@ bool alloc_groups(ccf_ctx* ctx)
 }
 
 // most bytes of a call's points or roots, and of its results, that go through
-// pinned memory (call_slots); above, a copy is as fast
+// the context's pinned memory (call_slots); above, the way in is the
+// runtime's copy, and the way out copy_out
 constexpr size_t CALL_BYTES = size_t(128) << 10;
 
 // the pinned host memory of a context, one allocation: the slots of the read-

@@ -84,3 +84,17 @@ def test_quad_sums_coincident_roots(workdir, copies):
     # (as in _check: roundings of the terms, and of f0 and f1)
     tol = 64 * EPS * (np.maximum(np.abs(roots), 1) + step * step * scale) + 1e-12 * step
     assert step.max() > 0 and np.all(np.abs(g - o) <= tol), (np.abs(g - o) / tol).max()
+
+
+@pytest.mark.parametrize("n", [20, 30, 300])
+@pytest.mark.parametrize("far", [1, 8])
+def test_quad_sums_between_the_ranges(workdir, n, far):
+    """roots so far off that a product of eight squared distances is out of
+    range and one of four is not: the dense form's terms one by one, the
+    sparse form's (at most 24 listed roots) in groups of four"""
+    sf = make_field(workdir, "cfg1")
+    rng = np.random.default_rng(n)
+    roots = 18 * (rng.uniform(-1, 1, n) + 1j * rng.uniform(-1, 1, n))
+    roots[:far] = 1e25 * np.exp(0.7j * np.arange(1, far + 1)) * np.arange(1, far + 1)
+    print(f"# quad sums, {n} roots, {far} of them far off", flush=True)
+    _check(sf, roots, dict(kappa_tot=0.3, shear=0.1, direct=1, num_phi=10))
