@@ -35,6 +35,7 @@ from ccf_amd import io  # noqa: E402
 
 METRIC = "converged cc points/s at 10k stars, mixed vs FP64 on 1 MI355X; max root error"
 PEAK_FP64_TFLOPS = 78.6   # MI355X FP64 vector (and matrix) peak
+FP64_SUMS = "k_sums64, k_sums64_quad"  # the FP64 form's Cauchy sums: branch centres, continuation
 PEAK_FP32_TFLOPS = 157.3
 
 WORKLOADS = {
@@ -535,14 +536,15 @@ def main():
     def region(r, which):
         # the two event-timed regions of a sweep: the root sums (FMM pass and
         # direct sums) and the Witt evaluation (k_witt, which also plans the sums)
+        fp64 = r is not res.get("mixed")
         if which == "sums":
             name = ("root sums: FMM pass (k_r*) + k_sums32" if r.get("root_fmm") else
-                    ("k_sums32" if r is res.get("mixed") else "k_sums64"))
+                    (FP64_SUMS if fp64 else "k_sums32"))
             return dict(kernel=name, achieved=r["sums_tflops"], total_ms=r["aberth_ms_total"],
                         avg_launch_ms=r["aberth_ms_avg"], launches=r["aberth_launches"])
         if which == "tail":
             n = max(1, r.get("tail_launches", 0))
-            return dict(kernel="k_tail (phase tails: Witt evaluations and Cauchy sums)", achieved=r.get("tail_tflops", 0.0),
+            return dict(kernel=("k_tail64" if fp64 else "k_tail") + " (phase tails: Witt evaluations and Cauchy sums)", achieved=r.get("tail_tflops", 0.0),
                         total_ms=r.get("tail_ms_total", 0.0), avg_launch_ms=r.get("tail_ms_total", 0.0) / n,
                         launches=r.get("tail_launches", 0))
         return dict(kernel="k_witt", achieved=r["witt_tflops"], total_ms=r["witt_ms_total"],
@@ -565,10 +567,11 @@ def main():
             "timed_with": "HIP events on the context's stream around each sweep's regions, during one step run after the timed steps",
             "regions": [dict(g, frac=g["achieved"] / pk) for g in regs]}
     if "fp64" in res:
-        roof["fp64_kernel"] = {"kernel": "k_sums64", "achieved": res["fp64"]["sums_tflops"], "peak": PEAK_FP64_TFLOPS,
+        roof["fp64_kernel"] = {"kernel": FP64_SUMS, "achieved": res["fp64"]["sums_tflops"], "peak": PEAK_FP64_TFLOPS,
                                "frac": res["fp64"]["sums_tflops"] / PEAK_FP64_TFLOPS,
                                "avg_launch_ms": res["fp64"]["aberth_ms_avg"],
-                               "traffic": measured_traffic(args.workload, "k_sums64")}
+                               "timed_with": "HIP events; the two sides of the branches run on two streams, whose events add",
+                               "traffic": measured_traffic(args.workload, FP64_SUMS)}
 
     cpu = None
     gate = None

@@ -40,3 +40,10 @@ def test_summary_launch_durations_come_from_the_event_step():
     assert abs(r["witt_tflops"] - 10.0) < 1e-12
     assert abs(r["tail_tflops"] - 0.1) < 1e-12
     assert r["tail_launches"] == 2
+
+
+def test_fp64_region_names_the_kernels_that_were_counted():
+    """the HBM traffic beside the FP64 form's sums is that of its own kernels"""
+    assert "k_sums64_quad" in bench.FP64_SUMS
+    assert bench.measured_traffic("cc10k", bench.FP64_SUMS) > 0
+    assert bench.measured_traffic("cc10k", "k_witt") > 0
