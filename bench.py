@@ -583,7 +583,7 @@ def main():
         cpu["host"] = host
         m = cpu["sampled_branches_vs_oracle"].get("mixed")
         if m is not None:
-            # north-star accuracy gate: max root error <= 1e-9 theta_E against
+            # accuracy gate: max root error <= 1e-9 theta_E against
             # the FP64 oracle's exact roots, on the sampled branches and at
             # every point of the job where the mixed and FP64 forms differ
             jm = cpu.get("job_mixed_vs_fp64_differing_points") or {}
